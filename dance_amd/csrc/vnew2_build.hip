@@ -75,7 +75,7 @@ constexpr uint32_t kFinalMinDegree = 64;    // FINAL_MIN_DEGREE
 constexpr uint32_t kWarmupSteps = 64;       // WARMUP_EXPAND_STEPS
 constexpr uint32_t kCoarseIters = 2;        // COARSE_WARMUP_ITERS
 constexpr uint32_t kMedoidCandidates = 1024;
-constexpr uint32_t kMedoidSamples = 4096;
+constexpr uint32_t kMedoidSamples = kMedoidMaxSamples;
 
 static const Profile kProfiles[] = {
     {"QUALITY", false, 0, 0},
@@ -157,8 +157,10 @@ static int launch_medoid(const Rows& rows, hipStream_t s, float* d_scores, uint3
                          uint32_t ns) {
   const int cpl = pick_cpl(rows.rs.nch);
   return with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
-    hipLaunchKernelGGL((k_medoid<decltype(dt)::value, decltype(c)::value>), dim3(wave_grid(nc)), dim3(kBlock), 0, s,
-                       rows.rs, rows.N, nc, ns, d_scores, d_cands);
+    constexpr int CPL = decltype(c)::value;
+    constexpr uint32_t KC = medoid_cands(CPL);
+    hipLaunchKernelGGL((k_medoid<decltype(dt)::value, CPL>), dim3((nc + KC - 1) / KC), dim3(64 * medoid_waves(CPL)),
+                       medoid_lds_bytes(CPL), s, rows.rs, rows.N, nc, ns, d_scores, d_cands);
     DHIP(hipGetLastError());
     return 0;
   });
