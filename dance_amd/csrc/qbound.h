@@ -2,11 +2,13 @@
 // distance gathers whose result cannot change the search state.
 //
 // Each vector row x gets a 128-byte companion row (one cache line):
-//   chunk 0      header {float s, float r, float a, unused}
+//   chunk 0      header {float s, float r, float lo, float hi}
 //   chunks 1..7  int8 codes q (16 dimensions per chunk, zero padded)
-// with x ~ s*q, a ~ s^2 * sum(q^2) (rounded to fp32) and r >= ||x - s*q||_2
-// (rounded up). For a pair (x, y) with code dot product c (an exact integer),
-//   Q = s_x^2 A_x + s_y^2 A_y - 2 s_x s_y c = ||s_x q_x - s_y q_y||^2,
+// with x ~ s*q, a = s^2 * sum(q^2), r >= ||x - s*q||_2 (rounded up),
+// lo <= a (1 - k) - r^2 (1 + k) (rounded down) and hi >= a (1 + k) -
+// r^2 (1 - k) (rounded up), k = kQSlack = 2^-18. For a pair (x, y) with code
+// dot product c (an exact integer),
+//   Q = a_x + a_y - 2 s_x s_y c = ||s_x q_x - s_y q_y||^2,
 // and the triangle inequality gives ||x - y|| >= sqrt(Q) - r_x - r_y.
 //
 // The canonical fp32 distance (fmaf per lane over n_lane non-negative terms,
@@ -17,15 +19,24 @@
 // square to binary16 (unit 2^-11): a term t^2 becomes at least
 // t^2 (1 - 3 2^-11) - 2^-24 (the absolute part covers the subnormal range),
 // so for fp16 rows kappa2 = 2 (3 2^-11 + (n_lane + 8) u) and
-// eta = 1e-30 + dim 2^-24. The test holds when Q >= (sqrt((T + eta)
-// (1 + kappa2)) + r_x + r_y)^2. The test is evaluated in fp32 with explicit slack factors 2^-19,
-// 32 times the accumulated rounding (|Q_computed - Q| <= 6 u (a_x + a_y),
-// since 2 s_x s_y |c| <= a_x + a_y). A candidate proved this way would be
-// rejected by the pool's threshold test, so skipping its exact distance
-// leaves every result bit-identical. Rows with non-finite values, or whose
-// scale leaves [2^-60, 2^50], get r = +inf and are never skipped.
-// The same rows give an upper bound, sqrt(Q) + r_x + r_y >= ||x - y||
-// (q_pair_ub), which proves pair tests of the form fl(alpha * dist) <= T0.
+// eta = 1e-30 + dim 2^-24.
+//
+// Lower test: with S >= sqrt((T + eta)(1 + kappa2)) + r_x, Q >= (S + r_y)^2
+// proves dist >= T. Expanded by what belongs to which row it reads
+//   (a_y - r_y^2) - 2 S r_y - 2 s_x s_y c >= S^2 - a_x,
+// two fmaf and a product per candidate against one number of the querying
+// row (q_lower, q_lower_proves). In fp32 with lo_y for a_y - r_y^2: a test
+// that passes has S^2, 2 S r_y and r_y^2 each at most 3.1 (a_x + a_y) (the
+// left side is at most 2 a_y + a_x up to rounding), so its roundings sum to
+// less than 32 u (a_x + a_y); lo and the right side give up
+// k (a_x + a_y) = 64 u (a_x + a_y), and 1e-30 covers underflow.
+// Upper test: with 0 <= r_y <= e and e <= root - r_x, Q <= (e - r_y)^2 proves
+// ||x - y|| <= root, in the same form with hi_y and e^2 lowered by k e^2 (its
+// roundings are at most 8 u (e^2 + a_x + a_y)); see q_upper.
+// A candidate the lower test proves would be rejected by the pool's threshold
+// test, so skipping its exact distance leaves every result bit-identical.
+// Rows with non-finite values, or whose scale leaves [2^-60, 2^50], get
+// r = +inf and are never proved either way.
 #pragma once
 
 #include "wave.h"
@@ -34,13 +45,20 @@ namespace dance {
 
 constexpr uint32_t kQChunks = 8;                      // 16-byte chunks per code row
 constexpr uint32_t kQMaxDim = (kQChunks - 1u) * 16u;  // dimensions a code row holds
-constexpr float kQSlack = 0x1p-19f;
+constexpr float kQSlack = 0x1p-18f;
 
 struct QBoundSet {
   const uint4* rows;  // N x kQChunks chunks; nullptr disables the bound
   float kappa2;       // relative rounding slack of the row type and width
   float eta;          // absolute slack (underflow; binary16 subnormals)
 };
+
+// The next fp32 value above (up) or below a finite x.
+__device__ __forceinline__ float next_toward(float x, bool up) {
+  if (x == 0.0f) return up ? __uint_as_float(1u) : __uint_as_float(0x80000001u);
+  const uint32_t b = __float_as_uint(x);
+  return __uint_as_float((x > 0.0f) == up ? b + 1u : b - 1u);
+}
 
 // One octet per row (8 rows per wave): lane sub owns code words sub, sub+8,
 // sub+16, sub+24 (word w = dimensions 4w..4w+3), so every load and store of
@@ -134,15 +152,22 @@ __global__ __launch_bounds__(256) void k_quantize(RowSet rs, uint32_t N, uint32_
       r = (float)rd;
       if ((double)r < rd) r = __uint_as_float(__float_as_uint(r) + 1u);  // r >= 0: next float up
     }
-    const float a = (float)((double)s * (double)s * (double)A);
-    reinterpret_cast<uint4*>(o)[0] = make_uint4(__float_as_uint(s), __float_as_uint(r), __float_as_uint(a), 0u);
+    float lo = 0.0f, hi = 0.0f;
+    if (usable) {
+      const double a = (double)s * (double)s * (double)A, r2 = (double)r * (double)r, k = (double)kQSlack;
+      // one fp32 step outward covers the conversion and the double roundings
+      lo = next_toward((float)(a * (1.0 - k) - r2 * (1.0 + k)), false);
+      hi = next_toward((float)(a * (1.0 + k) - r2 * (1.0 - k)), true);
+    }
+    reinterpret_cast<uint4*>(o)[0] =
+        make_uint4(__float_as_uint(s), __float_as_uint(r), __float_as_uint(lo), __float_as_uint(hi));
   }
 }
 
 // The querying row's header (scalars) and code row address.
 struct QSelf {
   const uint4* row;
-  float s, r, a;
+  float s, r, lo;
 };
 
 __device__ __forceinline__ void q_load_self(const QBoundSet& qb, uint32_t id, QSelf& me) {
@@ -151,56 +176,54 @@ __device__ __forceinline__ void q_load_self(const QBoundSet& qb, uint32_t id, QS
   const uint4 h = p[0];  // same address in every lane: kept as scalars
   me.s = __uint_as_float(uni_u(h.x));
   me.r = __uint_as_float(uni_u(h.y));
-  me.a = __uint_as_float(uni_u(h.z));
+  me.lo = __uint_as_float(uni_u(h.z));
 }
 
-// Upper bound of sqrt((T + eta)(1 + kappa2)) + r_self (uniform).
-__device__ __forceinline__ float q_threshold(const QBoundSet& qb, const QSelf& me, float T) {
+// Upper bound of sqrt((T + eta)(1 + kappa2)) + r, r the querying row's.
+__device__ __forceinline__ float q_threshold(const QBoundSet& qb, float r, float T) {
   const float t = (T + qb.eta) * (1.0f + qb.kappa2);
-  return uni_f((__builtin_sqrtf(t) + me.r) * (1.0f + kQSlack));
+  return (__builtin_sqrtf(t) + r) * (1.0f + kQSlack);
 }
 
 // Chunk `sub` of the code row of candidate `id`. An inactive lane loads
 // nothing and the value is left unset (as in load_row): `active` is the same
-// on the 8 lanes of an octet and q_proves_reject returns false for it.
+// on the 8 lanes of an octet, and callers discard the answers of inactive
+// octets.
 __device__ __forceinline__ uint4 q_load(const QBoundSet& qb, uint32_t id, bool active, uint32_t sub) {
   uint4 b;
   if (active) b = qb.rows[(size_t)id * kQChunks + sub];
   return b;
 }
-
-// The bound's test for one pair: the querying row's scale s and a, the
-// candidate's header (sy, ry, ay), sT from q_threshold (or the prune's root)
-// and the exact integer code dot c. Every caller evaluates this expression,
-// so a decision does not depend on how c was computed.
-__device__ __forceinline__ bool q_pair_proves(float s, float a, float sT, float sy, float ry, float ay, int c) {
-  const float sa = a + ay;
-  const float q = __builtin_fmaf(-2.0f * (s * sy), (float)c, sa) - kQSlack * sa - 1e-30f;
-  const float w = (sT + ry) * (1.0f + kQSlack);
-  return q >= w * w * (1.0f + kQSlack);
+// Chunk `sub` of the querying row's codes, its header replaced by zeros, so
+// that a candidate's header adds nothing to the dot.
+__device__ __forceinline__ uint4 q_codes(const uint4& chunk, uint32_t sub) {
+  return sub == 0u ? make_uint4(0u, 0u, 0u, 0u) : chunk;
 }
 
-// q_pair_proves with the querying row's scale passed as m2s = -2 s. Scaling
-// by -2 commutes with rounding for the scales k_quantize keeps ([2^-60,
-// 2^50], or 0), so fl(m2s * sy) = -2 fl(s * sy) and the decision is that of
-// q_pair_proves on the same inputs.
-__device__ __forceinline__ bool q_pair_proves_m2(float m2s, float a, float sT, float sy, float ry, float ay, int c) {
-  const float sa = a + ay;
-  const float q = __builtin_fmaf(m2s * sy, (float)c, sa) - kQSlack * sa - 1e-30f;
-  const float w = (sT + ry) * (1.0f + kQSlack);
-  return q >= w * w * (1.0f + kQSlack);
+// The querying side of the lower test (see above): row header s, r, lo and S.
+struct QLower {
+  float m2s;  // -2 s
+  float n2S;  // -2 S
+  float K;    // S^2 - a (1 - k), 1e-30 added
+};
+__device__ __forceinline__ QLower q_lower(float s, float r, float lo, float S) {
+  return QLower{-2.0f * s, -2.0f * S, __builtin_fmaf(S, S, 1e-30f) - __builtin_fmaf(r, r, lo)};
+}
+// Whether the bound proves dist >= T for a candidate with header s, r, lo and
+// code dot c. Non-finite r or S make a NaN or -inf here, which proves nothing.
+__device__ __forceinline__ bool q_lower_proves(const QLower& me, float s, float r, float lo, int c) {
+  return __builtin_fmaf(me.m2s * s, (float)c, __builtin_fmaf(me.n2S, r, lo)) >= me.K;
 }
 
-// Exact integer code dot of two rows whose chunk `sub` every lane of an
-// octet holds (chunk 0, the header, left out); every lane of the octet
-// receives it. Must be called by all 64 lanes.
-__device__ __forceinline__ int q_octet_dot(const uint4& code, const uint4& b, uint32_t sub) {
+// Exact integer code dot of a querying row (q_codes) and a row whose chunk
+// `sub` every lane of an octet holds; every lane of the octet receives it.
+// Must be called by all 64 lanes.
+__device__ __forceinline__ int q_octet_dot(const uint4& code, const uint4& b) {
   int c = 0;
   c = __builtin_amdgcn_sdot4((int)code.x, (int)b.x, c, false);
   c = __builtin_amdgcn_sdot4((int)code.y, (int)b.y, c, false);
   c = __builtin_amdgcn_sdot4((int)code.z, (int)b.z, c, false);
   c = __builtin_amdgcn_sdot4((int)code.w, (int)b.w, c, false);
-  if (sub == 0) c = 0;  // chunk 0 is the header
   c += dpp<kDppHalfMirror>(0, c);
   c += dpp<kDppQuadXor2>(0, c);
   c += dpp<kDppQuadXor1>(0, c);
@@ -210,11 +233,10 @@ __device__ __forceinline__ int q_octet_dot(const uint4& code, const uint4& b, ui
 // Octet test for a candidate: every lane of the octet holds one chunk `b` of
 // its code row (q_load); the lane with sub == 0 (which holds the header)
 // returns whether the bound proves dist >= T. `code` is chunk `sub` of the
-// querying row. Must be called by all 64 lanes.
-__device__ __forceinline__ bool q_proves_reject(const QSelf& me, const uint4& code, float sT, const uint4& b,
-                                                bool active, uint32_t sub) {
-  const int c = q_octet_dot(code, b, sub);
-  return active && q_pair_proves(me.s, me.a, sT, __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), c);
+// querying row (q_codes). Must be called by all 64 lanes.
+__device__ __forceinline__ bool q_proves_reject(const QLower& me, const uint4& code, const uint4& b) {
+  const int c = q_octet_dot(code, b);
+  return q_lower_proves(me, __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), c);
 }
 
 // The upper-bound side, for a pair test fl(alpha * dist) <= T0 (the online
@@ -243,17 +265,20 @@ __device__ __forceinline__ float q_ub_root_of(const QBoundSet& qb, float T0, flo
   const float r = q_ub_root(qb, T0, alpha);
   return DT == DANCE_F16 ? fminf(r, 254.0f) : r;
 }
-// Proves D <= root_ub^2 for the pair (querying row s, a, r; candidate
-// header sy, ry, ay; code dot c): by the triangle inequality ||x - y|| <=
-// sqrt(Q) + r_x + r_y, and Q <= Q_computed + 6 u (a_x + a_y); the fp32
-// evaluation adds kQSlack (a_x + a_y) + 1e-30 instead and rounds the sum up
-// by kQSlack. Rows with r = +inf are never proved.
-__device__ __forceinline__ bool q_pair_ub(float s, float a, float r, float root_ub, float sy, float ry, float ay,
-                                          int c) {
-  const float sa = a + ay;
-  const float q = __builtin_fmaf(-2.0f * (s * sy), (float)c, sa) + kQSlack * sa + 1e-30f;
-  const float lhs = (__builtin_sqrtf(fmaxf(q, 0.0f)) + r + ry) * (1.0f + kQSlack);
-  return lhs <= root_ub;
+// The querying side of the upper test (see above): row header s, r, hi and
+// the root that ||x - y|| must not pass (negative: nothing is proved).
+struct QUpper {
+  float m2s;  // -2 s
+  float e, e2;  // e <= root - r (-1 when not positive), 2 e
+  float K;    // e^2 (1 - k) - a (1 + k) - 1e-30
+};
+__device__ __forceinline__ QUpper q_upper(float s, float r, float hi, float root) {
+  float e = (root - r) * (1.0f - kQSlack);
+  if (!(e > 0.0f)) e = -1.0f;
+  return QUpper{-2.0f * s, e, 2.0f * e, e * e * (1.0f - kQSlack) - __builtin_fmaf(r, r, hi) - 1e-30f};
+}
+__device__ __forceinline__ bool q_upper_proves(const QUpper& me, float s, float r, float hi, int c) {
+  return r <= me.e && __builtin_fmaf(me.m2s * s, (float)c, __builtin_fmaf(me.e2, r, hi)) <= me.K;
 }
 
 // Threshold of the prune's bound for a candidate at stored distance sd: a

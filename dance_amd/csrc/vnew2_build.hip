@@ -259,11 +259,11 @@ static int build_qbound(const Rows& rows, DevBuf& buf, hipStream_t s, QBoundSet*
 // build then launches no k_init at L <= 128).
 static int launch_search(const Rows& rows, GraphBufs g, uint32_t L, uint32_t steps, float alpha, uint32_t start,
                          const uint32_t* order, VCounters* ctr, const QBoundSet& qb, hipStream_t s,
-                         bool insert_bound, bool hashed_cur) {
+                         bool insert_bound, bool hashed_cur, bool padded) {
   const int cpl = pick_cpl(rows.rs.nch);
   const uint32_t Cp = round64(g.C);
   const size_t lds = (size_t)kWavesPerBlock * search_lds_words(Cp) * 4;
-  SearchArgs a{rows.rs, g, L, steps, start, alpha, order, ctr, qb};
+  SearchArgs a{rows.rs, g, L, steps, start, alpha, order, ctr, qb, padded};
   if (L > kMaxBuildL) {
     std::fprintf(stderr, "[dance_hip] L=%u exceeds the supported maximum %u\n", L, kMaxBuildL);
     return -1;
@@ -785,7 +785,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     DCHECK(record(iev[it].s0, s));
     const QBoundSet qb_it = ((q_iters >> it) & 1u) ? qb : QBoundSet{nullptr, 0.0f, 0.0f};
     DCHECK(launch_search(rows, g, L, steps, alpha, start, order, ctr, qb_it, s, ((ib_iters >> it) & 1u) != 0,
-                         it == 0));  // k_init wrote cur just before
+                         it == 0, true));  // k_init wrote cur just before
     DCHECK(record(iev[it].s1, s));
     RevCsr rev{};
     DCHECK(build_reverse_csr(g, rws, s, &rev));
@@ -1123,12 +1123,11 @@ __global__ __launch_bounds__(kBlock) void k_qbound_pairs(QBoundSet qb, const uin
     // the querying row differs per octet here, so its header is read per lane
     const uint4* qa = qb.rows + (size_t)(act ? a[k] : 0u) * kQChunks;
     const uint4 h = qa[0];
-    const QSelf me{qa, __uint_as_float(h.x), __uint_as_float(h.y), __uint_as_float(h.z)};
-    const float t = ((act ? T[k] : 0.0f) + qb.eta) * (1.0f + qb.kappa2);
-    const float sT = (__builtin_sqrtf(t) + me.r) * (1.0f + kQSlack);
-    const uint4 code = qa[sub];
+    const float s = __uint_as_float(h.x), r = __uint_as_float(h.y), lo = __uint_as_float(h.z);
+    const QLower me = q_lower(s, r, lo, q_threshold(qb, r, act ? T[k] : 0.0f));
+    const uint4 code = q_codes(qa[sub], sub);
     const uint4 bc = q_load(qb, act ? b[k] : 0u, act, sub);
-    const bool rej = q_proves_reject(me, code, sT, bc, act, sub);
+    const bool rej = q_proves_reject(me, code, bc);
     if (act && sub == 0) flag[k] = rej ? 1u : 0u;
   }
 }
@@ -1152,16 +1151,16 @@ __global__ __launch_bounds__(kBlock) void k_insert_bound_pairs(QBoundSet qb, con
     // x differs per octet here, so its header is read per lane
     const uint4* qx = qb.rows + (size_t)(act ? a[k] : 0u) * kQChunks;
     const uint4 h = qx[0];
-    const float xs = __uint_as_float(h.x), xr = __uint_as_float(h.y), xa = __uint_as_float(h.z);
+    const float xs = __uint_as_float(h.x), xr = __uint_as_float(h.y);
+    const float xlo = __uint_as_float(h.z), xhi = __uint_as_float(h.w);
     const float t0 = act ? T0[k] : 0.0f;
-    const float ub = q_ub_root_of<DT>(qb, t0, alpha);
-    const float lbT = (prune_bound_root(qb, t0, alpha) + xr) * (1.0f + kQSlack);
-    const uint4 xcode = qx[sub];
+    const QUpper up = q_upper(xs, xr, xhi, q_ub_root_of<DT>(qb, t0, alpha));
+    const QLower low = q_lower(xs, xr, xlo, (prune_bound_root(qb, t0, alpha) + xr) * (1.0f + kQSlack));
     const uint4 bc = q_load(qb, act ? b[k] : 0u, act, sub);
-    const int c = q_octet_dot(xcode, bc, sub);
-    const float sy = __uint_as_float(bc.x), ry = __uint_as_float(bc.y), ay = __uint_as_float(bc.z);
-    const bool yes = q_pair_ub(xs, xa, xr, ub, sy, ry, ay, c);
-    const bool no = q_pair_proves(xs, xa, lbT, sy, ry, ay, c);
+    const int c = q_octet_dot(q_codes(qx[sub], sub), bc);
+    const float sy = __uint_as_float(bc.x), ry = __uint_as_float(bc.y);
+    const bool yes = q_upper_proves(up, sy, ry, __uint_as_float(bc.w), c);
+    const bool no = q_lower_proves(low, sy, ry, __uint_as_float(bc.z), c);
     if (act && sub == 0) out[k] = yes ? 1u : (no ? 2u : 0u);
   }
 }
@@ -1901,7 +1900,7 @@ int dance_stage_search(const void* h_data, int dtype, uint32_t N, uint32_t dim, 
   QBoundSet qb{};
   DCHECK(build_qbound(cx.rows, qbuf, cx.s, &qb));
   DCHECK(launch_search(cx.rows, cx.st.g(), L, steps, alpha, start, nullptr, nullptr, qb, cx.s,
-                       (insert_bound_iters() & 1u) != 0, false));  // cur comes from the caller
+                       (insert_bound_iters() & 1u) != 0, false, false));  // cur comes from the caller
   return download_state(cx.st, cur, deg_cur, work, deg_work, wd, cx.s);
 }
 

@@ -7,6 +7,15 @@
 // this search, and the vertex's own vector in VGPRs. Distances are gathered by
 // octets (see wave.h), 16 pairs in flight per wave.
 //
+// What bounds the searches: iteration 0 the random 128-byte gathers (55-64
+// billion lines a second, whichever memory level serves them); iterations 1-3
+// instruction issue, the scalar port first (79-85% of its rate on uint8
+// rows). So masks come from the predicate at hand instead of being rebuilt
+// from counts, states that only change once (the full pool, the clean row)
+// are flags, and distances are written by every lane of an octet instead of
+// under a lane mask: the searches of iterations 1-3 at 2M x 128 uint8 took
+// 69.5 / 75.3 / 95.3 ms before and 60.7 / 66.3 / 86.0 ms with these.
+//
 // Semantics follow /root/reference/src/gpu_vamana_vnew2.cu exactly; each
 // kernel cites the reference kernel it replaces. The visited cache never
 // changes a result: re-inserting an id the pool has already handled is a no-op
@@ -120,39 +129,77 @@ __device__ __forceinline__ bool valid_for(uint32_t id, uint32_t N, uint32_t node
 // Register-resident bounded top-L pool (vnew2.cu:520-734).
 //
 // Slot p = r*64 + lane lives in register r of that lane. Besides the id, each
-// slot keeps two ordering keys so that the max and the selection are one
-// wave reduction each, with no per-slot validity tests:
-//   mkey: the distance bits (an order-preserving int for non-negative floats)
-//         of a valid entry with a non-NaN distance, INT_MIN otherwise; the
-//         largest mkey, lowest slot, is the pool's worst entry.
-//   skey: mkey of an entry that can still be expanded (not expanded,
-//         distance < FLT_MAX), INT_MAX otherwise; the smallest skey, lowest
-//         slot, is the next entry to expand.
-// Distances are non-negative (squared L2), so mkey also stores the distance
-// itself; NaN entries (mkey INT_MIN) are never read back as distances.
+// slot keeps an ordering key, so that the max and the selection are one wave
+// reduction each, with no per-slot validity tests:
+//   key: the distance bits (an order-preserving int for non-negative floats)
+//        of a valid entry with a non-NaN distance, INT_MIN otherwise; the
+//        largest key, lowest slot, is the pool's worst entry.
+// The smallest key among the slots that can still be expanded (not expanded,
+// distance < FLT_MAX; see OpenSlots), lowest slot, is the next entry to expand.
+// Distances are non-negative (squared L2), so the key also stores the distance
+// itself; NaN entries (key INT_MIN) are never read back as distances.
 // ---------------------------------------------------------------------------
 constexpr int kSelLimit = 0x7F7FFFFF;  // bits of FLT_MAX: keys below it are selectable
 
-__device__ __forceinline__ int pool_mkey(float d) { return d == d ? __float_as_int(d) : INT_MIN; }
-__device__ __forceinline__ int pool_skey(int mk) { return mk != INT_MIN && mk < kSelLimit ? mk : INT_MAX; }
+__device__ __forceinline__ int pool_key(float d) { return d == d ? __float_as_int(d) : INT_MIN; }
+
+// Which slots can still be expanded. Pools of 2 slots per lane keep a second
+// key per slot (the key while it can be expanded, else INT_MAX), which the
+// selection reads directly; larger pools keep one bit per slot in a register
+// per lane: 4 registers fewer at 4 slots per lane, which is a wave more per
+// SIMD there (fp16 rows of 100 dims, L 150: searches of iterations 1-3 18.9 /
+// 19.9 / 24.4 -> 17.3 / 18.2 / 22.3 ms; at 2 slots per lane the bits' tests
+// cost more than they save: 38.9 -> 39.9 ms at 1M x 96).
+template <int PS, bool KEYS = (PS <= 2)>
+struct OpenSlots {
+  int k[PS];
+  __device__ __forceinline__ void init() {
+#pragma unroll
+    for (int r = 0; r < PS; ++r) k[r] = INT_MAX;
+  }
+  // `hit` lanes' slot r opens with the given key (a number or INT_MIN)
+  __device__ __forceinline__ void open(int r, bool hit, int key) {
+    const int v = key != INT_MIN && key < kSelLimit ? key : INT_MAX;
+    k[r] = hit ? v : k[r];
+  }
+  __device__ __forceinline__ void close(int r, bool hit) { k[r] = hit ? INT_MAX : k[r]; }
+  __device__ __forceinline__ int at(int r, int) const { return k[r]; }
+};
+template <int PS>
+struct OpenSlots<PS, false> {
+  uint32_t bits;
+  __device__ __forceinline__ void init() { bits = 0u; }
+  __device__ __forceinline__ void open(int r, bool hit, int key) {
+    const uint32_t b = 1u << r, v = key != INT_MIN && key < kSelLimit ? b : 0u;
+    bits = hit ? ((bits & ~b) | v) : bits;
+  }
+  __device__ __forceinline__ void close(int r, bool hit) { bits = hit ? (bits & ~(1u << r)) : bits; }
+  __device__ __forceinline__ int at(int r, int key) const { return (bits >> r) & 1u ? key : INT_MAX; }
+};
 
 template <int PS>
 struct RegPool {
   uint32_t id[PS];
-  int mkey[PS];
-  int skey[PS];
+  int key[PS];
+  OpenSlots<PS> open;
   uint32_t size;
   int max_pos;
   float max_d;
   uint32_t L;
+  bool full;  // update_full's answer: from then on it stays true
+
+  // Whether every slot is taken and the worst entry is a finite number, which
+  // later inserts preserve (the worst only decreases).
+  __device__ __forceinline__ void update_full() { full = size >= L && max_pos >= 0 && max_d <= FLT_MAX; }
 
   __device__ __forceinline__ void init(uint32_t L_) {
 #pragma unroll
     for (int r = 0; r < PS; ++r) {
       id[r] = DANCE_INV;
-      mkey[r] = INT_MIN;
-      skey[r] = INT_MAX;
+      key[r] = INT_MIN;
     }
+    open.init();
+    full = false;
     size = 0u;
     max_pos = -1;
     max_d = -FLT_MAX;
@@ -171,7 +218,7 @@ struct RegPool {
     int v = INT_MIN;
 #pragma unroll
     for (int r = 0; r < PS; ++r)
-      if (r == (pos >> 6)) v = mkey[r];
+      if (r == (pos >> 6)) v = key[r];
     const int k = __builtin_amdgcn_readlane(v, pos & 63);
     return k == INT_MIN ? __builtin_nanf("") : __int_as_float(k);
   }
@@ -181,40 +228,15 @@ struct RegPool {
   static __device__ __forceinline__ bool at_slot(uint32_t lane, int r, int pos) {
     return lane == (uint32_t)pos - 64u * (uint32_t)r;
   }
-  // Slot updates are select instructions on every lane (no divergent
-  // branch, so no register copies at the merge).
-  __device__ __forceinline__ void set_slot(int pos, uint32_t nid, float nd, uint32_t lane) {
-    const int mk = pool_mkey(nd), sk = pool_skey(mk);
-#pragma unroll
-    for (int r = 0; r < PS; ++r) {
-      const bool h = at_slot(lane, r, pos);
-      id[r] = h ? nid : id[r];
-      mkey[r] = h ? mk : mkey[r];
-      skey[r] = h ? sk : skey[r];
-    }
-  }
-  __device__ __forceinline__ void set_d(int pos, float nd, uint32_t lane) {
-    const int mk = pool_mkey(nd), sk = pool_skey(mk);
-#pragma unroll
-    for (int r = 0; r < PS; ++r) {
-      const bool h = at_slot(lane, r, pos);
-      mkey[r] = h ? mk : mkey[r];
-      skey[r] = h ? sk : skey[r];
-    }
-  }
-  __device__ __forceinline__ void set_expanded(int pos, uint32_t lane) {
-#pragma unroll
-    for (int r = 0; r < PS; ++r) skey[r] = at_slot(lane, r, pos) ? INT_MAX : skey[r];
-  }
 
   // recompute_max_pos_size_warp: largest distance, lowest slot on ties.
   // kHasNumber: the caller knows some slot holds a non-NaN distance, so the
-  // empty case (every mkey INT_MIN) cannot occur and is not tested.
+  // empty case (every key INT_MIN) cannot occur and is not tested.
   template <bool kHasNumber = false>
   __device__ __forceinline__ void recompute_max() {
-    int best = mkey[0];
+    int best = key[0];
 #pragma unroll
-    for (int r = 1; r < PS; ++r) best = max(best, mkey[r]);
+    for (int r = 1; r < PS; ++r) best = max(best, key[r]);
     const int M = wave_max_i(best);
     if (!kHasNumber && M == INT_MIN) {
       max_pos = -1;
@@ -225,7 +247,7 @@ struct RegPool {
 #pragma unroll
     for (int r = 0; r < PS; ++r) {
       if (pos < 0) {
-        const uint64_t m = wballot(mkey[r] == M);
+        const uint64_t m = wballot(key[r] == M);
         if (m) pos = r * 64 + ffs64(m);
       }
     }
@@ -251,14 +273,14 @@ struct RegPool {
     const bool append = same < 0 && size < L;
     const bool replace = same < 0 && size >= L && max_pos >= 0 && nd < max_d;
     const int pos = same >= 0 ? same : (append ? (int)size : max_pos);
-    const int mk = pool_mkey(nd), sk = pool_skey(mk);
+    const int mk = pool_key(nd);
     const bool any = refresh || append || replace;
 #pragma unroll
     for (int r = 0; r < PS; ++r) {
       const bool h = any && at_slot(lane, r, pos);
       id[r] = h ? nid : id[r];  // a duplicate keeps its id
-      mkey[r] = h ? mk : mkey[r];
-      skey[r] = h ? sk : skey[r];
+      key[r] = h ? mk : key[r];
+      open.open(r, h, mk);
     }
     if (append) {
       size = uni_u(size + 1u);
@@ -271,8 +293,8 @@ struct RegPool {
     }
   }
 
-  // insert() for a pool with size >= L and max_pos >= 0 (which every path
-  // below preserves) and a valid candidate id.
+  // insert() for a pool with size >= L, max_pos >= 0 and max_d <= FLT_MAX
+  // (which every path below preserves) and a valid candidate id.
   // The slot registers are updated by selects (no branch around them), so
   // the compiler keeps them in place instead of copying them at every join;
   // the uniform branches are the rare refresh of a duplicate and the max
@@ -280,9 +302,8 @@ struct RegPool {
   //
   // An id already in the pool (rare: the visited cache filters repeats until
   // it forgets them) refreshes its slot when closer. A new id replaces the
-  // worst slot; its distance is below max_d, so not NaN: its mkey is its bits
-  // and its skey those bits unless the distance is FLT_MAX or more (below an
-  // infinite worst entry), which pool_skey marks unselectable.
+  // worst slot; its distance is below max_d, so not NaN and below FLT_MAX: its
+  // key is its bits and the slot can be expanded.
   __device__ __forceinline__ void insert_full(uint32_t nid, float nd, uint32_t lane) {
     if (!(nd < max_d)) return;  // uniform; a NaN distance changes nothing either
     uint64_t dup = 0;
@@ -306,42 +327,55 @@ struct RegPool {
       moved = same == max_pos;
     }
     const int mk = __float_as_int(nd);
-    const int sk = mk < kSelLimit ? mk : INT_MAX;
 #pragma unroll
     for (int r = 0; r < PS; ++r) {
       const bool h = at_slot(lane, r, pos);
       id[r] = h ? nid : id[r];
-      mkey[r] = h ? mk : mkey[r];
-      skey[r] = h ? sk : skey[r];
+      key[r] = h ? mk : key[r];
+      if constexpr (PS <= 2)
+        open.k[r] = h ? mk : open.k[r];
+      else
+        open.bits = h ? (open.bits | (1u << r)) : open.bits;
     }
     if (moved) recompute_max<true>();  // nd is a number
   }
 
   // select_next_unexpanded_size_warp: smallest distance among unexpanded
-  // entries with distance < FLT_MAX, lowest slot on ties; -1 if none. The
-  // selected entry's distance goes to *dist (its skey holds the bits).
-  __device__ __forceinline__ int select(float* dist) const {
-    int best = skey[0];
+  // entries with distance < FLT_MAX, lowest slot on ties; false if none. The
+  // entry is marked expanded; its id and distance (its key holds the bits) go
+  // to *x and *dist.
+  __device__ __forceinline__ bool select_expand(uint32_t lane, uint32_t* x, float* dist) {
+    int k[PS];
 #pragma unroll
-    for (int r = 1; r < PS; ++r) best = min(best, skey[r]);
+    for (int r = 0; r < PS; ++r) k[r] = open.at(r, key[r]);
+    int best = k[0];
+#pragma unroll
+    for (int r = 1; r < PS; ++r) best = min(best, k[r]);
     const int M = wave_min_i(best);
-    if (M == INT_MAX) return -1;
+    if (M == INT_MAX) return false;
     *dist = __int_as_float(M);
-    int pos = -1;
+    // the lowest register that holds M, and its lowest lane
+    int at = 0, reg = PS - 1;
+    uint32_t v = id[PS - 1];
 #pragma unroll
-    for (int r = 0; r < PS; ++r) {
-      if (pos < 0) {
-        const uint64_t m = wballot(skey[r] == M);
-        if (m) pos = r * 64 + ffs64(m);
-      }
+    for (int r = PS - 1; r >= 0; --r) {
+      const uint64_t m = wballot(k[r] == M);
+      at = m ? ffs64(m) : at;
+      reg = m ? r : reg;
+      v = m ? id[r] : v;
     }
-    return pos;
+    *x = rdlane_u(v, at);
+#pragma unroll
+    for (int r = 0; r < PS; ++r) open.close(r, at_slot(lane, r, at + 64 * reg));
+    return true;
   }
 };
 
 __device__ __forceinline__ uint32_t vis_slot(uint32_t id) {
-  if constexpr (kVis == (1u << kVisBits)) return (id * 0x9E3779B1u) >> (32 - kVisBits);
-  return __umulhi(id * 0x9E3779B1u, kVis);
+  // multiplicative hash of the id's low 24 bits, scaled to the slot count: two
+  // full-rate 24-bit multiplies
+  const uint32_t h = __umul24(id, 0x9E3779u) & 0xFFFFFFu;
+  return (uint32_t)(((uint64_t)h * (uint64_t)(kVis << 8)) >> 32);
 }
 
 // Neighbour i of `node` in the random initial graph: the cur rows k_init
@@ -359,6 +393,9 @@ struct SearchArgs {
   const uint32_t* order;  // optional processing order (vertex = order[wave])
   VCounters* ctr;
   QBoundSet qb;  // quantized lower bound (qb.rows == nullptr: exact distances only)
+  // cur rows hold DANCE_INV past their degree (every graph the build makes):
+  // an expansion then needs no degree, one cache line less to gather
+  bool padded;
 };
 
 // Per-wave LDS words of the search kernel: visited cache, work row (ids,
@@ -386,7 +423,8 @@ struct SearchWave {
   RegPool<PS> P;
   QSelf qme;
   uint32_t wdeg;
-  uint32_t n_search, n_insert, n_skip, n_mut, n_try, n_bchk, n_bskip, n_ibchk, n_ibskip;
+  bool clean;  // every entry of the row is usable
+  uint32_t n_search, n_insert, n_skip, n_mut, n_bchk, n_bskip, n_ibchk, n_ibskip;
   uint64_t c_select = 0, c_insert = 0, c_dist = 0, c_pool = 0;
 
   __device__ SearchWave(const SearchArgs& args, uint32_t node_, uint32_t* base, uint32_t Cp_)
@@ -400,16 +438,25 @@ struct SearchWave {
     lst = reinterpret_cast<uint32_t*>(wdd + Cp);
     lsd = reinterpret_cast<float*>(lst + 64);
     ord = reinterpret_cast<uint32_t*>(lsd + 64);
-    n_search = n_insert = n_skip = n_mut = n_try = n_bchk = n_bskip = n_ibchk = n_ibskip = 0;
+    n_search = n_insert = n_skip = n_mut = n_bchk = n_bskip = n_ibchk = n_ibskip = 0;
   }
 
   // Drops from lst[0..n) the candidates whose distance the quantized bound
   // proves >= the pool threshold (they would be rejected unseen); keeps the
-  // others in order and returns their count.
+  // others in order and returns their count. The kept ids of a pass move down
+  // at once: a pass writes at or below the entries it read.
+  // A pass of 8 costs about 20 vector instructions (load address, 4 dot4, 3
+  // DPP adds, the test, the move); with the test on the unexpanded form of the
+  // bound (12 instructions instead of 5) and the kept bits of all passes
+  // gathered before one move, the bounded searches took 4-6% more (4M x 96,
+  // last iteration 318 ms then, 306 ms with this).
   __device__ __forceinline__ uint32_t bound_filter(uint32_t n) {
-    const float sT = q_threshold(a.qb, qme, P.max_d);
-    const uint4 code = qme.row[sub];
-    uint64_t keep = 0;
+    QLower me = q_lower(qme.s, qme.r, qme.lo, q_threshold(a.qb, qme.r, P.max_d));
+    me.m2s = uni_f(me.m2s);
+    me.n2S = uni_f(me.n2S);
+    me.K = uni_f(me.K);
+    const uint4 code = q_codes(qme.row[sub], sub);
+    uint32_t nk = 0;
     for (uint32_t p = 0; p < n; p += 8 * kQInFlight) {
       uint4 b[kQInFlight];
 #pragma unroll
@@ -417,23 +464,19 @@ struct SearchWave {
         const uint32_t k = p + 8 * u + grp;
         b[u] = q_load(a.qb, lst[k], k < n, sub);  // k < 64 (p steps by 8 kQInFlight, which divides 64)
       }
-      bool rej[kQInFlight];
 #pragma unroll
-      for (uint32_t u = 0; u < kQInFlight; ++u)
-        rej[u] = q_proves_reject(qme, code, sT, b[u], p + 8 * u + grp < n, sub);
-#pragma unroll
-      for (uint32_t u = 0; u < kQInFlight; ++u)
-        keep |= (uint64_t)octet_bits(wballot(sub == 0 && p + 8 * u + grp < n && !rej[u])) << (p + 8 * u);
+      for (uint32_t u = 0; u < kQInFlight; ++u) {
+        if (p + 8 * u >= n) break;  // uniform
+        const uint32_t k = p + 8 * u + grp;
+        const bool keep = !q_proves_reject(me, code, b[u]) && sub == 0u && k < n;
+        const uint64_t m = wballot(keep);
+        if (keep) lst[nk + mbcnt64(m)] = lst[k];
+        nk += popc64(m);
+      }
     }
-    const uint32_t nk = popc64(keep);
     n_bchk += n;
     n_bskip += n - nk;
-    if (nk < n) {
-      const uint32_t ck = lst[lane];
-      wave_sync();
-      if ((keep >> lane) & 1ull) lst[mbcnt64(keep)] = ck;
-      wave_sync();
-    }
+    wave_sync();
     return nk;
   }
 
@@ -454,7 +497,7 @@ struct SearchWave {
     if (need) lst[mbcnt64(m)] = c;
     wave_sync();
     const uint64_t t0 = dclock();
-    const bool full = P.size >= P.L && P.max_pos >= 0;
+    const bool full = P.full;
     const uint32_t nx = (QB && full && a.qb.rows) ? bound_filter(n) : n;
     if (nx) batch_dist<DT, CPL>(a.rs, av, av_sq, lst, lsd, nx, grp, sub);
     n_search += nx;
@@ -462,23 +505,19 @@ struct SearchWave {
     c_dist += t1 - t0;
     const uint32_t ck = lst[lane];  // read only where lane < nx (keep below)
     const float dk = lsd[lane];
-    uint64_t km = lanes_below(nx);
-    if (full) km &= wballot(dk < P.max_d);
     if (full) {
       // A pool that starts the batch full stays full with a valid worst
       // entry, so insert() reduces to: reject unless below the worst,
       // refresh a duplicate, else replace the worst slot.
+      uint64_t km = wballot(lane < nx && dk < P.max_d);
       while (km) {
         const int k = ffs64(km);
-        km &= ~(1ull << k);
+        clear_bit(km, k);
         P.insert_full(rdlane_u(ck, k), rdlane_f(dk, k), lane);
       }
     } else {
-      while (km) {
-        const int k = ffs64(km);
-        km &= ~(1ull << k);
-        P.insert(rdlane_u(ck, k), rdlane_f(dk, k), lane);
-      }
+      for (uint32_t k = 0; k < nx; ++k) P.insert(rdlane_u(ck, (int)k), rdlane_f(dk, (int)k), lane);
+      P.update_full();
     }
     if (need) vis[slot] = c;
     wave_sync();
@@ -575,7 +614,7 @@ struct SearchWave {
   }
 
   // The occlusion test of robust_insert with the insert bound: a pass of 8
-  // candidates first tests its pairs on the code rows (x's chunk in xcode).
+  // candidates first tests its pairs on the code rows (x's chunk in xchunk).
   // An upper bound that proves fl(alpha * d(y, x)) <= d_px proves an
   // occluder and ends the test; pairs whose lower bound proves the opposite
   // need nothing more; the others collect their ids in lst and lsd (128
@@ -583,14 +622,16 @@ struct SearchWave {
   // distances, in passes of 8, once the bound passes end. The answer is the
   // exact test's: every decision the bounds make is the one the exact
   // distance would give, and the answer does not depend on the order.
-  __device__ __forceinline__ bool occlusion_bounded(uint32_t x, float dpx, const uint4& xcode, uint32_t nU,
+  __device__ __forceinline__ bool occlusion_bounded(uint32_t x, float dpx, const uint4& xchunk, uint32_t nU,
                                                     uint32_t nA) {
     // x's header: lane 0 holds chunk 0 of its code row
-    const float xs = __uint_as_float(rdlane_u(xcode.x, 0));
-    const float xr = __uint_as_float(rdlane_u(xcode.y, 0));
-    const float xa = __uint_as_float(rdlane_u(xcode.z, 0));
-    const float ub = q_ub_root_of<DT>(a.qb, dpx, a.alpha);
-    const float lbT = (prune_bound_root(a.qb, dpx, a.alpha) + xr) * (1.0f + kQSlack);
+    const float xs = __uint_as_float(rdlane_u(xchunk.x, 0));
+    const float xr = __uint_as_float(rdlane_u(xchunk.y, 0));
+    const float xlo = __uint_as_float(rdlane_u(xchunk.z, 0));
+    const float xhi = __uint_as_float(rdlane_u(xchunk.w, 0));
+    const QUpper up = q_upper(xs, xr, xhi, q_ub_root_of<DT>(a.qb, dpx, a.alpha));
+    const QLower low = q_lower(xs, xr, xlo, (prune_bound_root(a.qb, dpx, a.alpha) + xr) * (1.0f + kQSlack));
+    const uint4 xcode = q_codes(xchunk, sub);
     uint32_t* pend = lst;
     uint32_t nopen = 0;
     for (uint32_t p = 0; p < nA; p += 8) {
@@ -598,16 +639,17 @@ struct SearchWave {
       const bool a0 = k0 < nA;
       const uint32_t y0 = a0 ? wid[ord[nU + k0]] : 0u;
       const uint4 b = q_load(a.qb, y0, a0, sub);
-      const int c = q_octet_dot(xcode, b, sub);
-      const float sy = __uint_as_float(b.x), ry = __uint_as_float(b.y), ay = __uint_as_float(b.z);
+      const int c = q_octet_dot(xcode, b);
+      const float sy = __uint_as_float(b.x), ry = __uint_as_float(b.y);
+      const float loy = __uint_as_float(b.z), hiy = __uint_as_float(b.w);
       const bool lead = sub == 0u && a0;
       const uint32_t np = min(8u, nA - p);
       n_ibchk += np;
-      if (wballot(lead && q_pair_ub(xs, xa, xr, ub, sy, ry, ay, c))) {
+      if (wballot(lead && q_upper_proves(up, sy, ry, hiy, c))) {
         n_ibskip += np;
         return true;
       }
-      const uint64_t und = wballot(lead && !q_pair_proves(xs, xa, lbT, sy, ry, ay, c));
+      const uint64_t und = wballot(lead && !q_lower_proves(low, sy, ry, loy, c));
       n_ibskip += np - popc64(und);
       if (lead && ((und >> lane) & 1ull)) pend[nopen + popc64(und & lanes_below(lane))] = y0;
       nopen += popc64(und);
@@ -624,18 +666,17 @@ struct SearchWave {
       uint4 b0[CPL];
       load_row<CPL>(a.rs, pend[act ? k : 0u], act, sub, b0);
       const float d0 = octet_finish<DT, CPL>(a.rs, sub, xv, b0, self_term<DT, CPL>(xv));
-      occ = (wballot(a.alpha * d0 <= dpx) & kOctetLeads & lanes_below(8u * (nopen - q))) != 0;
+      occ = wballot(act && a.alpha * d0 <= dpx) != 0;
     }
     n_insert += min(q, nopen);  // distances of the passes made
     wave_sync();
     return occ;
   }
 
-  // dynamic_robust_insert_C_warp (vnew2.cu:759-877) on the LDS work row.
+  // dynamic_robust_insert_C_warp (vnew2.cu:759-877) on the LDS work row. x is a
+  // pool entry: a valid id other than the vertex, at a distance below FLT_MAX.
   __device__ __forceinline__ void robust_insert(uint32_t x, float dpx) {
     const uint32_t N = a.g.N, C = a.g.C;
-    if (x == DANCE_INV || x >= N || x == node) return;
-    n_try++;
     // With the insert bound the occlusion test starts from x's code chunk
     // and x's row is loaded where exact distances are needed; otherwise x's
     // row is requested first (x < N), so its load overlaps the pass below (a
@@ -648,20 +689,35 @@ struct SearchWave {
     else
       load_row<CPL>(a.rs, x, true, sub, xv);
     // One pass over the row: x already there ends the insert; otherwise the
-    // usable entries nearer than x (nA, of which nL strictly) and farther
-    // (nB); dpx is a number, so a usable entry is exactly one of nA and nB.
+    // usable entries at most as far as x (nA; tie: those at the same distance)
+    // and farther (nB); dpx is a number, so a usable entry is exactly one of nA and nB.
     // The rest (nU), unusable, rank lowest in the order.
-    uint32_t nA = 0, nL = 0, nB = 0;
-    for (uint32_t b = 0; b < wdeg; b += 64) {
-      const uint32_t i = b + lane;  // < Cp: b < wdeg <= Cp, both multiples of 64
-      const uint64_t in = lanes_below(wdeg - b);
-      const uint32_t y = wid[i];
-      if (in & wballot(y == x)) return;
-      const float dpy = wdd[i];
-      const uint64_t v = in & wballot(y < N) & wballot(y != node);
-      nA += popc64(v & wballot(dpy <= dpx));
-      nL += popc64(v & wballot(dpy < dpx));
-      nB += popc64(v & wballot(dpy > dpx));
+    uint32_t nA = 0, nB = 0;
+    uint64_t dup = 0, tie = 0;  // x in the row; entries at distance dpx
+    if (clean) {
+      // every entry usable, and the slots past the row hold (DANCE_INV,
+      // FLT_MAX), which match nothing here (dpx is below FLT_MAX): no masks
+      for (uint32_t b = 0; b < wdeg; b += 64) {
+        const uint32_t i = b + lane;  // < Cp: b < wdeg <= Cp, both multiples of 64
+        const float dpy = wdd[i];
+        dup |= wballot(wid[i] == x);
+        nA += popc64(wballot(dpy <= dpx));
+        tie |= wballot(dpy == dpx);
+      }
+      if (dup) return;
+      nB = wdeg - nA;
+    } else {
+      for (uint32_t b = 0; b < wdeg; b += 64) {
+        const uint32_t i = b + lane;
+        const uint64_t in = lanes_below(wdeg - b);
+        const uint32_t y = wid[i];
+        if (in & wballot(y == x)) return;
+        const float dpy = wdd[i];
+        const uint64_t v = in & wballot(y < N) & wballot(y != node);
+        nA += popc64(v & wballot(dpy <= dpx));
+        nB += popc64(v & wballot(dpy > dpx));
+        tie |= v & wballot(dpy == dpx);
+      }
     }
     const uint32_t nU = wdeg - nA - nB;
     // Occlusion: exists y with d_py <= d_px and alpha * d(y, x) <= d_px. The
@@ -684,7 +740,7 @@ struct SearchWave {
         uint4 b0[CPL];
         load_row<CPL>(a.rs, y0, a0, sub, b0);
         const float d0 = octet_finish<DT, CPL>(a.rs, sub, xv, b0, xv_sq);
-        occluded = (wballot(a.alpha * d0 <= dpx) & kOctetLeads & lanes_below(8u * (nA - p))) != 0;
+        occluded = wballot(a0 && a.alpha * d0 <= dpx) != 0;  // the octet's 8 lanes agree
       }
       n_insert += min(p, nA);  // distances of the passes made
       if (occluded) return;
@@ -713,9 +769,9 @@ struct SearchWave {
       uint4 b0[CPL];
       load_row<CPL>(a.rs, y0, a0, sub, b0);
       const float d0 = octet_finish<DT, CPL>(a.rs, sub, xv, b0, xv_sq);
-      const uint64_t hit = wballot(a.alpha * d0 <= wdd[s0]) & kOctetLeads & lanes_below(8u * (nB - p));
+      const uint64_t hit = wballot(a0 && a.alpha * d0 <= wdd[s0]);
       if (hit) {
-        const int l = ffs64(hit);  // lane 8 g + 0 of the first octet that hit
+        const int l = ffs64(hit);  // lane 8 g of the first octet that hit
         vpos = (int)rdlane_u(s0, l);
         vrank = wdeg - 1u - (p + ((uint32_t)l >> 3));
       }
@@ -749,7 +805,7 @@ struct SearchWave {
       // Its new rank: the unusable entries and the usable ones strictly
       // nearer than x rank below it (the replaced entry was farther); ties
       // at distance dpx are ordered by slot, which only a count resolves.
-      ord_update((uint32_t)mslot, dpx, rold, nA == nL ? nU + nL : kRankUnknown, wdeg);
+      ord_update((uint32_t)mslot, dpx, rold, tie == 0 ? nU + nA : kRankUnknown, wdeg);
     }
   }
 
@@ -766,6 +822,7 @@ struct SearchWave {
     // from the cached row), so the build needs no k_init launch.
     const uint32_t deg_self = HC ? (N > 1u ? R : 0u) : min(g.deg_cur[node], R);
     const size_t wb = (size_t)node * C;
+    uint64_t bad = 0;  // lanes that saw an unusable entry of the row
     if constexpr (HC) {
       for (uint32_t b = 0; b < Cp; b += 64) {  // Cp is a multiple of 64
         const uint32_t i = b + lane;
@@ -776,13 +833,16 @@ struct SearchWave {
         if (v) lst[mbcnt64(m)] = nb;
         wave_sync();
         if (n) batch_dist<DT, CPL>(a.rs, av, av_sq, lst, lsd, n, grp, sub);
+        const float dist = v ? lsd[mbcnt64(m)] : FLT_MAX;
         wid[i] = nb;
-        wdd[i] = v ? lsd[mbcnt64(m)] : FLT_MAX;
+        wdd[i] = dist;
+        bad |= wballot(i < deg_self && (!v || dist != dist));
         wave_sync();
       }
     } else {
       const size_t cb = (size_t)node * R;
-      for (uint32_t i = lane; i < Cp; i += 64) {
+      for (uint32_t b = 0; b < Cp; b += 64) {
+        const uint32_t i = b + lane;
         uint32_t nb = DANCE_INV;
         float dist = FLT_MAX;
         if (i < deg_self) {
@@ -794,9 +854,11 @@ struct SearchWave {
         }
         wid[i] = nb;
         wdd[i] = dist;
+        bad |= wballot(i < deg_self && (nb == DANCE_INV || dist != dist));
       }
     }
     wdeg = deg_self;
+    clean = bad == 0;
     P.init(a.L);
     wave_sync();
     ord_init();
@@ -833,12 +895,13 @@ struct SearchWave {
 #pragma unroll
         for (int r = 0; r < PS; ++r) {
           const uint32_t p = (uint32_t)r * 64u + lane;
-          if (p >= base && p < base + n) {
-            const float d = lsd[p - base];
+          const bool in = p >= base && p < base + n;
+          const int k = in ? __float_as_int(lsd[p - base]) : INT_MIN;  // numbers
+          if (in) {
             P.id[r] = lst[p - base];
-            P.mkey[r] = pool_mkey(d);
-            P.skey[r] = pool_skey(P.mkey[r]);
+            P.key[r] = k;
           }
+          P.open.open(r, in, k);
         }
         // sequential appends keep the first strictly larger distance
         const int M = wave_max_i(v ? fkey(dd) : INT_MIN);
@@ -848,6 +911,7 @@ struct SearchWave {
           P.max_d = uni_f(__int_as_float(M));
         }
         P.size = uni_u(base + n);
+        P.update_full();
         if (v) vis[slot] = nb;
         wave_sync();
         appended = true;
@@ -864,6 +928,7 @@ struct SearchWave {
         m &= m - 1;
         P.insert(rdlane_u(nb, k), rdlane_f(dd, k), lane);
       }
+      P.update_full();
       if (v) vis[vis_slot(nb)] = nb;
       wave_sync();
     }
@@ -873,17 +938,14 @@ struct SearchWave {
     uint32_t n_exp = 0;
     const uint64_t t_seed = dclock() - t_run;
     (void)t_seed;
-    for (uint32_t step = 0; step < max_steps; ++step) {
+    while (n_exp < max_steps) {
       const uint64_t ts0 = dclock();
       float dx;
-      const int pos = P.select(&dx);
-      if (pos < 0) break;
-      const uint32_t x = P.get_id(pos);
-      P.set_expanded(pos, lane);
-      if (x == DANCE_INV || x >= N) break;
+      uint32_t x;  // a valid id: only such enter the pool
+      if (!P.select_expand(lane, &x, &dx)) break;
       n_exp++;
       // Issue the adjacency gather of x before the online insert.
-      const uint32_t degx = HC ? (N > 1u ? R : 0u) : min(g.deg_cur[x], R);
+      const uint32_t degx = HC ? (N > 1u ? R : 0u) : a.padded ? R : min(g.deg_cur[x], R);
       const size_t xb = (size_t)x * R;
       uint32_t c0 = DANCE_INV;
       if (lane < degx) c0 = HC ? init_neighbor(x, lane, N) : g.cur[xb + lane];
@@ -910,7 +972,7 @@ struct SearchWave {
         atomicAdd(&ctr_stripe(a.ctr)->expansions, (unsigned long long)n_exp);
         atomicAdd(&ctr_stripe(a.ctr)->vis_skips, (unsigned long long)n_skip);
         atomicAdd(&ctr_stripe(a.ctr)->insert_mut, (unsigned long long)n_mut);
-        atomicAdd(&ctr_stripe(a.ctr)->insert_try, (unsigned long long)n_try);
+        atomicAdd(&ctr_stripe(a.ctr)->insert_try, (unsigned long long)n_exp);  // one per expansion
         if (QB && a.qb.rows) {
           atomicAdd(&ctr_stripe(a.ctr)->bound_checks, (unsigned long long)n_bchk);
           atomicAdd(&ctr_stripe(a.ctr)->bound_skips, (unsigned long long)n_bskip);
@@ -933,21 +995,22 @@ struct SearchWave {
 };
 
 // Waves per SIMD the register allocator must leave room for, for the
-// narrow-row, L <= 128 variants (the common case): DANCE_SEARCH_WAVES_QB
-// (default 5) with the bound compiled in (the allocator would otherwise
-// settle at 4 by a few registers), and DANCE_SEARCH_WAVES (default 6)
-// without it; the exact search fits in 68 registers and runs 7 waves per
-// SIMD (asking for 7 changes nothing); the first-iteration exact variants of
-// one and two chunks per lane (uint8 rows of up to 256 bytes) ask for 8,
-// which their LDS allows at C <= 128, so that the neighbour hash does not
-// push the scalar registers past the 8-wave limit. The insert-bound variants
-// ask for DANCE_SEARCH_WAVES_IB (default 6: 79-80 registers at 3 chunks per
-// lane, no spills). No constraint elsewhere.
+// narrow-row variants: at L <= 128 DANCE_SEARCH_WAVES_QB (default 6) with the
+// bound compiled in, and DANCE_SEARCH_WAVES (default 6) without it; the exact
+// search fits in 70 registers and runs 7 waves per SIMD; the first-iteration
+// exact variants of one and two chunks per lane (uint8 rows of up to 256
+// bytes) ask for 8, which their LDS allows at C <= 128, so that the neighbour
+// hash does not push the scalar registers past the 8-wave limit. The
+// insert-bound variants ask for DANCE_SEARCH_WAVES_IB (default 6: 80 registers
+// at 3 chunks per lane; three row addresses live in scratch. 5 waves: first
+// search at 1M x 96 113 -> 108 ms, at 4M 457 -> 464 ms). At 129 <= L <= 256 two
+// chunks per lane fit 6 waves without the bound and 5 with it. No constraint
+// elsewhere.
 #ifndef DANCE_SEARCH_WAVES
 #define DANCE_SEARCH_WAVES 6
 #endif
 #ifndef DANCE_SEARCH_WAVES_QB
-#define DANCE_SEARCH_WAVES_QB 5
+#define DANCE_SEARCH_WAVES_QB 6
 #endif
 #ifndef DANCE_SEARCH_WAVES_IB
 #define DANCE_SEARCH_WAVES_IB 6
@@ -956,11 +1019,11 @@ template <int CPL, int PS, bool QB, bool IB, bool HC>
 constexpr int kSearchMinWaves =
     (CPL <= 3 && PS == 2)
         ? (IB ? DANCE_SEARCH_WAVES_IB : QB ? DANCE_SEARCH_WAVES_QB : (CPL <= 2 && HC) ? 8 : DANCE_SEARCH_WAVES)
-        : 1;
+        : (CPL <= 2 && PS == 4) ? (QB ? 5 : 6) : 1;
 
 // search_prune_kernel_shared (vnew2.cu:1119-1439).
 template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSearchMinWaves<CPL, PS, QB, IB, HC>))) void k_search(SearchArgs a, uint32_t Cp) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSearchMinWaves<CPL, PS, QB, IB, HC>, 8))) void k_search(SearchArgs a, uint32_t Cp) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t gw = xcd_block(grid_block(), grid_blocks()) * kWavesPerBlock + w;
@@ -1069,9 +1132,10 @@ __global__ __launch_bounds__(kBlock) void k_prune(PruneArgs a, uint32_t Cp, uint
       // Drop the candidates whose pair distance the bound proves large
       // enough to keep them; their exact distance cannot remove them.
       const uint4* qs = a.qb.rows + (size_t)sel * kQChunks;
-      const uint4 code = qs[sub];
-      const QSelf me{qs, __uint_as_float(uni_u(rdlane_u(code.x, 0))), __uint_as_float(uni_u(rdlane_u(code.y, 0))),
-                     __uint_as_float(uni_u(rdlane_u(code.z, 0)))};
+      const uint4 chunk = qs[sub];
+      const float ss = __uint_as_float(rdlane_u(chunk.x, 0)), sr = __uint_as_float(rdlane_u(chunk.y, 0)),
+                  slo = __uint_as_float(rdlane_u(chunk.z, 0));
+      const uint4 code = q_codes(chunk, sub);
       uint32_t nk = 0;
       for (uint32_t base = 0; base < nq; base += 64) {  // lst holds up to C entries
         const uint32_t nb = min(64u, nq - base);
@@ -1088,8 +1152,8 @@ __global__ __launch_bounds__(kBlock) void k_prune(PruneArgs a, uint32_t Cp, uint
 #pragma unroll
           for (uint32_t u = 0; u < kQInFlight; ++u) {
             const uint32_t k = p + 8 * u + grp;
-            const float sT = (sroot[si[u]] + me.r) * (1.0f + kQSlack);
-            const bool prove = q_proves_reject(me, code, sT, b[u], k < nb, sub);
+            const QLower me = q_lower(ss, sr, slo, (sroot[si[u]] + sr) * (1.0f + kQSlack));
+            const bool prove = q_proves_reject(me, code, b[u]);
             keep |= (uint64_t)octet_bits(wballot(sub == 0 && k < nb && !prove)) << (p + 8 * u);
           }
         }
@@ -1213,7 +1277,7 @@ enum : int { kRankExact = 0, kRankBound = 1, kRankGram = 2 };
 // Per-wave LDS: arrays of Cq = C rounded up to 32 entries (ids of the
 // exact-test list; rid, rd by rank; the exact-test list of ranks; per-rank
 // flags), and with MFMA tiles (bound or Gram) 4 words per rank of headers
-// (the bound's {-2 s, r, a, root}, later the open-pair list; the Gram's
+// (the bound's {s, r, lo, root}, later the open-pair list; the Gram's
 // squared row norms) and 4 mask words per rank.
 __host__ __device__ constexpr uint32_t prune_rank_lds_words(uint32_t Cq, bool tiles) {
   return 5u * Cq + (tiles ? 8u * Cq : 0u);
@@ -1265,7 +1329,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
   float* rd = reinterpret_cast<float*>(base + 2 * Cq);  // rank -> distance
   uint32_t* lst = base + 3 * Cq;                      // ranks needing an exact distance
   uint32_t* rmf = base + 4 * Cq;                      // per rank: removed this round / repeated id
-  // QB: per rank {-2 s, r, a, root} (a = -inf past the valid ranks), reused
+  // QB: per rank {s, r, lo, root} (r = inf past the valid ranks), reused
   // after the bound tiles as the list of open pairs; then per rank 4 words:
   // the candidate ranks the bound proves kept, later those it occludes.
   float4* hq = reinterpret_cast<float4*>(base + 5 * Cq);
@@ -1353,10 +1417,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
     for (int h = 0; h < 2; ++h) {
       const uint32_t r = lane + 64u * (uint32_t)h;
       if (r < Cq) {
-        float4 v = make_float4(0.0f, 0.0f, -__builtin_inff(), 0.0f);
+        float4 v = make_float4(0.0f, __builtin_inff(), 0.0f, 0.0f);
         if (r < nvalid) {
           const uint4 hd = a.qb.rows[(size_t)rid[r] * kQChunks];
-          v = make_float4(-2.0f * __uint_as_float(hd.x), __uint_as_float(hd.y), __uint_as_float(hd.z),
+          v = make_float4(__uint_as_float(hd.x), __uint_as_float(hd.y), __uint_as_float(hd.z),
                           prune_bound_root(a.qb, rd[r], a.alpha));
         }
         hq[r] = v;
@@ -1370,18 +1434,17 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
       v16i_t acc = {};
 #pragma unroll
       for (uint32_t s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s], fb[s], acc, 0, 0, 0);
-      // j-side values per lane; i-side per accumulator from LDS. Invalid
-      // ranks carry a = -inf, which fails the test.
+      // j-side values per lane (j queries with its own root); i-side per
+      // accumulator from LDS. Invalid ranks carry r = inf, which proves nothing.
       const uint32_t j = tj * 32u + jl;
       const float4 hj = hq[j];
-      const float sy = -0.5f * hj.x, ry = hj.y, ay = hj.z, rootj = hj.w;
+      const QLower me = q_lower(hj.x, hj.y, hj.z, (hj.w + hj.y) * (1.0f + kQSlack));
       uint32_t words = 0u;  // lane l < 32 collects the proof word of tile row l
       static_for<0, 16>([&](auto vc) {
         constexpr uint32_t v = decltype(vc)::value, ir = 8u * (v >> 2) + (v & 3u);
         const uint32_t i = ti * 32u + ir + ih;
         const float4 hi = hq[i];
-        const float sT = (rootj + hi.y) * (1.0f + kQSlack);
-        const bool pr = i < j && q_pair_proves_m2(hi.x, hi.z, sT, sy, ry, ay, acc[v]);
+        const bool pr = i < j && q_lower_proves(me, hi.x, hi.y, hi.z, acc[v]);
         const uint64_t m = wballot(pr);
         words = write_lane<ir>(words, (uint32_t)m);
         words = write_lane<ir + 4u>(words, (uint32_t)(m >> 32));

@@ -45,6 +45,8 @@ __device__ __forceinline__ int ffs64(uint64_t m) { return __ffsll((unsigned long
 __device__ __forceinline__ uint64_t lanes_below(uint32_t n) { return n >= 64u ? ~0ull : ((1ull << n) - 1ull); }
 // Lane 8 g of each octet g (the lanes that hold an octet's result).
 constexpr uint64_t kOctetLeads = 0x0101010101010101ull;
+// m &= ~(1 << k) in one scalar instruction (k uniform, < 64).
+__device__ __forceinline__ void clear_bit(uint64_t& m, int k) { asm("s_bitset0_b64 %0, %1" : "+s"(m) : "s"(k)); }
 __device__ __forceinline__ uint32_t popc64(uint64_t m) { return (uint32_t)__popcll((unsigned long long)m); }
 
 __device__ __forceinline__ int uni_i(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -326,7 +328,7 @@ __device__ __forceinline__ int fkey(float d) { return __float_as_int(d); }
 
 // Distances from a cached vector `av` to up to 64 ids lst[0..n) -> lsd[0..n).
 // Two passes of 8 octets are kept in flight (one for a last group of <= 8).
-// lst holds 64 entries; every index read stays below 64. Returns after lsd
+// lst and lsd hold 64 entries; every index stays below 64. Returns after lsd
 // is visible.
 template <int DT, int CPL>
 __device__ __forceinline__ void batch_dist(const RowSet& rs, const uint4 (&av)[CPL], uint32_t a_sq,
@@ -342,18 +344,17 @@ __device__ __forceinline__ void batch_dist(const RowSet& rs, const uint4 (&av)[C
     load_row<CPL>(rs, id1, a1, sub, b1);
     const float d0 = octet_finish<DT, CPL>(rs, sub, av, b0, a_sq);
     const float d1 = octet_finish<DT, CPL>(rs, sub, av, b1, a_sq);
-    if (sub == 0) {
-      if (a0) lsd[k0] = d0;
-      if (a1) lsd[k1] = d1;
-    }
+    // every lane writes its octet's distance of one of the two passes: equal
+    // values to equal addresses, no lane masks (the scalar port binds the
+    // searches); entries n and above receive values nobody reads
+    lsd[k0 + 8u * (sub & 1u)] = (sub & 1u) ? d1 : d0;
   }
   if (p < n) {  // a last group of at most 8: one pass
     const uint32_t k0 = p + grp;
     const bool a0 = k0 < n;
     uint4 b0[CPL];
     load_row<CPL>(rs, lst[k0], a0, sub, b0);
-    const float d0 = octet_finish<DT, CPL>(rs, sub, av, b0, a_sq);
-    if (sub == 0 && a0) lsd[k0] = d0;
+    lsd[k0] = octet_finish<DT, CPL>(rs, sub, av, b0, a_sq);
   }
   wave_sync();
 }
