@@ -231,9 +231,12 @@ __global__ __launch_bounds__(kBlock) void k_query(RowSet base, RowSet qrows, QAr
     }
     if ((int)lane == l) P.ex |= 1u << slot;
     ++nexp;
-    const uint32_t du = min(a.deg[u], a.R);
+    // the first entries are requested with the degree, not after it
     const size_t b = (size_t)u * a.R;
-    for (uint32_t j = 0; j < du; j += 64) batch(j + lane < du ? a.g[b + j + lane] : DANCE_INV, true);
+    const uint32_t c0 = lane < a.R ? a.g[b + lane] : DANCE_INV;
+    const uint32_t du = min(a.deg[u], a.R);
+    if (du) batch(lane < du ? c0 : DANCE_INV, true);
+    for (uint32_t j = 64; j < du; j += 64) batch(j + lane < du ? a.g[b + j + lane] : DANCE_INV, true);
   }
   // k best in (distance, id) order: lane i receives the i-th.
   uint32_t taken = 0, oid = DANCE_INV;
