@@ -284,6 +284,7 @@ int locality_order(const Rows& rows, const Labels& Ld, uint32_t N, uint32_t T, F
     hipLaunchKernelGGL(k_task_fill, dim3(grid_thr(N)), dim3(256), 0, s, N, Ld.off, st.rorder.as<const uint32_t>(),
                        pos, st.torder.as<uint32_t>());
     DHIP(hipGetLastError());
+    DCHECK(tasks_by_label(Ld, T, st, sort_ws, s));
     *torder = st.torder.as<const uint32_t>();
   }
   *rorder = st.rorder.as<const uint32_t>();
@@ -530,7 +531,7 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
     if (log) {
       unsigned long long rc[2] = {0, 0};
       DHIP(hipMemsetAsync(st.rcnt.p, 0, sizeof(rc), s));
-      hipLaunchKernelGGL(k_round_changes, dim3((N + 3) / 4), dim3(256), 0, s, N, R, st.prev_g.as<const uint32_t>(),
+      hipLaunchKernelGGL(k_round_changes, dim3(std::min((N + 3) / 4, kChangeBlocks)), dim3(256), 0, s, N, R, st.prev_g.as<const uint32_t>(),
                          st.prev_d.as<const uint32_t>(), static_cast<const uint32_t*>(ga),
                          static_cast<const uint32_t*>(da), static_cast<const uint32_t*>(roff),
                          st.rcnt.as<unsigned long long>());

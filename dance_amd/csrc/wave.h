@@ -140,6 +140,18 @@ __device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb_pad) {
   return (b & 7u) * per + (b >> 3);
 }
 
+// The same with each XCD taking every eighth chunk of kXcdChunk logical blocks,
+// for orders whose work per block drifts along the range (contiguous eighths
+// would leave the XCDs unequal loads). Blocks past the last whole group of
+// chunks keep their own index.
+constexpr uint32_t kXcdChunk = 64;
+__device__ __forceinline__ uint32_t xcd_chunk(uint32_t b, uint32_t nb) {
+  const uint32_t group = 8u * kXcdChunk, g = b / group;
+  if ((g + 1u) * group > nb) return b;
+  const uint32_t i = b - g * group;
+  return g * group + (i & 7u) * kXcdChunk + (i >> 3);
+}
+
 // Reference hashes: vnew2.cu:169-191.
 __device__ __forceinline__ uint32_t d_hash_u32(uint32_t x) {
   x ^= x >> 16;
