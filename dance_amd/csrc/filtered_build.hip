@@ -251,10 +251,31 @@ static uint32_t long_window() {
   return std::min(std::max(v, 64u), kLongList / 2u);
 }
 
+// Groups st.torder by label, keeping the row order within a label: a task's
+// traversal stays among the carriers of its label, so tasks of one label on
+// neighbouring rows share them in L2 (a rare label's whole subgraph fits it),
+// where a row's tasks of different labels share little.
+int tasks_by_label(const Labels& Ld, uint32_t T, FState& st, SortWorkspace& sort_ws, hipStream_t s) {
+  DevBuf keys[2], other;
+  DCHECK(keys[0].alloc((size_t)T * 4));
+  DCHECK(keys[1].alloc((size_t)T * 4));
+  DCHECK(other.alloc((size_t)T * 4));
+  hipLaunchKernelGGL(k_task_keys, dim3(grid_thr(T)), dim3(256), 0, s, T, Ld.num_labels, Ld.lab,
+                     st.torder.as<const uint32_t>(), keys[0].as<uint32_t>());
+  DHIP(hipGetLastError());
+  uint32_t* kb[2] = {keys[0].as<uint32_t>(), keys[1].as<uint32_t>()};
+  uint32_t* vb[2] = {st.torder.as<uint32_t>(), other.as<uint32_t>()};
+  int which = 0;
+  DCHECK(radix_sort_pairs(kb, vb, T, bit_length(Ld.num_labels), sort_ws, s, &which));
+  if (which) DHIP(hipMemcpyAsync(st.torder.p, other.p, (size_t)T * 4, hipMemcpyDeviceToDevice, s));
+  DHIP(hipStreamSynchronize(s));  // the sort's buffers are freed on return
+  return 0;
+}
+
 int locality_order(const Rows& rows, const Labels& Ld, uint32_t N, uint32_t T, FState& st, ScanWorkspace& scan,
                    SortWorkspace& sort_ws, hipStream_t s, const uint32_t** rorder, const uint32_t** torder) {
   const char* e = std::getenv("DANCE_LOCALITY_CELLS");
-  const uint32_t K = std::min(e && e[0] ? (uint32_t)std::strtoul(e, nullptr, 10) : 1024u, N);
+  const uint32_t K = e && e[0] ? std::min((uint32_t)std::strtoul(e, nullptr, 10), N) : cells_for(N, 1024u);
   *rorder = *torder = nullptr;
   if (K < 2) return 0;
   DevBuf piv;
@@ -263,14 +284,19 @@ int locality_order(const Rows& rows, const Labels& Ld, uint32_t N, uint32_t T, F
   DHIP(hipGetLastError());
   uint32_t* kb[2] = {st.lsort.as<uint32_t>(), st.lsort.as<uint32_t>() + N};
   uint32_t* vb[2] = {st.lrows.as<uint32_t>(), st.lsort.as<uint32_t>() + 2 * (size_t)N};
-  DCHECK(with_dt_cpl(rows.dtype, pick_cpl(rows.rs.nch), [&](auto dt, auto c) {
-    hipLaunchKernelGGL((k_cells<decltype(dt)::value, decltype(c)::value>), dim3(cells_grid(N)), dim3(kCellsBlock), 0,
-                       s, rows.rs, N, piv.as<const uint32_t>(), K, cell_levels(K, 3), kb[0], vb[0]);
-    DHIP(hipGetLastError());
-    return 0;
-  }));
+  const uint32_t lv = cell_levels(K, 3);
+  if (rows.dtype == DANCE_U8) {
+    DCHECK(launch_cells_u8(rows, N, piv.as<const uint32_t>(), K, lv, kb[0], vb[0], s));
+  } else {
+    DCHECK(with_cpl(pick_cpl(rows.rs.nch), [&](auto c) {  // float rows are searched as fp16
+      hipLaunchKernelGGL((k_cells<DANCE_F16, decltype(c)::value>), dim3(cells_grid(N)), dim3(kCellsBlock), 0, s,
+                         rows.rs, N, piv.as<const uint32_t>(), K, lv, kb[0], vb[0]);
+      DHIP(hipGetLastError());
+      return 0;
+    }));
+  }
   int which = 0;
-  const uint64_t nkeys = cell_levels(K, 3) == 3u ? (uint64_t)K * K * K : (uint64_t)K;
+  const uint64_t nkeys = lv == 3u ? (uint64_t)K * K * K : (uint64_t)K;
   DCHECK(radix_sort_pairs(kb, vb, N, bit_length((uint32_t)(nkeys - 1)), sort_ws, s, &which));
   DCHECK(st.rorder.alloc((size_t)N * 4));
   DHIP(hipMemcpyAsync(st.rorder.p, vb[which], (size_t)N * 4, hipMemcpyDeviceToDevice, s));

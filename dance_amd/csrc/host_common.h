@@ -16,6 +16,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "locality.h"
 #include "prims.h"
 #include "wave.h"
 
@@ -262,6 +263,18 @@ static __global__ void k_f32_to_f16_rows(const float* __restrict__ src, uint32_t
   if (i >= (size_t)N * dim) return;
   const size_t r = i / dim, c = i % dim;
   dst[r * dst_stride_elems + c] = (_Float16)src[i];  // round to nearest even
+}
+
+// Nearest pivots of uint8 rows from MFMA tiles (k_cells_mfma): keys to `cell`,
+// row ids to `vid`.
+inline int launch_cells_u8(const Rows& rows, uint32_t N, const uint32_t* piv, uint32_t K, uint32_t levels,
+                           uint32_t* cell, uint32_t* vid, hipStream_t s) {
+  return with_cpl(pick_cpl(rows.rs.nch), [&](auto c) {
+    hipLaunchKernelGGL((k_cells_mfma<true, 4 * decltype(c)::value>), dim3((uint32_t)(((uint64_t)N + 127) / 128)),
+                       dim3(256), 0, s, rows.rs.rows, rows.rs.stride16, N, piv, K, levels, cell, vid);
+    DHIP(hipGetLastError());
+    return 0;
+  });
 }
 
 // Copies between pageable host memory and device memory through pinned

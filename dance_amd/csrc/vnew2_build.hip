@@ -553,17 +553,17 @@ static uint32_t alpha_from_iter(uint32_t iters) {
 // (c3 3.588 s at 1024 against 3.596 at 1536 and 3.594 / 3.630 at 512 / 256;
 // c4 2.525 s at 1024 against 2.516 at 1536 and 2.539 at 1625). Uses the
 // reverse-sort buffers as scratch.
-static uint32_t locality_cells(int dtype) {
+static uint32_t locality_cells(int dtype, uint32_t N) {
   const char* e = std::getenv("DANCE_LOCALITY_CELLS");
-  if (e && e[0]) return (uint32_t)std::strtoul(e, nullptr, 10);
-  return dtype == DANCE_U8 ? 1536u : 1024u;
+  if (e && e[0]) return std::min((uint32_t)std::strtoul(e, nullptr, 10), N);
+  return cells_for(N, dtype == DANCE_U8 ? 1536u : 1024u);
 }
 
 
 static int build_schedule(const Rows& rows, const QBoundSet& qb, ReverseWs& ws, hipStream_t s,
                           const uint32_t** order_out) {
   const uint32_t N = rows.N;
-  const uint32_t K = std::min(locality_cells(rows.dtype), N);
+  const uint32_t K = locality_cells(rows.dtype, N);
   *order_out = nullptr;
   if (K < 2) return 0;
   DevBuf dpiv;
@@ -583,7 +583,7 @@ static int build_schedule(const Rows& rows, const QBoundSet& qb, ReverseWs& ws, 
   const bool mfma_cells = !(em && em[0] == '0');
   const dim3 mgrid((uint32_t)(((uint64_t)N + 127) / 128));
   if (qb.rows && mfma_cells) {
-    hipLaunchKernelGGL(k_cells_mfma<false>, mgrid, dim3(256), 0, s, qb.rows, kQChunks, N, dpiv.as<uint32_t>(), K,
+    hipLaunchKernelGGL((k_cells_mfma<false, 4>), mgrid, dim3(256), 0, s, qb.rows, kQChunks, N, dpiv.as<uint32_t>(), K,
                        lv, kb[0], vb[0]);
     DHIP(hipGetLastError());
   } else if (qb.rows) {
@@ -591,10 +591,8 @@ static int build_schedule(const Rows& rows, const QBoundSet& qb, ReverseWs& ws, 
     hipLaunchKernelGGL(k_cells_q<false>, dim3((N + 255) / 256), dim3(256), 0, s, qb.rows, kQChunks, kQChunks, N,
                        dpiv.as<uint32_t>(), K, lv, kb[0], vb[0]);
     DHIP(hipGetLastError());
-  } else if (rows.dtype == DANCE_U8 && rows.rs.stride16 == 8u && mfma_cells) {  // 128-byte rows
-    hipLaunchKernelGGL(k_cells_mfma<true>, mgrid, dim3(256), 0, s, rows.rs.rows, rows.rs.stride16, N,
-                       dpiv.as<uint32_t>(), K, lv, kb[0], vb[0]);
-    DHIP(hipGetLastError());
+  } else if (rows.dtype == DANCE_U8 && mfma_cells) {
+    DCHECK(launch_cells_u8(rows, N, dpiv.as<uint32_t>(), K, lv, kb[0], vb[0], s));
   } else if (rows.dtype == DANCE_U8 && rows.rs.nch <= 8) {
     hipLaunchKernelGGL(k_cells_q<true>, dim3((N + 255) / 256), dim3(256), 0, s, rows.rs.rows, rows.rs.stride16,
                        rows.rs.nch, N, dpiv.as<uint32_t>(), K, lv, kb[0], vb[0]);
@@ -796,7 +794,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     const QBoundSet qp_it = ((q_prune_iters >> it) & 1u) ? qb : QBoundSet{nullptr, 0.0f, 0.0f};
     DCHECK(launch_prune(rows, g, md, alpha, order, ctr, qp_it, ((p_rank >> it) & 1u) != 0u, s));
     DCHECK(record(iev[it].p1, s));
-    if (it == 0 && qb.rows && qbound_prune_adaptive() && !((q_prune_iters >> 1) & 1u) && iters > 1) {
+    if (it == 0 && qb.rows && iters > 1 && (qbound_prune_adaptive() || qbound_iters_adaptive())) {
       // pair density of iteration 0's prune (its bound checks), read once
       hipLaunchKernelGGL(k_ctr_sum, dim3(1), dim3(64), 0, s, static_cast<const VCounters*>(ctr),
                          csum.as<VCounters>());
@@ -1238,7 +1236,7 @@ static size_t resident_build_bytes(const void* d_data, int dtype, int store, uin
   add(kMedoidCandidates * 4);       // scores
   add(kMedoidCandidates * 4);       // cands
   add((size_t)N * kQChunks * 16);   // code rows of the bound
-  add((size_t)std::min(locality_cells(store), N) * 4);  // pivots
+  add((size_t)locality_cells(store, N) * 4);  // pivots
   add((size_t)N * 4);               // order
   for (size_t n : {(size_t)N, sort_items}) {  // the schedule's sort, then the reverse sort
     const size_t tiles = (n + kRadixTile - 1) / kRadixTile;
