@@ -180,24 +180,34 @@ static int launch_init(const Rows& rows, GraphBufs g, hipStream_t s) {
 // the build uses it in the iterations whose bit is set in DANCE_QBOUND_ITERS
 // (default kQBoundIters). Results are identical either way.
 constexpr uint32_t kQBoundIters = 0x1u;  // first iteration: random graph, HBM-bound
-// Without DANCE_QBOUND_ITERS the search also uses it in the last iteration
-// when the iteration before it computed more than kQBoundLastMinDist
-// candidate distances per expansion: the last iteration (alpha > 1) then
-// gathers more rows than the bound's extra work costs. Measured with both
-// variants of the last search launch (4 iterations): c1 (isotropic, 49.5
-// distances per expansion in iteration 2) 23.6 -> 14.7 ms with the bound; c3
-// (26.7) 935 -> 875 ms; c2 (20.1) 54.2 -> 69.3 ms and c2 with fp16 rows
-// (20.1) 70.3 -> 85.7 ms, so it stays off there.
+// Without DANCE_QBOUND_ITERS the search also uses it where the rows it spares
+// cost more than its own work, which depends on where they come from.
+// Dense data (kDenseFrac: isotropic rows, without clusters, reach 39-42% of
+// the candidate pairs in iteration 0's prune, clustered ones 7-11%) has no
+// locality for the schedule to use, so every gathered row misses L2 once the
+// rows outgrow it: every iteration then takes the bound, above kDenseMinBytes
+// of rows. Searches of iterations 1 / 2 / 3 without and with it: 20k x 96 fp32
+// 1.73 / 1.76 / 2.26 and 1.54 / 1.38 / 1.92 ms, 100k 17.1 / 18.4 / 23.6 and 11.3
+// / 10.5 / 14.7, 1M 202 / 226 / 294 and 128 / 130 / 181, 300k x 100 fp16 37.9 /
+// 42.1 / 54.4 and 28.2 / 28.8 / 38.6.
+// Clustered rows come mostly from L2, and the bound costs 15-30% (1M 36.2 /
+// 39.5 / 51.8 and 47.8 / 52.0 / 64.9 ms) until the rows are far beyond the
+// Infinity Cache: the last iteration at 4M 245 without and 294 ms with it,
+// at 6M (2.3 GB) 426 and 461, at 10M (3.8 GB) 914 and 810; so there it is
+// taken in the last iteration from kClusteredMinBytes on.
+// Either way the last iteration takes it only when the iteration before it
+// computed more than kQBoundLastMinDist candidate distances per expansion.
+constexpr double kDenseFrac = 0.25;
+constexpr double kDenseMinBytes = 4.0 * (1 << 20);  // one XCD's L2
+constexpr double kClusteredMinBytes = 3e9;
 constexpr double kQBoundLastMinDist = 24.0;
 static bool qbound_iters_adaptive() {
   const char* e = std::getenv("DANCE_QBOUND_ITERS");
   return !(e && e[0]);
 }
 // The prune uses it in the iterations of DANCE_QBOUND_PRUNE_ITERS (default
-// kQBoundPruneIters), and by default also in iteration 1 when iteration 0's
-// prune reached more than a quarter of all candidate pairs (its bound checks
-// per vertex above C (C - 1) / 8): the bound's one batch then replaces dense
-// exact rounds. Measured: iteration 1's prune at c1 (isotropic data, 41% of
+// kQBoundPruneIters), and by default also in iteration 1 of dense data
+// (kDenseFrac): the bound's one batch then replaces dense exact rounds. Measured: iteration 1's prune at c1 (isotropic data, 41% of
 // the pairs reached in iteration 0) 7.07 -> 1.05 ms with the bound; at c2 and
 // c3 (clustered, 7.6%) 4.46 -> 5.54 and 47.4 -> 57.2 ms, so it stays off there.
 constexpr uint32_t kQBoundPruneIters = ~0x2u;  // every iteration but 1 (0, 2 and 3 of the default 4)
@@ -751,7 +761,9 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   DCHECK(build_qbound(rows, qbuf, s, &qb));
   const uint32_t* order = nullptr;
   DCHECK(build_schedule(rows, qb, rws, s, &order));
-  uint32_t q_iters = qbound_iters();  // the last iteration's bit may be set after the one before it
+  uint32_t q_iters = qbound_iters();  // later iterations' bits may be set on the way (kDenseFrac)
+  bool dense = false;
+  const double row_bytes = (double)rows.rs.stride16 * 16.0 * (double)N;
   const uint32_t ib_iters = insert_bound_iters();
   uint32_t q_prune_iters = qbound_prune_iters();  // iteration 1's bit may be set after iteration 0
   const uint32_t iters = vamana_iters();
@@ -802,8 +814,11 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
       VCounters h{};
       DHIP(hipMemcpyAsync(&h, csum.p, sizeof(VCounters), hipMemcpyDeviceToHost, s));
       DHIP(hipStreamSynchronize(s));
-      const double pairs = (double)g.C * (double)(g.C > 0 ? g.C - 1 : 0) / 8.0;
-      if ((double)h.prune_bound_checks > pairs * (double)g.N) q_prune_iters |= 2u;
+      const double pairs = (double)g.C * (double)(g.C > 0 ? g.C - 1 : 0) / 2.0;
+      dense = (double)h.prune_bound_checks > kDenseFrac * pairs * (double)g.N;
+      if (dense && qbound_prune_adaptive()) q_prune_iters |= 2u;
+      if (dense && qbound_iters_adaptive() && row_bytes > kDenseMinBytes)
+        q_iters |= ((1u << (iters - 1)) - 1u) & ~1u;  // the iterations between the first and the last
     }
     if (qb.rows && qbound_iters_adaptive() && iters > 1 && it + 3 >= iters && it + 1 < iters) {
       // candidate distances per expansion of the iteration before the last:
@@ -820,7 +835,8 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
         const double cand = (double)(h.search_dist + h.bound_skips) -
                             (double)(before_last.search_dist + before_last.bound_skips);
         const double exps = (double)(h.expansions - before_last.expansions);
-        if (cand > kQBoundLastMinDist * exps) q_iters |= 1u << (iters - 1);
+        if (cand > kQBoundLastMinDist * exps && (dense || row_bytes >= kClusteredMinBytes))
+          q_iters |= 1u << (iters - 1);
       }
     }
     if (timed) {  // cumulative counters after this iteration

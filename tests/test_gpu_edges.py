@@ -36,3 +36,29 @@ def test_medoid_group_edges(kind, dim, n):
     same = gs.view(np.uint32) == os_.view(np.uint32)
     assert np.all(same | (np.isnan(gs) & np.isnan(os_)))
     assert gm == om
+
+
+# u8 rows of 1, 2, 4 and 8 chunks per lane take the schedule's MFMA cells; 4095
+# and 4096 rows are the two sides of the rule that needs 16 cells of 256 rows
+@pytest.mark.parametrize("n,dim", [(4095, 40), (4096, 40), (4097, 129), (5000, 300), (4500, 600)])
+def test_u8_schedule_widths(n, dim):
+    x = rows("u8", n, dim)
+    og, od, om = O.vnew2_build(x, 24, 48, 32, 24)
+    r = D.vamana_build(x, 24, 48, 32, 24)
+    assert r.medoid == om
+    assert np.array_equal(r.degree, od) and np.array_equal(r.graph, og)
+
+
+# rows without clusters: from 4 MiB of (padded) rows on every iteration takes the
+# code-row bound; the same rows below it, and clustered rows, keep 1 and 2 exact
+@pytest.mark.parametrize("n,centers,middle", [(11_000, 0, True), (10_900, 0, False), (11_000, 40, False)])
+def test_bound_in_every_iteration_of_dense_data(n, centers, middle):
+    x = rows("f32", n, 96, centers=centers)
+    assert (n * 384 > 4 << 20) == (n == 11_000)
+    og, od, om = O.vnew2_build(x, 48, 64, 64, 32)
+    r = D.vamana_build(x, 48, 64, 64, 32)
+    assert r.medoid == om
+    assert np.array_equal(r.degree, od) and np.array_equal(r.graph, og)
+    checks = r.kernel_profile["bound_checks_iter"]
+    assert checks[0] > 0
+    assert [c > 0 for c in checks[1:3]] == [middle, middle]
