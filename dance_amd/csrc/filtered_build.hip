@@ -288,9 +288,9 @@ int locality_order(const Rows& rows, const Labels& Ld, uint32_t N, uint32_t T, F
   if (rows.dtype == DANCE_U8) {
     DCHECK(launch_cells_u8(rows, N, piv.as<const uint32_t>(), K, lv, kb[0], vb[0], s));
   } else {
-    DCHECK(with_cpl(pick_cpl(rows.rs.nch), [&](auto c) {  // float rows are searched as fp16
-      hipLaunchKernelGGL((k_cells<DANCE_F16, decltype(c)::value>), dim3(cells_grid(N)), dim3(kCellsBlock), 0, s,
-                         rows.rs, N, piv.as<const uint32_t>(), K, lv, kb[0], vb[0]);
+    DCHECK(with_dt_cpl(rows.kind(), pick_cpl(rows.rs.nch), [&](auto dt, auto c) {
+      hipLaunchKernelGGL((k_cells<decltype(dt)::value, decltype(c)::value>), dim3(cells_grid(N)), dim3(kCellsBlock),
+                         0, s, rows.rs, N, piv.as<const uint32_t>(), K, lv, kb[0], vb[0]);
       DHIP(hipGetLastError());
       return 0;
     }));
@@ -466,7 +466,7 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
     }
     hipEvent_t r0 = E.mark(s);
     if (T > 0) {
-      DCHECK(with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+      DCHECK(with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
         hipLaunchKernelGGL((k_task_search<decltype(dt)::value, decltype(c)::value>), grid_xcd(T),
                            dim3(kBlock), search_lds, s, rows.rs, Ga, Ld, st.task_rows.as<const uint32_t>(), torder,
                            T, per_label_pool, per_label_keep, p.STEPS, st.tids.as<uint32_t>(), st.td.as<float>(),
@@ -478,7 +478,7 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
     hipEvent_t r1 = E.mark(s);
     RowArgs A{ordinary_pool, ordinary_keep, p.STEPS, p.global_start, work_C, per_label_keep, p.alpha,
               st.tids.as<const uint32_t>(), st.td.as<const float>(), gb, db, ctr, rorder};
-    DCHECK(with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+    DCHECK(with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
       hipLaunchKernelGGL((k_row<decltype(dt)::value, decltype(c)::value>), grid_xcd(N), dim3(kBlock),
                          search_lds, s, rows.rs, Ga, Ld, A);
       DHIP(hipGetLastError());
@@ -517,7 +517,7 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
     const Graph Gb{N, R, gb, db};
     CsrArgs Cs{p.alpha, roff, st.rids.as<const uint32_t>(), boff, st.bd.as<float>(), st.brem.as<uint8_t>(),
                st.bmask.as<uint32_t>(), ga, da, ctr, win};
-    DCHECK(with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+    DCHECK(with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
       // The three kernels write disjoint rows and run side by side: long
       // rows beyond the key window (the first tails[3] of the longest-first
       // list; workgroups of kLongWaves waves), the other long rows
@@ -583,7 +583,7 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
     const size_t pub_lds = (size_t)kWaves * kPubLds * 4;
     hipEvent_t p0 = E.mark(s);
     PubArgs P{p.alpha, PR, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, gb, db, ctr};
-    DCHECK(with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+    DCHECK(with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
       hipLaunchKernelGGL((k_publish<decltype(dt)::value, decltype(c)::value, false>), grid_xcd(N),
                          dim3(kBlock), pub_lds, s, rows.rs, Graph{N, R, ga, da}, Ld, P);
       DHIP(hipGetLastError());
@@ -608,7 +608,7 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
     DCHECK(ensure_big(st, tails[1]));
     P = PubArgs{p.alpha, PR, roff, st.rids.as<const uint32_t>(), boff, st.bmask.as<uint32_t>(), st.bd.as<float>(),
                 st.brem.as<uint8_t>(), gb, db, ctr};
-    DCHECK(with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+    DCHECK(with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
       hipLaunchKernelGGL((k_publish<decltype(dt)::value, decltype(c)::value, true>), grid_xcd(N),
                          dim3(kBlock), pub_lds, s, rows.rs, Graph{N, PR, gb, db}, Ld, P);
       DHIP(hipGetLastError());

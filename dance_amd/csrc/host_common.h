@@ -86,13 +86,14 @@ inline int with_cpl(int cpl, Fn&& fn) {
 }
 
 template <typename Fn>
-inline int with_dt_cpl(int dtype, int cpl, Fn&& fn) {
-  switch (dtype) {
+inline int with_dt_cpl(int kind, int cpl, Fn&& fn) {
+  switch (kind) {
     case DANCE_F32: return with_cpl(cpl, [&](auto c) { return fn(IC<DANCE_F32>{}, c); });
     case DANCE_U8: return with_cpl(cpl, [&](auto c) { return fn(IC<DANCE_U8>{}, c); });
     case DANCE_F16: return with_cpl(cpl, [&](auto c) { return fn(IC<DANCE_F16>{}, c); });
+    case kF16Odd: return with_cpl(cpl, [&](auto c) { return fn(IC<kF16Odd>{}, c); });
   }
-  std::fprintf(stderr, "[dance_hip] unsupported dtype %d\n", dtype);
+  std::fprintf(stderr, "[dance_hip] unsupported dtype %d\n", kind);
   return -1;
 }
 
@@ -255,6 +256,7 @@ struct Rows {
   int dtype = DANCE_F32;
   uint32_t N = 0, dim = 0;
   uint32_t vbytes() const { return dim * elem_bytes(dtype); }
+  int kind() const { return dtype == DANCE_F16 && rs.tail16 >= 0 ? kF16Odd : dtype; }  // see kF16Odd
 };
 
 static __global__ void k_f32_to_f16_rows(const float* __restrict__ src, uint32_t N, uint32_t dim,

@@ -263,7 +263,7 @@ __device__ __forceinline__ float q_ub_root(const QBoundSet& qb, float T0, float 
 template <int DT>
 __device__ __forceinline__ float q_ub_root_of(const QBoundSet& qb, float T0, float alpha) {
   const float r = q_ub_root(qb, T0, alpha);
-  return DT == DANCE_F16 ? fminf(r, 254.0f) : r;
+  return is_f16(DT) ? fminf(r, 254.0f) : r;
 }
 // The querying side of the upper test (see above): row header s, r, hi and
 // the root that ||x - y|| must not pass (negative: nothing is proved).

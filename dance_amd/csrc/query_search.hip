@@ -135,7 +135,7 @@ int run_search(const SearchIn& in) {
   const uint32_t grid = (in.nq + kWaves - 1) / kWaves;
   const size_t lds = (size_t)kWaves * kLds * 4;
   const int ps = pick_ps(in.L);
-  DCHECK(with_dt_cpl(base.dtype, cpl, [&](auto dt, auto c) {
+  DCHECK(with_dt_cpl(base.kind(), cpl, [&](auto dt, auto c) {
     constexpr int DT = decltype(dt)::value, CPL = decltype(c)::value;
     if (ps == 1)
       hipLaunchKernelGGL((k_query<DT, CPL, 1>), dim3(grid), dim3(kBlock), lds, s, base.rs, qr.rs, a);

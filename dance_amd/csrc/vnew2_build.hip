@@ -156,7 +156,7 @@ static dim3 xcd_grid(uint32_t n) { return grid_dims(wave_grid(n), kBlock, 8); }
 static int launch_medoid(const Rows& rows, hipStream_t s, float* d_scores, uint32_t* d_cands, uint32_t nc,
                          uint32_t ns) {
   const int cpl = pick_cpl(rows.rs.nch);
-  return with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+  return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int CPL = decltype(c)::value;
     constexpr uint32_t KC = medoid_cands(CPL);
     hipLaunchKernelGGL((k_medoid<decltype(dt)::value, CPL>), dim3((nc + KC - 1) / KC), dim3(64 * medoid_waves(CPL)),
@@ -168,7 +168,7 @@ static int launch_medoid(const Rows& rows, hipStream_t s, float* d_scores, uint3
 
 static int launch_init(const Rows& rows, GraphBufs g, hipStream_t s) {
   const int cpl = pick_cpl(rows.rs.nch);
-  return with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+  return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     hipLaunchKernelGGL((k_init<decltype(dt)::value, decltype(c)::value>), grid_dims(wave_grid(g.N), kBlock), dim3(kBlock), 0, s,
                        rows.rs, g);
     DHIP(hipGetLastError());
@@ -278,14 +278,14 @@ static int launch_search(const Rows& rows, GraphBufs g, uint32_t L, uint32_t ste
     std::fprintf(stderr, "[dance_hip] L=%u exceeds the supported maximum %u\n", L, kMaxBuildL);
     return -1;
   }
-  return with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+  return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int DT = decltype(dt)::value, CPL = decltype(c)::value;
     // Bounded variants exist only where build_qbound can produce code rows.
     constexpr bool kHasQB = DT != DANCE_U8 && CPL <= 4;
     if constexpr (kHasQB) {
       if (qb.rows && L <= 256) {
         // (fp16 rows of at most 112 dims take 2 chunks per lane)
-        if constexpr (CPL <= (DT == DANCE_F16 ? 2 : 3)) {
+        if constexpr (CPL <= (is_f16(DT) ? 2 : 3)) {
           if (insert_bound && L <= 128 && g.C <= 128) {  // nA <= C <= 128 fits the open-pair list
             if (hashed_cur)
               hipLaunchKernelGGL((k_search<DT, CPL, 2, true, true, true>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp);
@@ -348,7 +348,7 @@ static int launch_prune(const Rows& rows, GraphBufs g, uint32_t min_degree, floa
   const uint32_t Cp = round64(g.C), Rp = round64(g.R), Cq = (g.C + 31u) / 32u * 32u;
   PruneArgs a{rows.rs, g, min_degree, alpha, order, ctr, qb};
   const bool rank = Cp <= kRankCap && rank_kernel;
-  return with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+  return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int DT = decltype(dt)::value, CPL = decltype(c)::value;
     constexpr bool kHasQB = DT != DANCE_U8 && CPL <= 4;
     if (rank) {
@@ -510,26 +510,21 @@ static int build_reverse_csr(GraphBufs g, ReverseWs& ws, hipStream_t s, RevCsr* 
   return 0;
 }
 
-static int launch_merge(const Rows& rows, GraphBufs g, const RevCsr& rev, const Profile& prof, const uint32_t* order,
+static int launch_merge(GraphBufs g, const RevCsr& rev, const Profile& prof, const uint32_t* order,
                         VCounters* ctr, hipStream_t s) {
-  const int cpl = pick_cpl(rows.rs.nch);
   const uint32_t Cp = round64(g.C);
-  MergeArgs a{rows.rs, g, rev.offs, rev.srcs, rev.snap, prof.heavy_threshold, prof.heavy_sample, order, ctr,
-              rev.offs64};
-  return with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
-    constexpr int DT = decltype(dt)::value, CPL = decltype(c)::value;
-    if (g.C <= 64)
-      hipLaunchKernelGGL((k_merge_reg<DT, CPL, 1>), xcd_grid(g.N), dim3(kBlock), 0, s, a);
-    else if (g.C <= 128)
-      hipLaunchKernelGGL((k_merge_reg<DT, CPL, 2>), xcd_grid(g.N), dim3(kBlock), 0, s, a);
-    else if (g.C <= 256)
-      hipLaunchKernelGGL((k_merge_reg<DT, CPL, 4>), xcd_grid(g.N), dim3(kBlock), 0, s, a);
-    else
-      hipLaunchKernelGGL((k_merge<DT, CPL>), xcd_grid(g.N), dim3(kBlock),
-                         (size_t)kWavesPerBlock * merge_lds_words(Cp) * 4, s, a, Cp);
-    DHIP(hipGetLastError());
-    return 0;
-  });
+  MergeArgs a{g, rev.offs, rev.srcs, rev.snap, prof.heavy_threshold, prof.heavy_sample, order, ctr, rev.offs64};
+  if (g.C <= 64)
+    hipLaunchKernelGGL(k_merge_reg<1>, xcd_grid(g.N), dim3(kBlock), 0, s, a);
+  else if (g.C <= 128)
+    hipLaunchKernelGGL(k_merge_reg<2>, xcd_grid(g.N), dim3(kBlock), 0, s, a);
+  else if (g.C <= 256)
+    hipLaunchKernelGGL(k_merge_reg<4>, xcd_grid(g.N), dim3(kBlock), 0, s, a);
+  else
+    hipLaunchKernelGGL(k_merge, xcd_grid(g.N), dim3(kBlock), (size_t)kWavesPerBlock * merge_lds_words(Cp) * 4, s, a,
+                       Cp);
+  DHIP(hipGetLastError());
+  return 0;
 }
 
 // Iteration count (VAMANA_ITERS, gpu_vamana_config.h:78-79, a compile-time
@@ -608,7 +603,7 @@ static int build_schedule(const Rows& rows, const QBoundSet& qb, ReverseWs& ws, 
                        rows.rs.nch, N, dpiv.as<uint32_t>(), K, lv, kb[0], vb[0]);
     DHIP(hipGetLastError());
   } else {
-    DCHECK(with_dt_cpl(rows.dtype, cpl, [&](auto dt, auto c) {
+    DCHECK(with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
       hipLaunchKernelGGL((k_cells<decltype(dt)::value, decltype(c)::value>), dim3(cells_grid(N)),
                          dim3(kCellsBlock), 0, s, rows.rs, N, dpiv.as<uint32_t>(), K, lv, kb[0], vb[0]);
       DHIP(hipGetLastError());
@@ -800,7 +795,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     RevCsr rev{};
     DCHECK(build_reverse_csr(g, rws, s, &rev));
     DCHECK(record(iev[it].r1, s));
-    DCHECK(launch_merge(rows, g, rev, prof, order, ctr, s));
+    DCHECK(launch_merge(g, rev, prof, order, ctr, s));
     DCHECK(record(iev[it].m1, s));
     const uint32_t md = (it + 1 == iters) ? kFinalMinDegree : 0u;
     const QBoundSet qp_it = ((q_prune_iters >> it) & 1u) ? qb : QBoundSet{nullptr, 0.0f, 0.0f};
@@ -1774,7 +1769,7 @@ int dance_stage_distances(const void* h_data, int dtype, uint32_t N, uint32_t di
   DCHECK(up(db.p, b, n * 4, cx.s));
   const int cpl = pick_cpl(cx.rows.rs.nch);
   const uint64_t waves = (n + 63) / 64;
-  DCHECK(with_dt_cpl(dtype, cpl, [&](auto dt, auto c) {
+  DCHECK(with_dt_cpl(cx.rows.kind(), cpl, [&](auto dt, auto c) {
     if (waves == 0) return 0;
     hipLaunchKernelGGL((k_pair_dist<decltype(dt)::value, decltype(c)::value>),
                        dim3((uint32_t)((waves + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kBlock), 0, cx.s,
@@ -1948,7 +1943,8 @@ int dance_stage_reverse_merge(const void* h_data, int dtype, uint32_t N, uint32_
       for (uint32_t e = 0; e < off[N]; ++e) ids[e] /= R;  // forward slot -> source
   }
   Profile prof{"stage", false, heavy_threshold, heavy_sample};
-  DCHECK(launch_merge(cx.rows, g, rev, prof, nullptr, nullptr, cx.s));
+  DCHECK(with_dt_cpl(cx.rows.kind(), pick_cpl(cx.rows.rs.nch), [](auto, auto) { return 0; }));  // types and widths
+  DCHECK(launch_merge(g, rev, prof, nullptr, nullptr, cx.s));
   return download_state(cx.st, nullptr, nullptr, work, deg_work, wd, cx.s);
 }
 

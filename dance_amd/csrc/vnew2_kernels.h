@@ -1004,8 +1004,9 @@ struct SearchWave {
 // insert-bound variants ask for DANCE_SEARCH_WAVES_IB (default 6: 80 registers
 // at 3 chunks per lane; three row addresses live in scratch. 5 waves: first
 // search at 1M x 96 113 -> 108 ms, at 4M 457 -> 464 ms). At 129 <= L <= 256 two
-// chunks per lane fit 6 waves without the bound and 5 with it. No constraint
-// elsewhere.
+// chunks per lane fit 6 waves without the bound and 5 with it. Without the bound
+// 4 chunks per lane fit 6 waves and 8 chunks 4 (fp16 rows of 4 chunks took 198
+// registers, 2 waves, with no floor). No constraint elsewhere.
 #ifndef DANCE_SEARCH_WAVES
 #define DANCE_SEARCH_WAVES 6
 #endif
@@ -1019,7 +1020,7 @@ template <int CPL, int PS, bool QB, bool IB, bool HC>
 constexpr int kSearchMinWaves =
     (CPL <= 3 && PS == 2)
         ? (IB ? DANCE_SEARCH_WAVES_IB : QB ? DANCE_SEARCH_WAVES_QB : (CPL <= 2 && HC) ? 8 : DANCE_SEARCH_WAVES)
-        : (CPL <= 2 && PS == 4) ? (QB ? 5 : 6) : 1;
+        : (CPL <= 2 && PS == 4) ? (QB ? 5 : 6) : (PS == 2 && !QB && CPL <= 8) ? (CPL == 4 ? 6 : 4) : 1;
 
 // search_prune_kernel_shared (vnew2.cu:1119-1439).
 template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false>
@@ -1307,10 +1308,10 @@ __device__ __forceinline__ uint32_t ffs128(uint64_t m0, uint64_t m1) {
 // Occupancy floor: the bound's variant holds every code fragment of up to 96
 // ranks (48 registers) next to its MFMA accumulators, which fits 5 waves per
 // SIMD; the variant without it fits 6 at rows of up to 4 chunks per lane.
-// Wider rows (and fp16 rows of 4 chunks per lane, whose tail selects take a
-// few more registers) get no floor, so no variant spills.
+// Wider rows (and fp16 rows of 4 chunks per lane) get no floor, so no variant
+// spills.
 template <int DT, int CPL, int PM>
-constexpr int kRankMinWaves = PM != kRankExact ? 5 : (CPL < 4 || (CPL == 4 && DT != DANCE_F16)) ? 6 : 1;
+constexpr int kRankMinWaves = PM != kRankExact ? 5 : (CPL < 4 || (CPL == 4 && !is_f16(DT))) ? 6 : 1;
 template <int DT, int CPL, int PM>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMinWaves<DT, CPL, PM>, 8))) void k_prune_rank(PruneArgs a, uint32_t Cq) {
   constexpr bool QB = PM == kRankBound, XG = PM == kRankGram;
@@ -1901,7 +1902,6 @@ static __global__ void k_seg_offsets(const uint32_t* __restrict__ keys, size_t n
 }
 
 struct MergeArgs {
-  RowSet rs;
   GraphBufs g;
   const uint32_t* offsets;  // N+1
   const uint32_t* srcs;     // sorted forward slots s*R + i
@@ -1936,8 +1936,7 @@ struct MergeArgs {
 
 __host__ __device__ constexpr uint32_t merge_lds_words(uint32_t Cp) { return 2u * Cp + 128u; }
 
-template <int DT, int CPL>
-__global__ __launch_bounds__(kBlock) void k_merge(MergeArgs a, uint32_t Cp) {
+static __global__ __launch_bounds__(kBlock) void k_merge(MergeArgs a, uint32_t Cp) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t gw = xcd_block(grid_block(), grid_blocks()) * kWavesPerBlock + w;
@@ -2111,7 +2110,7 @@ struct MergeRow {
   }
 };
 
-template <int DT, int CPL, int MS>
+template <int MS>
 __global__ __launch_bounds__(kBlock) void k_merge_reg(MergeArgs a) {
   const uint32_t w = wave_index();
   const uint32_t gw = xcd_block(grid_block(), grid_blocks()) * kWavesPerBlock + w;
