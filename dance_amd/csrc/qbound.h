@@ -1,9 +1,10 @@
 // Quantized lower bound on the canonical distance, used to skip exact
 // distance gathers whose result cannot change the search state.
 //
-// Each vector row x gets a 128-byte companion row (one cache line):
-//   chunk 0      header {float s, float r, float lo, float hi}
-//   chunks 1..7  int8 codes q (16 dimensions per chunk, zero padded)
+// Each vector row x gets a companion row of QC chunk groups (128 bytes, a cache
+// line, each; QC = 1 up to 112 dimensions, 2 up to 240):
+//   chunk 0                header {float s, float r, float lo, float hi}
+//   chunks 1..(8 QC - 1)   int8 codes q (16 dimensions per chunk, zero padded)
 // with x ~ s*q, a = s^2 * sum(q^2), r >= ||x - s*q||_2 (rounded up),
 // lo <= a (1 - k) - r^2 (1 + k) (rounded down) and hi >= a (1 + k) -
 // r^2 (1 - k) (rounded up), k = kQSlack = 2^-18. For a pair (x, y) with code
@@ -43,12 +44,22 @@
 
 namespace dance {
 
-constexpr uint32_t kQChunks = 8;                      // 16-byte chunks per code row
-constexpr uint32_t kQMaxDim = (kQChunks - 1u) * 16u;  // dimensions a code row holds
+constexpr uint32_t kQChunks = 8;  // 16-byte chunks per chunk group
+constexpr uint32_t q_chunks(int qc) { return kQChunks * (uint32_t)qc; }  // per code row
+constexpr uint32_t q_max_dim(int qc) { return (q_chunks(qc) - 1u) * 16u; }  // dimensions it holds
+constexpr uint32_t kQMaxDim = q_max_dim(1);
+// Whether rows of this kind and width (chunks per lane) can have code rows of
+// QC groups: the widths that hold 1..112 (QC = 1) or 113..240 dimensions.
+constexpr bool q_width(int dt, int cpl, int qc) {
+  if (dt == DANCE_U8) return false;
+  if (is_f16(dt)) return qc == 1 ? cpl <= 2 : cpl >= 2 && cpl <= 4;
+  return qc == 1 ? cpl <= 4 : cpl == 4 || cpl == 8;
+}
 constexpr float kQSlack = 0x1p-18f;
 
 struct QBoundSet {
-  const uint4* rows;  // N x kQChunks chunks; nullptr disables the bound
+  const uint4* rows;  // N code rows; nullptr disables the bound
+  int groups;         // chunk groups per code row (QC)
   float kappa2;       // relative rounding slack of the row type and width
   float eta;          // absolute slack (underflow; binary16 subnormals)
 };
@@ -64,18 +75,19 @@ __device__ __forceinline__ float next_toward(float x, bool up) {
 // sub+16, sub+24 (word w = dimensions 4w..4w+3), so every load and store of
 // an octet covers contiguous bytes. Computes codes, scale and radius from the
 // first `dim` elements of the row.
-template <int DT>
+template <int DT, int QC>
 __global__ __launch_bounds__(256) void k_quantize(RowSet rs, uint32_t N, uint32_t dim, uint4* __restrict__ out) {
-  constexpr uint32_t kWords = (kQChunks - 1) * 4;  // 28 code words
+  constexpr uint32_t kWords = (q_chunks(QC) - 1) * 4;  // code words
+  constexpr uint32_t kPer = 4 * QC;                    // of each lane
   constexpr uint32_t kEB = DT == DANCE_F32 ? 4u : 2u;  // element bytes
   const uint32_t lane = threadIdx.x & 63u, sub = lane & 7u;
   const uint32_t row = (blockIdx.x * 256u + threadIdx.x) >> 3;
   const bool act = row < N;
   const uint8_t* rb = reinterpret_cast<const uint8_t*>(rs.rows + (size_t)(act ? row : 0u) * rs.stride16);
   const uint32_t row_bytes = rs.stride16 * 16u;
-  float v[4][4];
+  float v[kPer][4];
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) {
+  for (uint32_t k = 0; k < kPer; ++k) {
     const uint32_t w = sub + 8u * k;
     const bool in = act && w < kWords && 4u * w < dim && (4u * w + 4u) * kEB <= row_bytes;
     if constexpr (DT == DANCE_F32) {
@@ -98,7 +110,7 @@ __global__ __launch_bounds__(256) void k_quantize(RowSet rs, uint32_t N, uint32_
   float mx = 0.0f;
   int fin = 1;
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k)
+  for (uint32_t k = 0; k < kPer; ++k)
 #pragma unroll
     for (uint32_t e = 0; e < 4; ++e) {
       fin &= __builtin_isfinite(v[k][e]) ? 1 : 0;
@@ -117,9 +129,9 @@ __global__ __launch_bounds__(256) void k_quantize(RowSet rs, uint32_t N, uint32_
   if (!usable || mx == 0.0f) s = 0.0f;
   int A = 0;
   double err = 0.0;
-  uint32_t words[4];
+  uint32_t words[kPer];
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) {
+  for (uint32_t k = 0; k < kPer; ++k) {
     uint32_t word = 0u;
 #pragma unroll
     for (uint32_t e = 0; e < 4; ++e) {
@@ -139,9 +151,9 @@ __global__ __launch_bounds__(256) void k_quantize(RowSet rs, uint32_t N, uint32_
   err += __shfl_xor(err, 2);
   err += __shfl_xor(err, 4);
   if (!act) return;
-  uint32_t* o = reinterpret_cast<uint32_t*>(out + (size_t)row * kQChunks);
+  uint32_t* o = reinterpret_cast<uint32_t*>(out + (size_t)row * q_chunks(QC));
 #pragma unroll
-  for (uint32_t k = 0; k < 4; ++k) {
+  for (uint32_t k = 0; k < kPer; ++k) {
     const uint32_t w = sub + 8u * k;
     if (w < kWords) o[4u + w] = words[k];
   }
@@ -170,8 +182,9 @@ struct QSelf {
   float s, r, lo;
 };
 
+template <int QC>
 __device__ __forceinline__ void q_load_self(const QBoundSet& qb, uint32_t id, QSelf& me) {
-  const uint4* p = qb.rows + (size_t)id * kQChunks;
+  const uint4* p = qb.rows + (size_t)id * q_chunks(QC);
   me.row = p;
   const uint4 h = p[0];  // same address in every lane: kept as scalars
   me.s = __uint_as_float(uni_u(h.x));
@@ -185,19 +198,31 @@ __device__ __forceinline__ float q_threshold(const QBoundSet& qb, float r, float
   return (__builtin_sqrtf(t) + r) * (1.0f + kQSlack);
 }
 
-// Chunk `sub` of the code row of candidate `id`. An inactive lane loads
+// Chunks sub, sub + 8, ... of a code row.
+template <int QC>
+struct QCodes {
+  uint4 c[QC];
+};
+
+// The lane's chunks of the code row of candidate `id`. An inactive lane loads
 // nothing and the value is left unset (as in load_row): `active` is the same
 // on the 8 lanes of an octet, and callers discard the answers of inactive
 // octets.
-__device__ __forceinline__ uint4 q_load(const QBoundSet& qb, uint32_t id, bool active, uint32_t sub) {
-  uint4 b;
-  if (active) b = qb.rows[(size_t)id * kQChunks + sub];
+template <int QC>
+__device__ __forceinline__ QCodes<QC> q_load(const QBoundSet& qb, uint32_t id, bool active, uint32_t sub) {
+  QCodes<QC> b;
+  const uint4* p = qb.rows + (size_t)id * q_chunks(QC);
+#pragma unroll
+  for (int c = 0; c < QC; ++c)
+    if (active) b.c[c] = p[sub + 8u * (uint32_t)c];
   return b;
 }
-// Chunk `sub` of the querying row's codes, its header replaced by zeros, so
-// that a candidate's header adds nothing to the dot.
-__device__ __forceinline__ uint4 q_codes(const uint4& chunk, uint32_t sub) {
-  return sub == 0u ? make_uint4(0u, 0u, 0u, 0u) : chunk;
+// The querying row's chunks, its header replaced by zeros, so that a
+// candidate's header adds nothing to the dot.
+template <int QC>
+__device__ __forceinline__ QCodes<QC> q_codes(QCodes<QC> row, uint32_t sub) {
+  if (sub == 0u) row.c[0] = make_uint4(0u, 0u, 0u, 0u);
+  return row;
 }
 
 // The querying side of the lower test (see above): row header s, r, lo and S.
@@ -215,28 +240,33 @@ __device__ __forceinline__ bool q_lower_proves(const QLower& me, float s, float 
   return __builtin_fmaf(me.m2s * s, (float)c, __builtin_fmaf(me.n2S, r, lo)) >= me.K;
 }
 
-// Exact integer code dot of a querying row (q_codes) and a row whose chunk
-// `sub` every lane of an octet holds; every lane of the octet receives it.
-// Must be called by all 64 lanes.
-__device__ __forceinline__ int q_octet_dot(const uint4& code, const uint4& b) {
+// Exact integer code dot of a querying row (q_codes) and a row whose chunks an
+// octet holds (q_load); every lane of the octet receives it. Must be called by
+// all 64 lanes.
+template <int QC>
+__device__ __forceinline__ int q_octet_dot(const QCodes<QC>& code, const QCodes<QC>& b) {
   int c = 0;
-  c = __builtin_amdgcn_sdot4((int)code.x, (int)b.x, c, false);
-  c = __builtin_amdgcn_sdot4((int)code.y, (int)b.y, c, false);
-  c = __builtin_amdgcn_sdot4((int)code.z, (int)b.z, c, false);
-  c = __builtin_amdgcn_sdot4((int)code.w, (int)b.w, c, false);
+#pragma unroll
+  for (int k = 0; k < QC; ++k) {
+    c = __builtin_amdgcn_sdot4((int)code.c[k].x, (int)b.c[k].x, c, false);
+    c = __builtin_amdgcn_sdot4((int)code.c[k].y, (int)b.c[k].y, c, false);
+    c = __builtin_amdgcn_sdot4((int)code.c[k].z, (int)b.c[k].z, c, false);
+    c = __builtin_amdgcn_sdot4((int)code.c[k].w, (int)b.c[k].w, c, false);
+  }
   c += dpp<kDppHalfMirror>(0, c);
   c += dpp<kDppQuadXor2>(0, c);
   c += dpp<kDppQuadXor1>(0, c);
   return c;
 }
 
-// Octet test for a candidate: every lane of the octet holds one chunk `b` of
-// its code row (q_load); the lane with sub == 0 (which holds the header)
-// returns whether the bound proves dist >= T. `code` is chunk `sub` of the
-// querying row (q_codes). Must be called by all 64 lanes.
-__device__ __forceinline__ bool q_proves_reject(const QLower& me, const uint4& code, const uint4& b) {
-  const int c = q_octet_dot(code, b);
-  return q_lower_proves(me, __uint_as_float(b.x), __uint_as_float(b.y), __uint_as_float(b.z), c);
+// Octet test for a candidate: the lanes of the octet hold its code row `b`
+// (q_load); the lane with sub == 0 (which holds the header) returns whether the
+// bound proves dist >= T. `code` is the querying row (q_codes). Must be called
+// by all 64 lanes.
+template <int QC>
+__device__ __forceinline__ bool q_proves_reject(const QLower& me, const QCodes<QC>& code, const QCodes<QC>& b) {
+  const int c = q_octet_dot<QC>(code, b);
+  return q_lower_proves(me, __uint_as_float(b.c[0].x), __uint_as_float(b.c[0].y), __uint_as_float(b.c[0].z), c);
 }
 
 // The upper-bound side, for a pair test fl(alpha * dist) <= T0 (the online

@@ -12,8 +12,8 @@
 //   work   N x C   u32 + wd N x C f32   candidate rows with distances
 //   keys/vals 2 x 2 x N*R u32     reverse-edge radix sort double buffers
 //   offs   N+1 u32                reverse CSR offsets
-//   qrows  N x 128 B              int8 codes + header for the distance lower
-//                                 bound (fp32/fp16 rows of <= 112 dims)
+//   qrows  N x 128 or 256 B       int8 codes + header for the distance bounds
+//                                 (fp32/fp16 rows of <= 112 or <= 240 dims)
 // All kernels run on one stream; stages are timed with HIP events.
 //
 // Algorithmic bytes reported for the roofline (per kernel, summed over the
@@ -238,23 +238,29 @@ static uint32_t qbound_prune_iters() { return env_mask("DANCE_QBOUND_PRUNE_ITERS
 
 // Builds the code rows for `rows` into buf; returns a disabled set when the
 // row type or width has no bound.
-static int build_qbound(const Rows& rows, DevBuf& buf, hipStream_t s, QBoundSet* out) {
-  *out = QBoundSet{nullptr, 0.0f, 0.0f};
-  if (!qbound_enabled() || rows.dtype == DANCE_U8 || rows.dim > kQMaxDim || rows.N == 0) return 0;
+static int build_qbound(const Rows& rows, DevBuf& buf, hipStream_t s, QBoundSet* out, bool wide = true) {
+  *out = QBoundSet{};
+  if (!qbound_enabled() || rows.dtype == DANCE_U8 || rows.dim > q_max_dim(wide ? 2 : 1) || rows.N == 0)
+    return 0;
   const int cpl = pick_cpl(rows.rs.nch);
   if (cpl < 0) return 0;
-  DCHECK(buf.alloc((size_t)rows.N * kQChunks * 16));
+  const int qc = rows.dim <= q_max_dim(1) ? 1 : 2;
+  DCHECK(buf.alloc((size_t)rows.N * q_chunks(qc) * 16));
   const uint32_t grid = (uint32_t)(((uint64_t)rows.N * 8 + 255) / 256);  // one octet per row
+  auto go = [&](auto dt, auto q) {
+    hipLaunchKernelGGL((k_quantize<decltype(dt)::value, decltype(q)::value>), dim3(grid), dim3(256), 0, s, rows.rs,
+                       rows.N, rows.dim, buf.as<uint4>());
+  };
   if (rows.dtype == DANCE_F32)
-    hipLaunchKernelGGL(k_quantize<DANCE_F32>, dim3(grid), dim3(256), 0, s, rows.rs, rows.N, rows.dim, buf.as<uint4>());
+    qc == 1 ? go(IC<DANCE_F32>{}, IC<1>{}) : go(IC<DANCE_F32>{}, IC<2>{});
   else
-    hipLaunchKernelGGL(k_quantize<DANCE_F16>, dim3(grid), dim3(256), 0, s, rows.rs, rows.N, rows.dim, buf.as<uint4>());
+    qc == 1 ? go(IC<DANCE_F16>{}, IC<1>{}) : go(IC<DANCE_F16>{}, IC<2>{});
   DHIP(hipGetLastError());
   const double lane_terms = (double)cpl * (16.0 / elem_bytes(rows.dtype));
   if (rows.dtype == DANCE_F32) {
-    *out = QBoundSet{buf.as<uint4>(), (float)(2.0 * (lane_terms + 8.0) * 0x1p-24), 1e-30f};
+    *out = QBoundSet{buf.as<uint4>(), qc, (float)(2.0 * (lane_terms + 8.0) * 0x1p-24), 1e-30f};
   } else {  // binary16 differences and squares (see qbound.h)
-    *out = QBoundSet{buf.as<uint4>(), (float)(2.0 * (3.0 * 0x1p-11 + (lane_terms + 8.0) * 0x1p-24)),
+    *out = QBoundSet{buf.as<uint4>(), qc, (float)(2.0 * (3.0 * 0x1p-11 + (lane_terms + 8.0) * 0x1p-24)),
                      (float)(1e-30 + (double)rows.dim * 0x1p-24)};
   }
   return 0;
@@ -281,9 +287,8 @@ static int launch_search(const Rows& rows, GraphBufs g, uint32_t L, uint32_t ste
   return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int DT = decltype(dt)::value, CPL = decltype(c)::value;
     // Bounded variants exist only where build_qbound can produce code rows.
-    constexpr bool kHasQB = DT != DANCE_U8 && CPL <= 4;
-    if constexpr (kHasQB) {
-      if (qb.rows && L <= 256) {
+    if constexpr (q_width(DT, CPL, 1)) {
+      if (qb.rows && qb.groups == 1 && L <= 256) {
         // (fp16 rows of at most 112 dims take 2 chunks per lane)
         if constexpr (CPL <= (is_f16(DT) ? 2 : 3)) {
           if (insert_bound && L <= 128 && g.C <= 128) {  // nA <= C <= 128 fits the open-pair list
@@ -301,6 +306,18 @@ static int launch_search(const Rows& rows, GraphBufs g, uint32_t L, uint32_t ste
           hipLaunchKernelGGL((k_search<DT, CPL, 2, true>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp);
         else
           hipLaunchKernelGGL((k_search<DT, CPL, 4, true>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp);
+        DHIP(hipGetLastError());
+        return 0;
+      }
+    }
+    if constexpr (q_width(DT, CPL, 2)) {
+      if (qb.rows && qb.groups == 2 && L <= 256) {
+        if (L <= 128 && hashed_cur)
+          hipLaunchKernelGGL((k_search<DT, CPL, 2, true, false, true, 2>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp);
+        else if (L <= 128)
+          hipLaunchKernelGGL((k_search<DT, CPL, 2, true, false, false, 2>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp);
+        else
+          hipLaunchKernelGGL((k_search<DT, CPL, 4, true, false, false, 2>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp);
         DHIP(hipGetLastError());
         return 0;
       }
@@ -350,11 +367,18 @@ static int launch_prune(const Rows& rows, GraphBufs g, uint32_t min_degree, floa
   const bool rank = Cp <= kRankCap && rank_kernel;
   return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int DT = decltype(dt)::value, CPL = decltype(c)::value;
-    constexpr bool kHasQB = DT != DANCE_U8 && CPL <= 4;
     if (rank) {
-      if constexpr (kHasQB) {
-        if (qb.rows) {
+      if constexpr (q_width(DT, CPL, 1)) {
+        if (qb.rows && qb.groups == 1) {
           hipLaunchKernelGGL((k_prune_rank<DT, CPL, kRankBound>), xcd_grid(g.N), dim3(kBlock),
+                             (size_t)kWavesPerBlock * prune_rank_lds_words(Cq, true) * 4, s, a, Cq);
+          DHIP(hipGetLastError());
+          return 0;
+        }
+      }
+      if constexpr (q_width(DT, CPL, 2)) {
+        if (qb.rows && qb.groups == 2) {
+          hipLaunchKernelGGL((k_prune_rank<DT, CPL, kRankBound, 2>), xcd_grid(g.N), dim3(kBlock),
                              (size_t)kWavesPerBlock * prune_rank_lds_words(Cq, true) * 4, s, a, Cq);
           DHIP(hipGetLastError());
           return 0;
@@ -362,7 +386,7 @@ static int launch_prune(const Rows& rows, GraphBufs g, uint32_t min_degree, floa
       }
       // without code rows the bound is off: uint8 rows take every pair's
       // distance from Gram tiles, other rows test every pair exactly
-      a.qb = QBoundSet{nullptr, 0.0f, 0.0f};
+      a.qb = QBoundSet{};
       if constexpr (DT == DANCE_U8) {
         if (prune_gram()) {
           hipLaunchKernelGGL((k_prune_rank<DT, CPL, kRankGram>), xcd_grid(g.N), dim3(kBlock),
@@ -376,8 +400,15 @@ static int launch_prune(const Rows& rows, GraphBufs g, uint32_t min_degree, floa
       DHIP(hipGetLastError());
       return 0;
     }
-    hipLaunchKernelGGL((k_prune<DT, CPL>), xcd_grid(g.N), dim3(kBlock),
-                       (size_t)kWavesPerBlock * prune_lds_words(Cp, Rp) * 4, s, a, Cp, Rp);
+    const size_t lds = (size_t)kWavesPerBlock * prune_lds_words(Cp, Rp) * 4;
+    if constexpr (q_width(DT, CPL, 2)) {
+      if (qb.rows && qb.groups == 2) {
+        hipLaunchKernelGGL((k_prune<DT, CPL, 2>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp, Rp);
+        DHIP(hipGetLastError());
+        return 0;
+      }
+    }
+    hipLaunchKernelGGL((k_prune<DT, CPL, 1>), xcd_grid(g.N), dim3(kBlock), lds, s, a, Cp, Rp);
     DHIP(hipGetLastError());
     return 0;
   });
@@ -587,7 +618,11 @@ static int build_schedule(const Rows& rows, const QBoundSet& qb, ReverseWs& ws, 
   const char* em = std::getenv("DANCE_CELLS_MFMA");
   const bool mfma_cells = !(em && em[0] == '0');
   const dim3 mgrid((uint32_t)(((uint64_t)N + 127) / 128));
-  if (qb.rows && mfma_cells) {
+  if (qb.rows && qb.groups == 2) {
+    hipLaunchKernelGGL((k_cells_mfma<false, 8>), mgrid, dim3(256), 0, s, qb.rows, q_chunks(2), N, dpiv.as<uint32_t>(),
+                       K, lv, kb[0], vb[0]);
+    DHIP(hipGetLastError());
+  } else if (qb.rows && mfma_cells) {
     hipLaunchKernelGGL((k_cells_mfma<false, 4>), mgrid, dim3(256), 0, s, qb.rows, kQChunks, N, dpiv.as<uint32_t>(), K,
                        lv, kb[0], vb[0]);
     DHIP(hipGetLastError());
@@ -701,7 +736,7 @@ static int validate(uint32_t N, uint32_t dim, uint32_t R, uint32_t L, uint32_t C
 // Callers hold g_mu and pass the active profile.
 static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint32_t STEPS, const Profile& prof,
                      State& st, hipStream_t s, GPUVamanaStats* stats, DanceKernelProfile* kp, uint32_t* medoid_out,
-                     bool timed = true) {
+                     bool timed = true, bool wide_bound = true) {
   const uint32_t N = rows.N;
   if (pick_cpl(rows.rs.nch) < 0) {
     std::fprintf(stderr, "[gpu_vamana_build] dim=%u is beyond the supported row width\n", rows.dim);
@@ -753,7 +788,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   if (!init_in_search) DCHECK(launch_init(rows, g, s));
   DevBuf qbuf;
   QBoundSet qb{};
-  DCHECK(build_qbound(rows, qbuf, s, &qb));
+  DCHECK(build_qbound(rows, qbuf, s, &qb, wide_bound));
   const uint32_t* order = nullptr;
   DCHECK(build_schedule(rows, qb, rws, s, &order));
   uint32_t q_iters = qbound_iters();  // later iterations' bits may be set on the way (kDenseFrac)
@@ -788,7 +823,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     if (verbose())
       std::printf("[gpu_vamana_build] iteration %u / %u, alpha=%.3f\n", it + 1, iters, (double)alpha);
     DCHECK(record(iev[it].s0, s));
-    const QBoundSet qb_it = ((q_iters >> it) & 1u) ? qb : QBoundSet{nullptr, 0.0f, 0.0f};
+    const QBoundSet qb_it = ((q_iters >> it) & 1u) ? qb : QBoundSet{};
     DCHECK(launch_search(rows, g, L, steps, alpha, start, order, ctr, qb_it, s, ((ib_iters >> it) & 1u) != 0,
                          it == 0, true));  // k_init wrote cur just before
     DCHECK(record(iev[it].s1, s));
@@ -798,7 +833,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     DCHECK(launch_merge(g, rev, prof, order, ctr, s));
     DCHECK(record(iev[it].m1, s));
     const uint32_t md = (it + 1 == iters) ? kFinalMinDegree : 0u;
-    const QBoundSet qp_it = ((q_prune_iters >> it) & 1u) ? qb : QBoundSet{nullptr, 0.0f, 0.0f};
+    const QBoundSet qp_it = ((q_prune_iters >> it) & 1u) ? qb : QBoundSet{};
     DCHECK(launch_prune(rows, g, md, alpha, order, ctr, qp_it, ((p_rank >> it) & 1u) != 0u, s));
     DCHECK(record(iev[it].p1, s));
     if (it == 0 && qb.rows && iters > 1 && (qbound_prune_adaptive() || qbound_iters_adaptive())) {
@@ -902,6 +937,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   p.insert_bound_checks = hc_ctr.insert_bound_checks;
   p.insert_bound_skips = hc_ctr.insert_bound_skips;
   const double V = rows.vbytes();
+  const double qrow_bytes = q_chunks(qb.rows ? qb.groups : 1) * 16.0;
   for (uint32_t it = 0; timed && it < iters; ++it) {
     const VCounters& c = hsnap[it];
     const VCounters z{};
@@ -926,7 +962,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     const double per_vertex = init_it ? V + R * V + 8.0 * C : V + 4.0 * R + 4.0 + 16.0 * C;
     p.search_bytes_iter[it] = (double)(p.search_dist_iter[it] + p.insert_dist_iter[it]) * V +
                               (double)p.expansions_iter[it] * adj + (double)N * per_vertex +
-                              (double)(p.bound_checks_iter[it] + p.insert_bound_checks_iter[it]) * (kQChunks * 16.0);
+                              (double)(p.bound_checks_iter[it] + p.insert_bound_checks_iter[it]) * qrow_bytes;
     // the rank kernel with the bound reads every candidate's code row once;
     // k_prune reads the code rows of the pairs it tests; the rank kernel's
     // Gram tiles (uint8 rows) read every candidate's row once for all pairs
@@ -934,14 +970,14 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     const bool rank_it = ((p_rank >> it) & 1u) && C <= kRankCap;
     const bool gram_it = rank_it && rows.dtype == DANCE_U8 && prune_gram();
     const double qbytes = !q_it ? 0.0
-                          : rank_it ? (double)N * C * (kQChunks * 16.0)
-                                    : (double)p.prune_bound_checks_iter[it] * (kQChunks * 16.0);
+                          : rank_it ? (double)N * C * qrow_bytes
+                                    : (double)p.prune_bound_checks_iter[it] * qrow_bytes;
     const double pair_rows = gram_it ? (double)N * C : (double)p.prune_dist_iter[it];
     p.prune_bytes_iter[it] = pair_rows * V + (double)N * (24.0 * C) + qbytes;
   }
   p.search_bytes = (double)(p.search_dist + p.insert_dist) * V + (double)p.expansions * (4.0 * R + 4.0) +
                    (double)iters * N * (V + 4.0 * R + 4.0 + 16.0 * C) +
-                   (double)(p.bound_checks + p.insert_bound_checks) * (kQChunks * 16.0);
+                   (double)(p.bound_checks + p.insert_bound_checks) * qrow_bytes;
   if (timed) {  // the per-launch figures know which launch recomputed its adjacency rows
     p.search_bytes = 0.0;
     for (uint32_t it = 0; it < iters; ++it) p.search_bytes += p.search_bytes_iter[it];
@@ -949,7 +985,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   p.merge_bytes = (double)p.merge_dist * 4.0 + (double)p.reverse_edges * 4.0 +
                   (double)p.touched_rows * (16.0 * C + 8.0);
   p.prune_bytes = (double)p.prune_dist * V + (double)iters * N * (24.0 * C) +
-                  (double)p.prune_bound_checks * (kQChunks * 16.0);
+                  (double)p.prune_bound_checks * qrow_bytes;
   if (timed) {  // the per-launch figures know which launches used Gram tiles
     p.prune_bytes = 0.0;
     for (uint32_t it = 0; it < iters; ++it) p.prune_bytes += p.prune_bytes_iter[it];
@@ -1134,9 +1170,9 @@ __global__ __launch_bounds__(kBlock) void k_qbound_pairs(QBoundSet qb, const uin
     const uint4 h = qa[0];
     const float s = __uint_as_float(h.x), r = __uint_as_float(h.y), lo = __uint_as_float(h.z);
     const QLower me = q_lower(s, r, lo, q_threshold(qb, r, act ? T[k] : 0.0f));
-    const uint4 code = q_codes(qa[sub], sub);
-    const uint4 bc = q_load(qb, act ? b[k] : 0u, act, sub);
-    const bool rej = q_proves_reject(me, code, bc);
+    const QCodes<1> code = q_codes<1>(q_load<1>(qb, act ? a[k] : 0u, true, sub), sub);
+    const QCodes<1> bc = q_load<1>(qb, act ? b[k] : 0u, act, sub);
+    const bool rej = q_proves_reject<1>(me, code, bc);
     if (act && sub == 0) flag[k] = rej ? 1u : 0u;
   }
 }
@@ -1165,11 +1201,11 @@ __global__ __launch_bounds__(kBlock) void k_insert_bound_pairs(QBoundSet qb, con
     const float t0 = act ? T0[k] : 0.0f;
     const QUpper up = q_upper(xs, xr, xhi, q_ub_root_of<DT>(qb, t0, alpha));
     const QLower low = q_lower(xs, xr, xlo, (prune_bound_root(qb, t0, alpha) + xr) * (1.0f + kQSlack));
-    const uint4 bc = q_load(qb, act ? b[k] : 0u, act, sub);
-    const int c = q_octet_dot(q_codes(qx[sub], sub), bc);
-    const float sy = __uint_as_float(bc.x), ry = __uint_as_float(bc.y);
-    const bool yes = q_upper_proves(up, sy, ry, __uint_as_float(bc.w), c);
-    const bool no = q_lower_proves(low, sy, ry, __uint_as_float(bc.z), c);
+    const QCodes<1> bc = q_load<1>(qb, act ? b[k] : 0u, act, sub);
+    const int c = q_octet_dot<1>(q_codes<1>(q_load<1>(qb, act ? a[k] : 0u, true, sub), sub), bc);
+    const float sy = __uint_as_float(bc.c[0].x), ry = __uint_as_float(bc.c[0].y);
+    const bool yes = q_upper_proves(up, sy, ry, __uint_as_float(bc.c[0].w), c);
+    const bool no = q_lower_proves(low, sy, ry, __uint_as_float(bc.c[0].z), c);
     if (act && sub == 0) out[k] = yes ? 1u : (no ? 2u : 0u);
   }
 }
@@ -1217,7 +1253,7 @@ static int scratch_base(void** out) {
 // same buffers run_build, setup_rows and the radix sort allocate, each rounded
 // up to the arena's 256-byte alignment.
 static size_t resident_build_bytes(const void* d_data, int dtype, int store, uint32_t N, uint32_t dim, uint32_t R,
-                                   uint32_t C, bool rows_ready = false) {
+                                   uint32_t C, bool rows_ready = false, bool wide_bound = true) {
   size_t total = 0;
   auto add = [&](size_t b) { total += (b + 255u) & ~(size_t)255u; };
   const size_t row_bytes = (size_t)dim * elem_bytes(store);
@@ -1246,7 +1282,8 @@ static size_t resident_build_bytes(const void* d_data, int dtype, int store, uin
   add(sizeof(VCounters));           // summed counters (the prune bound's choice for iteration 1)
   add(kMedoidCandidates * 4);       // scores
   add(kMedoidCandidates * 4);       // cands
-  add((size_t)N * kQChunks * 16);   // code rows of the bound
+  const bool wide = wide_bound && store != DANCE_U8 && dim > q_max_dim(1) && dim <= q_max_dim(2);
+  add((size_t)N * q_chunks(wide ? 2 : 1) * 16);  // code rows of the bound
   add((size_t)locality_cells(store, N) * 4);  // pivots
   add((size_t)N * 4);               // order
   for (size_t n : {(size_t)N, sort_items}) {  // the schedule's sort, then the reverse sort
@@ -1284,8 +1321,13 @@ static int resident_build(const void* d_data, int dtype, uint32_t N, uint32_t di
   const int store = (dtype == DANCE_F32 && prof.fp16) ? DANCE_F16 : dtype;
   DCHECK(check_width(dim, store));
   Arena arena;
+  bool wide_bound = true;
   if (noalloc) {
-    const size_t need = resident_build_bytes(d_data, dtype, store, N, dim, R, C);
+    size_t need = resident_build_bytes(d_data, dtype, store, N, dim, R, C);
+    if (need > kScratchBytes) {  // without the two-group code rows, which only save time
+      wide_bound = false;
+      need = resident_build_bytes(d_data, dtype, store, N, dim, R, C, false, false);
+    }
     if (need > kScratchBytes) {
       std::fprintf(stderr,
                    "[gpu_vamana_build] allocation-free build: N=%u dim=%u R=%u C=%u needs %zu bytes of scratch, "
@@ -1315,7 +1357,7 @@ static int resident_build(const void* d_data, int dtype, uint32_t N, uint32_t di
   GPUVamanaStats stats{};
   DanceKernelProfile kp{};
   uint32_t medoid = 0;
-  int r = run_build(rows, R, L, C, STEPS, prof, st, s, &stats, &kp, &medoid, !noalloc);
+  int r = run_build(rows, R, L, C, STEPS, prof, st, s, &stats, &kp, &medoid, !noalloc, wide_bound);
   st.cur.release();
   st.deg_cur.release();
   if (r != 0) return r;
@@ -1795,7 +1837,7 @@ int dance_stage_qbound(const void* h_data, int dtype, uint32_t N, uint32_t dim, 
   DevBuf qbuf, da, db, dt, dout;
   QBoundSet qb{};
   DCHECK(build_qbound(cx.rows, qbuf, cx.s, &qb));
-  if (!qb.rows) {
+  if (!qb.rows || qb.groups != 1) {
     std::fprintf(stderr, "[dance_hip] no distance bound for this row type / width (or DANCE_QBOUND=0)\n");
     return -1;
   }
@@ -1831,7 +1873,7 @@ int dance_stage_insert_bound(const void* h_data, int dtype, uint32_t N, uint32_t
   DevBuf qbuf, da, db, dt, dout;
   QBoundSet qb{};
   DCHECK(build_qbound(cx.rows, qbuf, cx.s, &qb));
-  if (!qb.rows) {
+  if (!qb.rows || qb.groups != 1) {
     std::fprintf(stderr, "[dance_hip] no distance bound for this row type / width (or DANCE_QBOUND=0)\n");
     return -1;
   }

@@ -412,7 +412,7 @@ __host__ __device__ constexpr uint32_t search_lds_words(uint32_t Cp) { return kV
 // cur row and degree: the same values, without three random cache lines per
 // expansion; and it computes the vertex's own initial row and distances as
 // k_init would, so that the build skips k_init.
-template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false>
+template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false, int QC = 1>
 struct SearchWave {
   const SearchArgs& a;
   uint32_t node, lane, grp, sub, Cp;
@@ -455,20 +455,21 @@ struct SearchWave {
     me.m2s = uni_f(me.m2s);
     me.n2S = uni_f(me.n2S);
     me.K = uni_f(me.K);
-    const uint4 code = q_codes(qme.row[sub], sub);
+    const QCodes<QC> code = q_codes<QC>(q_load<QC>(a.qb, node, true, sub), sub);
+    constexpr uint32_t F = kQInFlight / QC;
     uint32_t nk = 0;
-    for (uint32_t p = 0; p < n; p += 8 * kQInFlight) {
-      uint4 b[kQInFlight];
+    for (uint32_t p = 0; p < n; p += 8 * F) {
+      QCodes<QC> b[F];
 #pragma unroll
-      for (uint32_t u = 0; u < kQInFlight; ++u) {
+      for (uint32_t u = 0; u < F; ++u) {
         const uint32_t k = p + 8 * u + grp;
-        b[u] = q_load(a.qb, lst[k], k < n, sub);  // k < 64 (p steps by 8 kQInFlight, which divides 64)
+        b[u] = q_load<QC>(a.qb, lst[k], k < n, sub);  // k < 64 (p steps by 8 F, which divides 64)
       }
 #pragma unroll
-      for (uint32_t u = 0; u < kQInFlight; ++u) {
+      for (uint32_t u = 0; u < F; ++u) {
         if (p + 8 * u >= n) break;  // uniform
         const uint32_t k = p + 8 * u + grp;
-        const bool keep = !q_proves_reject(me, code, b[u]) && sub == 0u && k < n;
+        const bool keep = !q_proves_reject<QC>(me, code, b[u]) && sub == 0u && k < n;
         const uint64_t m = wballot(keep);
         if (keep) lst[nk + mbcnt64(m)] = lst[k];
         nk += popc64(m);
@@ -614,7 +615,7 @@ struct SearchWave {
   }
 
   // The occlusion test of robust_insert with the insert bound: a pass of 8
-  // candidates first tests its pairs on the code rows (x's chunk in xchunk).
+  // candidates first tests its pairs on the code rows (x's code row in xrow).
   // An upper bound that proves fl(alpha * d(y, x)) <= d_px proves an
   // occluder and ends the test; pairs whose lower bound proves the opposite
   // need nothing more; the others collect their ids in lst and lsd (128
@@ -622,26 +623,26 @@ struct SearchWave {
   // distances, in passes of 8, once the bound passes end. The answer is the
   // exact test's: every decision the bounds make is the one the exact
   // distance would give, and the answer does not depend on the order.
-  __device__ __forceinline__ bool occlusion_bounded(uint32_t x, float dpx, const uint4& xchunk, uint32_t nU,
+  __device__ __forceinline__ bool occlusion_bounded(uint32_t x, float dpx, const QCodes<QC>& xrow, uint32_t nU,
                                                     uint32_t nA) {
     // x's header: lane 0 holds chunk 0 of its code row
-    const float xs = __uint_as_float(rdlane_u(xchunk.x, 0));
-    const float xr = __uint_as_float(rdlane_u(xchunk.y, 0));
-    const float xlo = __uint_as_float(rdlane_u(xchunk.z, 0));
-    const float xhi = __uint_as_float(rdlane_u(xchunk.w, 0));
+    const float xs = __uint_as_float(rdlane_u(xrow.c[0].x, 0));
+    const float xr = __uint_as_float(rdlane_u(xrow.c[0].y, 0));
+    const float xlo = __uint_as_float(rdlane_u(xrow.c[0].z, 0));
+    const float xhi = __uint_as_float(rdlane_u(xrow.c[0].w, 0));
     const QUpper up = q_upper(xs, xr, xhi, q_ub_root_of<DT>(a.qb, dpx, a.alpha));
     const QLower low = q_lower(xs, xr, xlo, (prune_bound_root(a.qb, dpx, a.alpha) + xr) * (1.0f + kQSlack));
-    const uint4 xcode = q_codes(xchunk, sub);
+    const QCodes<QC> xcode = q_codes<QC>(xrow, sub);
     uint32_t* pend = lst;
     uint32_t nopen = 0;
     for (uint32_t p = 0; p < nA; p += 8) {
       const uint32_t k0 = p + grp;
       const bool a0 = k0 < nA;
       const uint32_t y0 = a0 ? wid[ord[nU + k0]] : 0u;
-      const uint4 b = q_load(a.qb, y0, a0, sub);
-      const int c = q_octet_dot(xcode, b);
-      const float sy = __uint_as_float(b.x), ry = __uint_as_float(b.y);
-      const float loy = __uint_as_float(b.z), hiy = __uint_as_float(b.w);
+      const QCodes<QC> b = q_load<QC>(a.qb, y0, a0, sub);
+      const int c = q_octet_dot<QC>(xcode, b);
+      const float sy = __uint_as_float(b.c[0].x), ry = __uint_as_float(b.c[0].y);
+      const float loy = __uint_as_float(b.c[0].z), hiy = __uint_as_float(b.c[0].w);
       const bool lead = sub == 0u && a0;
       const uint32_t np = min(8u, nA - p);
       n_ibchk += np;
@@ -683,9 +684,9 @@ struct SearchWave {
     // repeated x leaves it unused).
     constexpr bool kIB = QB && IB && DT != DANCE_U8;
     uint4 xv[CPL];
-    uint4 xcode;
+    QCodes<QC> xcode;
     if constexpr (kIB)
-      xcode = a.qb.rows[(size_t)x * kQChunks + sub];  // launched only with code rows present
+      xcode = q_load<QC>(a.qb, x, true, sub);  // launched only with code rows present
     else
       load_row<CPL>(a.rs, x, true, sub, xv);
     // One pass over the row: x already there ends the insert; otherwise the
@@ -815,7 +816,7 @@ struct SearchWave {
     const uint32_t N = g.N, R = g.R, C = g.C;
     load_row<CPL>(a.rs, node, true, sub, av);
     av_sq = self_term<DT, CPL>(av);
-    if (QB && a.qb.rows) q_load_self(a.qb, node, qme);
+    if (QB && a.qb.rows) q_load_self<QC>(a.qb, node, qme);
     // Work row := current row with its stored distances (vnew2.cu:1186-1212).
     // With HC the current row is the random initial graph's, computed here
     // with its distances as k_init computes them (init_neighbor, batch_dist
@@ -1023,14 +1024,14 @@ constexpr int kSearchMinWaves =
         : (CPL <= 2 && PS == 4) ? (QB ? 5 : 6) : (PS == 2 && !QB && CPL <= 8) ? (CPL == 4 ? 6 : 4) : 1;
 
 // search_prune_kernel_shared (vnew2.cu:1119-1439).
-template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false>
+template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false, int QC = 1>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSearchMinWaves<CPL, PS, QB, IB, HC>, 8))) void k_search(SearchArgs a, uint32_t Cp) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t gw = xcd_block(grid_block(), grid_blocks()) * kWavesPerBlock + w;
   if (gw >= a.g.N) return;
   const uint32_t node = a.order ? a.order[gw] : gw;
-  SearchWave<DT, CPL, PS, QB, IB, HC> sw(a, node, smem + w * search_lds_words(Cp), Cp);
+  SearchWave<DT, CPL, PS, QB, IB, HC, QC> sw(a, node, smem + w * search_lds_words(Cp), Cp);
   sw.run();
 }
 
@@ -1052,7 +1053,7 @@ __host__ __device__ constexpr uint32_t prune_lds_words(uint32_t Cp, uint32_t Rp)
 
 constexpr uint32_t PR_REMOVED = 1u, PR_INOUT = 2u;
 
-template <int DT, int CPL>
+template <int DT, int CPL, int QC>
 __global__ __launch_bounds__(kBlock) void k_prune(PruneArgs a, uint32_t Cp, uint32_t Rp) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
@@ -1132,29 +1133,29 @@ __global__ __launch_bounds__(kBlock) void k_prune(PruneArgs a, uint32_t Cp, uint
     if (qon) {
       // Drop the candidates whose pair distance the bound proves large
       // enough to keep them; their exact distance cannot remove them.
-      const uint4* qs = a.qb.rows + (size_t)sel * kQChunks;
-      const uint4 chunk = qs[sub];
-      const float ss = __uint_as_float(rdlane_u(chunk.x, 0)), sr = __uint_as_float(rdlane_u(chunk.y, 0)),
-                  slo = __uint_as_float(rdlane_u(chunk.z, 0));
-      const uint4 code = q_codes(chunk, sub);
+      const QCodes<QC> qs = q_load<QC>(a.qb, sel, true, sub);
+      const float ss = __uint_as_float(rdlane_u(qs.c[0].x, 0)), sr = __uint_as_float(rdlane_u(qs.c[0].y, 0)),
+                  slo = __uint_as_float(rdlane_u(qs.c[0].z, 0));
+      const QCodes<QC> code = q_codes<QC>(qs, sub);
+      constexpr uint32_t F = kQInFlight / QC;
       uint32_t nk = 0;
       for (uint32_t base = 0; base < nq; base += 64) {  // lst holds up to C entries
         const uint32_t nb = min(64u, nq - base);
         uint64_t keep = 0;
-        for (uint32_t p = 0; p < nb; p += 8 * kQInFlight) {
-          uint4 b[kQInFlight];
-          uint32_t si[kQInFlight];
+        for (uint32_t p = 0; p < nb; p += 8 * F) {
+          QCodes<QC> b[F];
+          uint32_t si[F];
 #pragma unroll
-          for (uint32_t u = 0; u < kQInFlight; ++u) {
+          for (uint32_t u = 0; u < F; ++u) {
             const uint32_t k = p + 8 * u + grp;
             si[u] = lst[min(base + k, Cp - 1u)];
-            b[u] = q_load(a.qb, sid[si[u]], k < nb, sub);
+            b[u] = q_load<QC>(a.qb, sid[si[u]], k < nb, sub);
           }
 #pragma unroll
-          for (uint32_t u = 0; u < kQInFlight; ++u) {
+          for (uint32_t u = 0; u < F; ++u) {
             const uint32_t k = p + 8 * u + grp;
             const QLower me = q_lower(ss, sr, slo, (sroot[si[u]] + sr) * (1.0f + kQSlack));
-            const bool prove = q_proves_reject(me, code, b[u]);
+            const bool prove = q_proves_reject<QC>(me, code, b[u]);
             keep |= (uint64_t)octet_bits(wballot(sub == 0 && k < nb && !prove)) << (p + 8 * u);
           }
         }
@@ -1285,17 +1286,18 @@ __host__ __device__ constexpr uint32_t prune_rank_lds_words(uint32_t Cq, bool ti
 }
 
 // 16 code bytes of rank row `row` for MFMA K-step `step`: code chunk
-// 1 + 2 step + lane/32 (chunk 0 is the header; chunks past 7 are zero).
+// 1 + 2 step + lane/32 (chunk 0 is the header; chunks past the row are zero).
 // Both operands of a Gram tile take their rows this way, so the tile sums
 // every code byte of a pair exactly once (layout checked on gfx950: lane l
 // supplies row l % 32, and D[i][j] sits in accumulator v of lane l with
 // j = l % 32, i = 8 (v / 4) + 4 (l / 32) + v % 4).
+template <int QC>
 __device__ __forceinline__ v4i_t code_frag(const QBoundSet& qb, const uint32_t* rid, uint32_t row, uint32_t nvalid,
                                            uint32_t step, uint32_t lane) {
   const uint32_t chunk = 1u + 2u * step + (lane >> 5);
   v4i_t v = {0, 0, 0, 0};
-  if (row < nvalid && chunk < kQChunks) {
-    const uint4 c = qb.rows[(size_t)rid[row] * kQChunks + chunk];
+  if (row < nvalid && chunk < q_chunks(QC)) {
+    const uint4 c = qb.rows[(size_t)rid[row] * q_chunks(QC) + chunk];
     v = v4i_t{(int)c.x, (int)c.y, (int)c.z, (int)c.w};
   }
   return v;
@@ -1307,12 +1309,15 @@ __device__ __forceinline__ uint32_t ffs128(uint64_t m0, uint64_t m1) {
 
 // Occupancy floor: the bound's variant holds every code fragment of up to 96
 // ranks (48 registers) next to its MFMA accumulators, which fits 5 waves per
-// SIMD; the variant without it fits 6 at rows of up to 4 chunks per lane.
-// Wider rows (and fp16 rows of 4 chunks per lane) get no floor, so no variant
-// spills.
+// SIMD; at 8 chunks per lane its batch of exact pairs holds 4 rows of 32
+// registers, which 3 waves leave room for (5 spilled 264 bytes and took 7.3
+// instead of 2.5 ms at 200k x 200). The variant without it fits 6 at rows of
+// up to 4 chunks per lane. Wider rows (and fp16 rows of 4 chunks per lane) get
+// no floor, so no variant spills.
 template <int DT, int CPL, int PM>
-constexpr int kRankMinWaves = PM != kRankExact ? 5 : (CPL < 4 || (CPL == 4 && !is_f16(DT))) ? 6 : 1;
-template <int DT, int CPL, int PM>
+constexpr int kRankMinWaves =
+    PM != kRankExact ? (PM == kRankBound && CPL >= 8 ? 3 : 5) : (CPL < 4 || (CPL == 4 && !is_f16(DT))) ? 6 : 1;
+template <int DT, int CPL, int PM, int QC = 1>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMinWaves<DT, CPL, PM>, 8))) void k_prune_rank(PruneArgs a, uint32_t Cq) {
   constexpr bool QB = PM == kRankBound, XG = PM == kRankGram;
   static_assert(!XG || DT == DANCE_U8, "Gram tiles give exact distances of uint8 rows only");
@@ -1420,7 +1425,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
       if (r < Cq) {
         float4 v = make_float4(0.0f, __builtin_inff(), 0.0f, 0.0f);
         if (r < nvalid) {
-          const uint4 hd = a.qb.rows[(size_t)rid[r] * kQChunks];
+          const uint4 hd = a.qb.rows[(size_t)rid[r] * q_chunks(QC)];
           v = make_float4(__uint_as_float(hd.x), __uint_as_float(hd.y), __uint_as_float(hd.z),
                           prune_bound_root(a.qb, rd[r], a.alpha));
         }
@@ -1431,10 +1436,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
     const uint32_t nt = (nvalid + 31u) >> 5;
     const uint32_t jl = lane & 31u, ih = 4u * (lane >> 5);
     // One 32 x 32 tile of pair decisions: rows ti, columns tj >= ti.
-    auto tile = [&](uint32_t ti, uint32_t tj, const v4i_t(&fa)[4], const v4i_t(&fb)[4]) {
-      v16i_t acc = {};
-#pragma unroll
-      for (uint32_t s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s], fb[s], acc, 0, 0, 0);
+    auto tile = [&](uint32_t ti, uint32_t tj, const v16i_t& acc) {
       // j-side values per lane (j queries with its own root); i-side per
       // accumulator from LDS. Invalid ranks carry r = inf, which proves nothing.
       const uint32_t j = tj * 32u + jl;
@@ -1452,32 +1454,40 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
       });
       if (lane < 32u) pm[4u * (ti * 32u + lane) + tj] = words;
     };
-    if (nt <= 3u) {
+    constexpr uint32_t S = 4u * QC;  // K-steps of 32 code bytes
+    if (QC == 1 && nt <= 3u) {
       // up to 96 ranks: every code fragment loaded at once, then the tiles
-      v4i_t F[3][4];
+      v4i_t F[3][S];
       static_for<0, 3>([&](auto tc) {
         constexpr uint32_t t = decltype(tc)::value;
 #pragma unroll
-        for (uint32_t s = 0; s < 4; ++s) F[t][s] = code_frag(a.qb, rid, t * 32u + jl, nvalid, s, lane);
+        for (uint32_t s = 0; s < S; ++s) F[t][s] = code_frag<QC>(a.qb, rid, t * 32u + jl, nvalid, s, lane);
       });
       static_for<0, 3>([&](auto ic) {
         constexpr uint32_t ti = decltype(ic)::value;
         static_for<ti, 3>([&](auto jc) {
           constexpr uint32_t tj = decltype(jc)::value;
-          if (tj < nt) tile(ti, tj, F[ti], F[tj]);
+          if (tj < nt) {
+            v16i_t acc = {};
+#pragma unroll
+            for (uint32_t s = 0; s < S; ++s) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(F[ti][s], F[tj][s], acc, 0, 0, 0);
+            tile(ti, tj, acc);
+          }
         });
       });
     } else {
       for (uint32_t ti = 0; ti < nt; ++ti) {
-        v4i_t fa[4];
+        v4i_t fa[S];
 #pragma unroll
-        for (uint32_t s = 0; s < 4; ++s) fa[s] = code_frag(a.qb, rid, ti * 32u + jl, nvalid, s, lane);
-        tile(ti, ti, fa, fa);
-        for (uint32_t tj = ti + 1u; tj < nt; ++tj) {
-          v4i_t fb[4];
+        for (uint32_t s = 0; s < S; ++s) fa[s] = code_frag<QC>(a.qb, rid, ti * 32u + jl, nvalid, s, lane);
+        for (uint32_t tj = ti; tj < nt; ++tj) {
+          v16i_t acc = {};
 #pragma unroll
-          for (uint32_t s = 0; s < 4; ++s) fb[s] = code_frag(a.qb, rid, tj * 32u + jl, nvalid, s, lane);
-          tile(ti, tj, fa, fb);
+          for (uint32_t s = 0; s < S; ++s) {
+            const v4i_t fb = tj == ti ? fa[s] : code_frag<QC>(a.qb, rid, tj * 32u + jl, nvalid, s, lane);
+            acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[s], fb, acc, 0, 0, 0);
+          }
+          tile(ti, tj, acc);
         }
       }
     }

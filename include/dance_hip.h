@@ -39,7 +39,7 @@ typedef struct DanceKernelProfile {
     double search_bytes, merge_bytes, prune_bytes, reverse_bytes;
     /* Search-kernel phase cycles (zero unless built with DANCE_SEARCH_TIMING=1). */
     uint64_t cyc_select, cyc_insert, cyc_dist, cyc_pool, cyc_seed, cyc_total;
-    /* Quantized lower bound of the search (fp32/fp16 rows of <= 112 dims):
+    /* Quantized lower bound of the search (fp32/fp16 rows of <= 240 dims):
      * candidates tested, and those whose exact distance it made unnecessary
      * (proved >= the pool threshold). DANCE_QBOUND=0 disables the bound;
      * DANCE_QBOUND_ITERS selects the iterations (bit i = iteration i);

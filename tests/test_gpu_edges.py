@@ -62,3 +62,29 @@ def test_bound_in_every_iteration_of_dense_data(n, centers, middle):
     checks = r.kernel_profile["bound_checks_iter"]
     assert checks[0] > 0
     assert [c > 0 for c in checks[1:3]] == [middle, middle]
+
+
+# code rows of two chunk groups: widths on both sides of 112, 128 and 240
+# dimensions and of each compiled row group, pools of 2 and 4 slots per lane
+@pytest.mark.parametrize("kind,dim,L", [("f32", 113, 64), ("f32", 128, 140), ("f32", 129, 64), ("f32", 240, 64),
+                                        ("f32", 241, 64), ("f16", 113, 64), ("f16", 128, 64), ("f16", 191, 140),
+                                        ("f16", 192, 64), ("f16", 240, 64), ("f16", 241, 64)])
+@pytest.mark.parametrize("centers", [0, 20])
+def test_wide_code_rows(kind, dim, L, centers):
+    import torch
+    n, R, C, steps = 4000, 32, 48, 32
+    x = rows(kind, n, dim, centers=centers)
+    x[5:9] = x[4]  # equal rows
+    x[30] *= 100 if kind == "f32" else 4
+    if centers == 0:
+        x[11] = np.inf
+        x[12, 3] = np.nan
+    og, od, om = O.vnew2_build(x, R, L, C, steps)
+    xt = torch.from_numpy(x).cuda()
+    g = torch.empty((n, R), dtype=torch.int32, device="cuda")
+    d = torch.empty((n,), dtype=torch.int32, device="cuda")
+    D.vamana_build_resident(xt.data_ptr(), D.dtype_code(x), n, dim, R, L, C, steps, g.data_ptr(), d.data_ptr())
+    assert D.last_medoid() == om
+    assert np.array_equal(d.cpu().numpy().view(np.uint32), od)
+    assert np.array_equal(g.cpu().numpy().view(np.uint32), og)
+    assert (D.last_kernel_profile()["bound_checks"] > 0) == (dim <= 240)
