@@ -351,22 +351,29 @@ inline int copy_pageable(void* dst, const void* src, size_t bytes, hipMemcpyKind
   return 0;
 }
 
-inline int setup_rows(Rows& out, const void* src, bool src_on_device, int src_dtype, int store_dtype, uint32_t N,
-                      uint32_t dim, hipStream_t s) {
+// Fills everything of `out` but the row pointer: the padded layout of N rows.
+// Rows are padded with zeros to the compiled chunk group (8 lanes x CPL
+// chunks of 16 bytes), so every chunk slot of a row holds data and row loads
+// need no per-chunk bounds test; zeros add nothing to a distance. Returns the
+// bytes of a padded row.
+inline size_t row_layout(Rows& out, int store_dtype, uint32_t N, uint32_t dim) {
   out.dtype = store_dtype;
   out.N = N;
   out.dim = dim;
   const size_t row_bytes = (size_t)dim * elem_bytes(store_dtype);
-  // Rows are padded with zeros to the compiled chunk group (8 lanes x CPL
-  // chunks of 16 bytes), so every chunk slot of a row holds data and row
-  // loads need no per-chunk bounds test; zeros add nothing to a distance.
   const uint32_t data_chunks = (uint32_t)((row_bytes + 15) / 16);
   const int cpl = pick_cpl(data_chunks);
   const uint32_t nch = cpl > 0 ? 8u * (uint32_t)cpl : data_chunks;
-  const size_t stride = (size_t)nch * 16;
   out.rs.stride16 = nch;
   out.rs.nch = nch;
   out.rs.tail16 = (store_dtype == DANCE_F16 && (dim & 1u)) ? (int32_t)((dim - 1u) / 2u) : -1;
+  return (size_t)nch * 16;
+}
+
+inline int setup_rows(Rows& out, const void* src, bool src_on_device, int src_dtype, int store_dtype, uint32_t N,
+                      uint32_t dim, hipStream_t s) {
+  const size_t stride = row_layout(out, store_dtype, N, dim);
+  const size_t row_bytes = (size_t)dim * elem_bytes(store_dtype);
   const size_t src_row_bytes = (size_t)dim * elem_bytes(src_dtype);
   if (src_dtype == store_dtype && src_on_device && stride == row_bytes &&
       (reinterpret_cast<uintptr_t>(src) & 15u) == 0) {

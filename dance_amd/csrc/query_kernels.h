@@ -156,6 +156,9 @@ struct QArgs {
   uint32_t* out_ids;     // nq x k
   float* out_d;
   unsigned long long* ctr;  // distances, expansions, capped queries
+  // packed base rows (PACKED kernels): the caller's rows as they are
+  const uint8_t* packed;
+  uint32_t row_bytes;
 };
 
 __device__ __forceinline__ bool q_has_label(const QArgs& a, uint32_t p, uint32_t l) {
@@ -168,7 +171,8 @@ __device__ __forceinline__ bool q_has_label(const QArgs& a, uint32_t p, uint32_t
   return false;
 }
 
-template <int DT, int CPL, int PS>
+// PACKED: the base rows are read where the caller has them (load_packed_row).
+template <int DT, int CPL, int PS, bool PACKED>
 __global__ __launch_bounds__(kBlock) void k_query(RowSet base, RowSet qrows, QArgs a) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
@@ -198,7 +202,15 @@ __global__ __launch_bounds__(kBlock) void k_query(RowSet base, RowSet qrows, QAr
       const uint32_t n = popc64(m);
       if (need) lst[mbcnt64(m)] = c;
       wave_sync();
-      batch_dist<DT, CPL>(base, av, lst, lsd, n, grp, sub);
+      if constexpr (PACKED)
+        batch_dist_by<DT, CPL>(
+            base,
+            [&](uint32_t id, bool active, uint4(&v)[CPL]) {
+              load_packed_row<CPL>(a.packed, a.row_bytes, id, active, sub, v);
+            },
+            av, self_term<DT, CPL>(av), lst, lsd, n, grp, sub);
+      else
+        batch_dist<DT, CPL>(base, av, lst, lsd, n, grp, sub);
       ndist += n;
       const uint32_t ck = lane < n ? lst[lane] : DANCE_INV;
       const float dk = lane < n ? lsd[lane] : FLT_MAX;

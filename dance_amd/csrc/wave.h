@@ -203,6 +203,40 @@ __device__ __forceinline__ void load_row(const RowSet& rs, uint32_t id, bool act
   }
 }
 
+// load_row from packed rows of any byte length and alignment, for callers that
+// read too few rows to be worth a padded copy of all of them: whole chunks by
+// unaligned 16-byte loads, the row's partial last chunk word by word and byte
+// by byte (nothing past the row's end is read), zeros beyond it. row_bytes is
+// a kernel argument.
+template <int CPL>
+__device__ __forceinline__ void load_packed_row(const uint8_t* rows, uint32_t row_bytes, uint32_t id, bool active,
+                                                uint32_t sub, uint4 (&v)[CPL]) {
+  const uint8_t* p = rows + (size_t)id * row_bytes;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    const uint32_t off = 16u * (sub + 8u * (uint32_t)c);
+    v[c] = make_uint4(0u, 0u, 0u, 0u);
+    if (!active || off >= row_bytes) continue;
+    if (off + 16u <= row_bytes) {
+      __builtin_memcpy(&v[c], p + off, 16);
+      continue;
+    }
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+    const uint32_t left = row_bytes - off;  // 1..15, the same for every row
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+      if (4u * k + 4u <= left) {
+        __builtin_memcpy(&w[k], p + off + 4u * k, 4);
+      } else {
+#pragma unroll
+        for (uint32_t b = 0; b < 3; ++b)
+          if (4u * k + b < left) w[k] |= (uint32_t)p[off + 4u * k + b] << (8u * b);
+      }
+    }
+    v[c] = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+}
+
 __device__ __forceinline__ float fma_sq(float a, float b, float acc) {
   const float t = a - b;
   return __builtin_fmaf(t, t, acc);
@@ -349,18 +383,19 @@ __device__ __forceinline__ int fkey(float d) { return __float_as_int(d); }
 // Two passes of 8 octets are kept in flight (one for a last group of <= 8).
 // lst and lsd hold 64 entries; every index stays below 64. Returns after lsd
 // is visible.
-template <int DT, int CPL>
-__device__ __forceinline__ void batch_dist(const RowSet& rs, const uint4 (&av)[CPL], uint32_t a_sq,
-                                           const uint32_t* lst, float* lsd, uint32_t n, uint32_t grp,
-                                           uint32_t sub) {
+// load(id, active, v) fetches the lane's chunks of row `id` (load_row).
+template <int DT, int CPL, typename Load>
+__device__ __forceinline__ void batch_dist_by(const RowSet& rs, const Load& load, const uint4 (&av)[CPL], uint32_t a_sq,
+                                              const uint32_t* lst, float* lsd, uint32_t n, uint32_t grp,
+                                              uint32_t sub) {
   uint32_t p = 0;
   for (; p + 8 < n; p += 16) {
     const uint32_t k0 = p + grp, k1 = p + 8 + grp;
     const bool a0 = k0 < n, a1 = k1 < n;
     const uint32_t id0 = lst[k0], id1 = lst[k1];  // k0, k1 < 64: in bounds; inactive ids are not loaded
     uint4 b0[CPL], b1[CPL];
-    load_row<CPL>(rs, id0, a0, sub, b0);
-    load_row<CPL>(rs, id1, a1, sub, b1);
+    load(id0, a0, b0);
+    load(id1, a1, b1);
     const float d0 = octet_finish<DT, CPL>(rs, sub, av, b0, a_sq);
     const float d1 = octet_finish<DT, CPL>(rs, sub, av, b1, a_sq);
     // every lane writes its octet's distance of one of the two passes: equal
@@ -372,10 +407,18 @@ __device__ __forceinline__ void batch_dist(const RowSet& rs, const uint4 (&av)[C
     const uint32_t k0 = p + grp;
     const bool a0 = k0 < n;
     uint4 b0[CPL];
-    load_row<CPL>(rs, lst[k0], a0, sub, b0);
+    load(lst[k0], a0, b0);
     lsd[k0] = octet_finish<DT, CPL>(rs, sub, av, b0, a_sq);
   }
   wave_sync();
+}
+template <int DT, int CPL>
+__device__ __forceinline__ void batch_dist(const RowSet& rs, const uint4 (&av)[CPL], uint32_t a_sq,
+                                           const uint32_t* lst, float* lsd, uint32_t n, uint32_t grp,
+                                           uint32_t sub) {
+  batch_dist_by<DT, CPL>(
+      rs, [&](uint32_t id, bool active, uint4(&v)[CPL]) { load_row<CPL>(rs, id, active, sub, v); }, av, a_sq, lst, lsd,
+      n, grp, sub);
 }
 template <int DT, int CPL>
 __device__ __forceinline__ void batch_dist(const RowSet& rs, const uint4 (&av)[CPL], const uint32_t* lst,

@@ -88,3 +88,33 @@ def test_wide_code_rows(kind, dim, L, centers):
     assert np.array_equal(d.cpu().numpy().view(np.uint32), od)
     assert np.array_equal(g.cpu().numpy().view(np.uint32), og)
     assert (D.last_kernel_profile()["bound_checks"] > 0) == (dim <= 240)
+
+
+# base rows read packed: row lengths that leave a last chunk of 1 to 15 bytes,
+# rows that start at any byte, both sides of the rule (one query and many),
+# pools of 1 and 2 slots per lane and beyond, and rows too wide for it
+@pytest.mark.parametrize("kind,dim", [("u8", 1), ("u8", 15), ("u8", 17), ("u8", 99), ("u8", 131), ("u8", 509), ("u8", 513),
+                                      ("f16", 7), ("f16", 101), ("f16", 130), ("f32", 3), ("f32", 33), ("f32", 97),
+                                      ("f32", 127), ("f32", 130)])
+@pytest.mark.parametrize("shift,nq,L", [(0, 1, 10), (1, 2, 65), (5, 1, 129), (0, 200, 20)])
+def test_packed_base_rows(kind, dim, shift, nq, L):
+    import torch
+    n, R, k = 5000, 16, 10
+    x = rows(kind, n, dim, seed=dim)
+    qs = rows(kind, nq, dim, seed=dim + 1)
+    if kind != "u8":
+        x[17] = np.inf
+    rng = np.random.default_rng(dim)
+    graph = rng.integers(0, n, (n, R), dtype=np.uint32)
+    degree = rng.integers(0, R + 1, n).astype(np.uint32)
+    starts = np.array([7], np.uint32)
+    want = O.query_search(x, graph, degree, starts, qs, k, L)
+    shift -= shift % x.itemsize if kind != "u8" else 0  # elements stay aligned
+    flat = torch.zeros(x.nbytes + 64, dtype=torch.uint8, device="cuda")
+    flat[shift:shift + x.nbytes] = torch.from_numpy(x.reshape(-1).view(np.uint8)).cuda()
+    g, d = torch.from_numpy(graph.view(np.int32)).cuda(), torch.from_numpy(degree.view(np.int32)).cuda()
+    got = D.search_resident(flat.data_ptr() + shift, D.dtype_code(x), n, dim, g.data_ptr(), d.data_ptr(), R, starts, qs,
+                            k, L)
+    for a in (got, D.search(x, graph, degree, starts, qs, k, L)):
+        assert np.array_equal(a[0], want[0])
+        assert np.array_equal(a[1].view(np.uint32), want[1].view(np.uint32))
