@@ -105,10 +105,12 @@ inline int with_dt_cpl(int kind, int cpl, Fn&& fn) {
 // build's scratch array). While an ArenaScope is alive on a thread, every
 // DevBuf::alloc on that thread takes its bytes from the arena instead of
 // hipMalloc, and nothing is freed: the arena's contents end with the scope.
+// With `spill`, what does not fit is allocated on its own instead of refused.
 struct Arena {
   char* base = nullptr;
   size_t cap = 0;
   size_t used = 0;
+  bool spill = false;
 };
 inline thread_local Arena* tl_arena = nullptr;
 struct ArenaScope {
@@ -118,6 +120,8 @@ struct ArenaScope {
   ArenaScope(const ArenaScope&) = delete;
   ArenaScope& operator=(const ArenaScope&) = delete;
 };
+
+inline bool drop_idle_slabs();  // frees what CallPool keeps on this GPU; whether there was any
 
 struct DevBuf {
   void* p = nullptr;
@@ -139,17 +143,23 @@ struct DevBuf {
     if (b == 0) return 0;
     if (Arena* a = tl_arena) {
       const size_t off = (a->used + 255u) & ~(size_t)255u;
-      if (off > a->cap || b > a->cap - off) {
+      if (off <= a->cap && b <= a->cap - off) {
+        p = a->base + off;
+        a->used = off + b;
+        borrowed = true;
+        return 0;
+      }
+      if (!a->spill) {
         std::fprintf(stderr, "[dance_hip] scratch arena exhausted: %zu bytes requested, %zu of %zu in use\n", b,
                      a->used, a->cap);
         return -1;
       }
-      p = a->base + off;
-      a->used = off + b;
-      borrowed = true;
-      return 0;
     }
     hipError_t e = hipMalloc(&p, b);
+    if (e != hipSuccess && drop_idle_slabs()) {
+      (void)hipGetLastError();
+      e = hipMalloc(&p, b);
+    }
     if (e != hipSuccess) {
       std::fprintf(stderr, "[dance_hip] hipMalloc(%zu) failed: %s\n", b, hipGetErrorString(e));
       p = nullptr;
@@ -167,6 +177,180 @@ struct DevBuf {
     return static_cast<T*>(p);
   }
 };
+
+// ---------------------------------------------------------------------------
+// What a call borrows for its duration: a slab of device memory for all its
+// buffers, a stream, two timing events and a little pinned memory. A call
+// otherwise makes and frees 7 (query search) to 25 (build) device allocations,
+// each of which maps or unmaps memory, and a free waits for the device.
+// The calls of 16 to 10k queries take 0.15 ms less with it, a build of 100k x 96
+// 2.4 ms (58.3 -> 55.9).
+// Idle slabs are bounded by kKeepBytes over all GPUs, the oldest freed first,
+// and all of a GPU's are freed when an allocation on it fails; a call that
+// needs more than kLeaseBytes allocates for itself. A lease goes back only
+// after the call's work has completed (CallLease), so the next call, on
+// whatever thread, may write the slab at once.
+// ---------------------------------------------------------------------------
+constexpr size_t kKeepBytes = 512ull << 20;
+constexpr size_t kLeaseBytes = kKeepBytes;
+constexpr size_t kKeepStreams = 4;
+constexpr size_t kCallHostBytes = 16ull << 20;
+
+struct Slab {
+  void* p = nullptr;
+  size_t bytes = 0;
+  int dev = 0;
+};
+struct StreamSet {
+  hipStream_t s = nullptr;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  void* host = nullptr;  // kCallHostBytes of pinned memory, made on first use
+  int dev = 0;
+};
+
+class CallPool {
+ public:
+  static CallPool& get() {
+    static CallPool* pool = new CallPool;  // never destroyed: the runtime may be gone before a static's end
+    return *pool;
+  }
+  int take(size_t need, int dev, Slab* out) {
+    std::lock_guard<std::mutex> lk(mu_);
+    size_t best = idle_.size();
+    for (size_t i = 0; i < idle_.size(); ++i)
+      if (idle_[i].dev == dev && idle_[i].bytes >= need && (best == idle_.size() || idle_[i].bytes < idle_[best].bytes))
+        best = i;
+    if (best < idle_.size()) {
+      *out = idle_[best];
+      kept_ -= out->bytes;
+      idle_.erase(idle_.begin() + (ptrdiff_t)best);
+      return 0;
+    }
+    const size_t bytes = (need + kGrain - 1) / kGrain * kGrain;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      drop_locked(dev);
+      const hipError_t e = hipMalloc(&p, bytes);
+      if (e != hipSuccess) {
+        std::fprintf(stderr, "[dance_hip] hipMalloc(%zu) failed: %s\n", bytes, hipGetErrorString(e));
+        return -1;
+      }
+    }
+    *out = Slab{p, bytes, dev};
+    return 0;
+  }
+  void give(const Slab& s) {
+    std::lock_guard<std::mutex> lk(mu_);
+    idle_.push_back(s);
+    kept_ += s.bytes;
+    while (kept_ > kKeepBytes) free_locked(0);
+  }
+  // Frees the idle slabs of a GPU (an allocation on it failed).
+  bool drop(int dev) {
+    std::lock_guard<std::mutex> lk(mu_);
+    return drop_locked(dev);
+  }
+  int take_stream(int dev, StreamSet* out) {
+    {
+      std::lock_guard<std::mutex> lk(mu_);
+      for (size_t i = 0; i < streams_.size(); ++i)
+        if (streams_[i].dev == dev) {
+          *out = streams_[i];
+          streams_.erase(streams_.begin() + (ptrdiff_t)i);
+          return 0;
+        }
+    }
+    out->dev = dev;
+    DHIP(hipStreamCreate(&out->s));
+    DHIP(hipEventCreate(&out->e0));
+    DHIP(hipEventCreate(&out->e1));
+    return 0;
+  }
+  void give_stream(const StreamSet& st) {
+    if (!st.s) return;
+    if (st.e1) {
+      std::lock_guard<std::mutex> lk(mu_);
+      if (streams_.size() < kKeepStreams) {
+        streams_.push_back(st);
+        return;
+      }
+    }
+    if (st.e0) (void)hipEventDestroy(st.e0);
+    if (st.e1) (void)hipEventDestroy(st.e1);
+    if (st.host) (void)hipHostFree(st.host);
+    (void)hipStreamDestroy(st.s);
+  }
+
+ private:
+  static constexpr size_t kGrain = 2ull << 20;
+  void free_locked(size_t i) {
+    kept_ -= idle_[i].bytes;
+    (void)hipFree(idle_[i].p);
+    idle_.erase(idle_.begin() + (ptrdiff_t)i);
+  }
+  bool drop_locked(int dev) {
+    bool any = false;
+    for (size_t i = idle_.size(); i-- > 0;)
+      if (idle_[i].dev == dev) {
+        free_locked(i);
+        any = true;
+      }
+    return any;
+  }
+  std::mutex mu_;
+  std::vector<Slab> idle_;  // oldest first
+  size_t kept_ = 0;
+  std::vector<StreamSet> streams_;
+};
+
+inline bool drop_idle_slabs() {
+  int dev = 0;
+  return hipGetDevice(&dev) == hipSuccess && CallPool::get().drop(dev);
+}
+
+// One call's lease, declared before every buffer that uses it. From open() on
+// the thread's DevBuf allocations come from the slab (beyond it, or with no
+// slab, from hipMalloc). done() says that the caller has waited for all its
+// work; otherwise (an error return) the end of the lease waits for the device.
+struct CallLease {
+  Arena arena;
+  Slab slab;
+  StreamSet set;
+  Arena* prev = nullptr;
+  bool opened = false, finished = false;
+  CallLease() = default;
+  CallLease(const CallLease&) = delete;
+  CallLease& operator=(const CallLease&) = delete;
+  int open(size_t need) {
+    int dev = 0;
+    DHIP(hipGetDevice(&dev));
+    opened = true;
+    prev = tl_arena;
+    DCHECK(CallPool::get().take_stream(dev, &set));
+    if (need <= kLeaseBytes) {
+      DCHECK(CallPool::get().take(need, dev, &slab));
+      arena = Arena{static_cast<char*>(slab.p), slab.bytes, 0, true};
+      tl_arena = &arena;
+    }
+    return 0;
+  }
+  hipStream_t stream() const { return set.s; }
+  int host(char** out) {
+    if (!set.host) DHIP(hipHostMalloc(&set.host, kCallHostBytes, hipHostMallocPortable));
+    *out = static_cast<char*>(set.host);
+    return 0;
+  }
+  void done() { finished = true; }
+  ~CallLease() {
+    if (!opened) return;
+    tl_arena = prev;
+    if (!finished) (void)hipDeviceSynchronize();
+    if (slab.p) CallPool::get().give(slab);
+    CallPool::get().give_stream(set);
+  }
+};
+inline size_t arena_bytes(size_t b) { return (b + 255u) & ~(size_t)255u; }
 
 // ---------------------------------------------------------------------------
 // Scan / sort drivers.
@@ -265,6 +449,28 @@ static __global__ void k_f32_to_f16_rows(const float* __restrict__ src, uint32_t
   if (i >= (size_t)N * dim) return;
   const size_t r = i / dim, c = i % dim;
   dst[r * dst_stride_elems + c] = (_Float16)src[i];  // round to nearest even
+}
+
+// Packed rows of row_bytes -> rows of nch 16-byte chunks padded with zeros, one
+// chunk per thread; nothing past a row's end is read. Bound by the copy itself;
+// one pass instead of a fill and a strided copy.
+static __global__ void k_pad_rows(const uint8_t* __restrict__ src, uint32_t row_bytes, uint32_t N, uint32_t nch,
+                                  uint4* __restrict__ dst) {
+  const uint64_t i = (uint64_t)grid_block() * blockDim.x + threadIdx.x;
+  if (i >= (uint64_t)N * nch) return;
+  const uint32_t r = (uint32_t)(i / nch), c = (uint32_t)(i % nch), off = 16u * c;
+  const uint8_t* p = src + (size_t)r * row_bytes + off;
+  uint4 v = make_uint4(0u, 0u, 0u, 0u);
+  if (off + 16u <= row_bytes) {
+    __builtin_memcpy(&v, p, 16);
+  } else if (off < row_bytes) {
+    uint32_t w[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (uint32_t b = 0; b < 15; ++b)
+      if (off + b < row_bytes) w[b >> 2] |= (uint32_t)p[b] << (8u * (b & 3u));
+    v = make_uint4(w[0], w[1], w[2], w[3]);
+  }
+  dst[i] = v;
 }
 
 // Nearest pivots of uint8 rows from MFMA tiles (k_cells_mfma): keys to `cell`,
@@ -370,6 +576,12 @@ inline size_t row_layout(Rows& out, int store_dtype, uint32_t N, uint32_t dim) {
   return (size_t)nch * 16;
 }
 
+// Upper bound of what setup_rows allocates for rows in host memory.
+inline size_t host_rows_bytes(int src_dtype, int store_dtype, uint32_t N, uint32_t dim) {
+  Rows r;
+  return arena_bytes(row_layout(r, store_dtype, N, dim) * N) + arena_bytes((size_t)dim * elem_bytes(src_dtype) * N);
+}
+
 inline int setup_rows(Rows& out, const void* src, bool src_on_device, int src_dtype, int store_dtype, uint32_t N,
                       uint32_t dim, hipStream_t s) {
   const size_t stride = row_layout(out, store_dtype, N, dim);
@@ -397,9 +609,11 @@ inline int setup_rows(Rows& out, const void* src, bool src_on_device, int src_dt
         DCHECK(copy_pageable(tmp.p, src, row_bytes * N, hipMemcpyHostToDevice));
         dsrc = tmp.p;
       }
-      DHIP(hipMemsetAsync(out.owned.p, 0, stride * N, s));
-      DHIP(hipMemcpy2DAsync(out.owned.p, stride, dsrc, row_bytes, row_bytes, N, hipMemcpyDeviceToDevice, s));
-      DHIP(hipStreamSynchronize(s));  // tmp is freed on return
+      hipLaunchKernelGGL(k_pad_rows, grid_dims(((uint64_t)N * out.rs.nch + 255) / 256, 256), dim3(256), 0, s,
+                         static_cast<const uint8_t*>(dsrc), (uint32_t)row_bytes, N, out.rs.nch,
+                         out.owned.as<uint4>());
+      DHIP(hipGetLastError());
+      if (!src_on_device) DHIP(hipStreamSynchronize(s));  // tmp is freed on return
     }
   } else {
     // fp32 input stored as fp16 (FAST_SMALL): upload, convert on device.
@@ -415,7 +629,7 @@ inline int setup_rows(Rows& out, const void* src, bool src_on_device, int src_dt
     hipLaunchKernelGGL(k_f32_to_f16_rows, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s,
                        static_cast<const float*>(fsrc), N, dim, out.owned.as<_Float16>(), (uint32_t)(stride / 2));
     DHIP(hipGetLastError());
-    DHIP(hipStreamSynchronize(s));
+    if (!src_on_device) DHIP(hipStreamSynchronize(s));
   }
   out.rs.rows = out.owned.as<const uint4>();
   return 0;

@@ -9,6 +9,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cstring>
 #include <mutex>
 
 #include "../../include/dance_hip.h"
@@ -23,6 +24,8 @@ using namespace qs;
 std::mutex g_qmu;
 DanceSearchStats g_qstats{};
 
+constexpr size_t kCtrBytes = 3 * 8;           // distances, expansions, capped queries
+constexpr size_t kSendBytes = 512ull << 10;  // least bytes of an input copy that is followed by another
 constexpr uint32_t kMaxL = 1024;  // 16 slots per lane
 constexpr uint64_t kGathersPerL = 24;  // rows a query gathers per list entry
 // Widest rows and lists that have a kernel for packed rows.
@@ -80,16 +83,24 @@ int run_search(const SearchIn& in) {
   }
   std::lock_guard<std::mutex> lk(g_qmu);
   g_qstats = DanceSearchStats{};
-  hipStream_t s = nullptr;
-  DHIP(hipStreamCreate(&s));
-  struct SG {
-    hipStream_t s;
-    ~SG() {
-      if (s) (void)hipStreamDestroy(s);
-    }
-  } sg{s};
-  Rows base, qr;
   const size_t row_bytes = (size_t)in.dim * elem_bytes(in.dtype);
+  // The call's small inputs and its results lie in one block, in copy order:
+  // starts, their offsets, query labels, queries, counters, ids, distances.
+  const size_t b_starts = arena_bytes((size_t)in.nstarts * 4);
+  const size_t b_off = in.start_off ? arena_bytes((size_t)(in.nq + 1) * 4) : 0;
+  const size_t b_qlab = filt ? arena_bytes((size_t)in.nq * 4) : 0;
+  const size_t b_q = arena_bytes(row_bytes * in.nq);
+  const size_t b_in = b_starts + b_off + b_qlab + b_q + arena_bytes(kCtrBytes);
+  const size_t b_res = arena_bytes((size_t)in.nq * in.k * 4);
+  const uint32_t ntotal = filt ? in.label_offsets[in.N] : 0u;
+  size_t need = b_in + 2 * b_res + host_rows_bytes(in.dtype, in.dtype, in.nq, in.dim) +
+                host_rows_bytes(in.dtype, in.dtype, in.N, in.dim);
+  if (!in.graph_on_device) need += arena_bytes((size_t)in.N * in.R * 4) + arena_bytes((size_t)in.N * 4);
+  if (filt) need += arena_bytes((size_t)(in.N + 1) * 4) + arena_bytes((size_t)std::max(1u, ntotal) * 4);
+  CallLease lease;
+  DCHECK(lease.open(need));
+  const hipStream_t s = lease.stream();
+  Rows base, qr;
   const size_t stride = row_layout(base, in.dtype, in.N, in.dim);
   const void* packed = in.data;  // the base rows in device memory, as the caller packed them
   DevBuf up;
@@ -114,13 +125,52 @@ int run_search(const SearchIn& in) {
     base.rs.rows = static_cast<const uint4*>(packed);
   else if (!in_place)
     DCHECK(setup_rows(base, packed, true, in.dtype, in.dtype, in.N, in.dim, s));
-  DCHECK(setup_rows(qr, in.queries, false, in.dtype, in.dtype, in.nq, in.dim, s));
   const int cpl = pick_cpl(base.rs.nch);
   if (cpl < 0) {
     std::fprintf(stderr, "[dance_search] dim=%u is beyond the supported row width\n", in.dim);
     return -1;
   }
-  DevBuf g, dg, st, soff, off, lab, qlab, oi, od, ctr;
+  DevBuf blk, g, dg, off, lab;
+  DCHECK(blk.alloc(b_in + 2 * b_res));
+  char* const d_in = blk.as<char>();
+  char* const d_ctr = d_in + b_in - arena_bytes(kCtrBytes);
+  // Pinned halves of the lease: inputs, results. A copy from or to pageable
+  // memory moves 8 GB/s and takes 10 us or more; inputs are sent while the rest
+  // is still written. With the leased memory and stream: 16 queries of L 50 over
+  // 200k x 96 0.40 -> 0.25 ms (kernel 0.22), 10k of L 100 over 1M x 96 2.85 ->
+  // 2.69 ms (kernel 2.42), 1k filtered over 100k 0.87 -> 0.66 ms (kernel 0.50).
+  char* pin = nullptr;
+  DCHECK(lease.host(&pin));
+  if (b_in <= kCallHostBytes / 2) {
+    size_t sent = 0, at = 0;
+    auto put = [&](const void* src, size_t bytes, size_t room) -> int {
+      for (size_t o = 0; o < bytes; o += kSendBytes) {  // the first pieces travel while the next are written
+        const size_t n = std::min(kSendBytes, bytes - o);
+        std::memcpy(pin + at + o, static_cast<const char*>(src) + o, n);
+        if (at + o + n - sent >= kSendBytes) {
+          DHIP(hipMemcpyAsync(d_in + sent, pin + sent, at + o + n - sent, hipMemcpyHostToDevice, s));
+          sent = at + o + n;
+        }
+      }
+      at += room;
+      return 0;
+    };
+    DCHECK(put(in.starts, (size_t)in.nstarts * 4, b_starts));
+    if (in.start_off) DCHECK(put(in.start_off, (size_t)(in.nq + 1) * 4, b_off));
+    if (filt) DCHECK(put(in.query_labels, (size_t)in.nq * 4, b_qlab));
+    DCHECK(put(in.queries, row_bytes * in.nq, b_q));
+    std::memset(pin + at, 0, kCtrBytes);
+    DHIP(hipMemcpyAsync(d_in + sent, pin + sent, at + kCtrBytes - sent, hipMemcpyHostToDevice, s));
+  } else {
+    if (in.nstarts) DHIP(hipMemcpyAsync(d_in, in.starts, (size_t)in.nstarts * 4, hipMemcpyHostToDevice, s));
+    if (in.start_off)
+      DHIP(hipMemcpyAsync(d_in + b_starts, in.start_off, (size_t)(in.nq + 1) * 4, hipMemcpyHostToDevice, s));
+    if (filt)
+      DHIP(hipMemcpyAsync(d_in + b_starts + b_off, in.query_labels, (size_t)in.nq * 4, hipMemcpyHostToDevice, s));
+    DCHECK(copy_pageable(d_in + b_starts + b_off + b_qlab, in.queries, row_bytes * in.nq, hipMemcpyHostToDevice));
+    DHIP(hipMemsetAsync(d_ctr, 0, kCtrBytes, s));
+  }
+  DCHECK(setup_rows(qr, d_in + b_starts + b_off + b_qlab, true, in.dtype, in.dtype, in.nq, in.dim, s));
   const uint32_t* dgraph = in.graph;
   const uint32_t* ddeg = in.degree;
   if (!in.graph_on_device) {
@@ -131,34 +181,21 @@ int run_search(const SearchIn& in) {
     dgraph = g.as<uint32_t>();
     ddeg = dg.as<uint32_t>();
   }
-  DCHECK(st.alloc((size_t)std::max(1u, in.nstarts) * 4));
-  if (in.nstarts) DHIP(hipMemcpyAsync(st.p, in.starts, (size_t)in.nstarts * 4, hipMemcpyHostToDevice, s));
-  if (in.start_off) {
-    DCHECK(soff.alloc((size_t)(in.nq + 1) * 4));
-    DHIP(hipMemcpyAsync(soff.p, in.start_off, (size_t)(in.nq + 1) * 4, hipMemcpyHostToDevice, s));
-  }
   if (filt) {
-    const uint32_t total = in.label_offsets[in.N];
     DCHECK(off.alloc((size_t)(in.N + 1) * 4));
-    DCHECK(lab.alloc((size_t)std::max(1u, total) * 4));
-    DCHECK(qlab.alloc((size_t)in.nq * 4));
+    DCHECK(lab.alloc((size_t)std::max(1u, ntotal) * 4));
     DHIP(hipMemcpyAsync(off.p, in.label_offsets, (size_t)(in.N + 1) * 4, hipMemcpyHostToDevice, s));
-    if (total) DHIP(hipMemcpyAsync(lab.p, in.labels, (size_t)total * 4, hipMemcpyHostToDevice, s));
-    DHIP(hipMemcpyAsync(qlab.p, in.query_labels, (size_t)in.nq * 4, hipMemcpyHostToDevice, s));
+    if (ntotal) DHIP(hipMemcpyAsync(lab.p, in.labels, (size_t)ntotal * 4, hipMemcpyHostToDevice, s));
   }
-  DCHECK(oi.alloc((size_t)in.nq * in.k * 4));
-  DCHECK(od.alloc((size_t)in.nq * in.k * 4));
-  DCHECK(ctr.alloc(3 * 8));
-  DHIP(hipMemsetAsync(ctr.p, 0, 3 * 8, s));
-  QArgs a{in.N, in.R, dgraph, ddeg, st.as<uint32_t>(), in.nstarts,
-          in.start_off ? soff.as<uint32_t>() : nullptr, in.nq, in.k, in.L, 16u * in.L + 1024u,
-          filt ? off.as<uint32_t>() : nullptr, filt ? lab.as<uint32_t>() : nullptr,
-          filt ? qlab.as<uint32_t>() : nullptr, oi.as<uint32_t>(), od.as<float>(),
-          ctr.as<unsigned long long>(), static_cast<const uint8_t*>(packed), (uint32_t)row_bytes};
-  hipEvent_t e0, e1;
-  DHIP(hipEventCreate(&e0));
-  DHIP(hipEventCreate(&e1));
-  DHIP(hipEventRecord(e0, s));
+  char* const d_ids = d_in + b_in;
+  char* const d_dist = d_ids + b_res;
+  QArgs a{in.N, in.R, dgraph, ddeg, reinterpret_cast<const uint32_t*>(d_in), in.nstarts,
+          in.start_off ? reinterpret_cast<const uint32_t*>(d_in + b_starts) : nullptr, in.nq, in.k, in.L,
+          16u * in.L + 1024u, filt ? off.as<uint32_t>() : nullptr, filt ? lab.as<uint32_t>() : nullptr,
+          filt ? reinterpret_cast<const uint32_t*>(d_in + b_starts + b_off) : nullptr,
+          reinterpret_cast<uint32_t*>(d_ids), reinterpret_cast<float*>(d_dist),
+          reinterpret_cast<unsigned long long*>(d_ctr), static_cast<const uint8_t*>(packed), (uint32_t)row_bytes};
+  DHIP(hipEventRecord(lease.set.e0, s));
   const uint32_t grid = (in.nq + kWaves - 1) / kWaves;
   const size_t lds = (size_t)kWaves * kLds * 4;
   DCHECK(with_dt_cpl(base.kind(), cpl, [&](auto dt, auto c) {
@@ -186,16 +223,26 @@ int run_search(const SearchIn& in) {
     DHIP(hipGetLastError());
     return 0;
   }));
-  DHIP(hipEventRecord(e1, s));
-  DHIP(hipMemcpyAsync(in.ids_out, oi.p, (size_t)in.nq * in.k * 4, hipMemcpyDeviceToHost, s));
-  DHIP(hipMemcpyAsync(in.d_out, od.p, (size_t)in.nq * in.k * 4, hipMemcpyDeviceToHost, s));
-  unsigned long long c3[3];
-  DHIP(hipMemcpyAsync(c3, ctr.p, sizeof(c3), hipMemcpyDeviceToHost, s));
-  DHIP(hipStreamSynchronize(s));
+  DHIP(hipEventRecord(lease.set.e1, s));
+  unsigned long long c3[kCtrBytes / 8];
+  const size_t res_bytes = (size_t)in.nq * in.k * 4;
+  const size_t b_out = arena_bytes(kCtrBytes) + 2 * b_res;
+  if (b_out <= kCallHostBytes / 2) {
+    char* const out = pin + kCallHostBytes / 2;
+    DHIP(hipMemcpyAsync(out, d_ctr, b_out, hipMemcpyDeviceToHost, s));
+    DHIP(hipStreamSynchronize(s));
+    std::memcpy(c3, out, sizeof(c3));
+    std::memcpy(in.ids_out, out + (d_ids - d_ctr), res_bytes);
+    std::memcpy(in.d_out, out + (d_dist - d_ctr), res_bytes);
+  } else {
+    DHIP(hipMemcpyAsync(in.ids_out, d_ids, res_bytes, hipMemcpyDeviceToHost, s));
+    DHIP(hipMemcpyAsync(in.d_out, d_dist, res_bytes, hipMemcpyDeviceToHost, s));
+    DHIP(hipMemcpyAsync(c3, d_ctr, sizeof(c3), hipMemcpyDeviceToHost, s));
+    DHIP(hipStreamSynchronize(s));
+  }
+  lease.done();
   float ms = 0.f;
-  (void)hipEventElapsedTime(&ms, e0, e1);
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
+  (void)hipEventElapsedTime(&ms, lease.set.e0, lease.set.e1);
   g_qstats.kernel_ms = ms;
   g_qstats.distances = c3[0];
   g_qstats.expansions = c3[1];

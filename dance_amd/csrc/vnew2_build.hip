@@ -53,6 +53,9 @@ static_assert(offsetof(GPUVamanaStats, distance_computations) == 56, "GPUVamanaS
 static_assert(offsetof(GPUVamanaStats, reverse_csr_seconds) == 104, "GPUVamanaStats layout");
 static_assert(offsetof(GPUVamanaStats, selective_active_nodes) == 112, "GPUVamanaStats layout");
 
+static size_t resident_build_bytes(const void* d_data, int dtype, int store, uint32_t N, uint32_t dim, uint32_t R,
+                                   uint32_t C, bool rows_ready = false, bool wide_bound = true);
+
 namespace dance {
 
 // ---------------------------------------------------------------------------
@@ -1012,6 +1015,9 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   return 0;
 }
 
+// What a timed build allocates beyond resident_build_bytes: the counters after each iteration.
+constexpr size_t kTimedBytes = sizeof(VCounters) * kMaxIters + 256;
+
 template <typename HostT>
 static int build_host(const HostT* h_data, int src_dtype, uint32_t N, uint32_t dim, uint32_t R, uint32_t L,
                       uint32_t C, uint32_t STEPS, uint32_t* h_graph, uint32_t* h_degree, void** keep_data,
@@ -1033,14 +1039,12 @@ static int build_host(const HostT* h_data, int src_dtype, uint32_t N, uint32_t d
                 store == DANCE_F16 ? "float16" : (src_dtype == DANCE_U8 ? "uint8" : "float"), N, dim, R, L,
                 C, std::min(STEPS, L), (double)kAlpha, vamana_iters(), prof.name, prof.fp16 ? 1u : 0u);
   DCHECK(check_width(dim, store));
-  hipStream_t s = nullptr;
-  DHIP(hipStreamCreate(&s));
-  struct StreamGuard {
-    hipStream_t s;
-    ~StreamGuard() {
-      if (s) (void)hipStreamDestroy(s);
-    }
-  } sg{s};
+  // The hand-off's buffers outlive the call, so none of it is leased.
+  CallLease lease;
+  DCHECK(lease.open(handoff ? SIZE_MAX
+                            : resident_build_bytes(nullptr, src_dtype, store, N, dim, R, C) + kTimedBytes +
+                                  host_rows_bytes(src_dtype, store, N, dim) + ((size_t)N * R + N) * 4 + 512));
+  hipStream_t s = lease.stream();
   GPUVamanaStats stats{};
   const double th = now_sec();
   Rows rows;
@@ -1071,6 +1075,7 @@ static int build_host(const HostT* h_data, int src_dtype, uint32_t N, uint32_t d
     DCHECK(copy_pageable(h_graph, st.cur.p, (size_t)N * R * 4, hipMemcpyDeviceToHost));
     DCHECK(copy_pageable(h_degree, st.deg_cur.p, (size_t)N * 4, hipMemcpyDeviceToHost));
   }
+  lease.done();
   stats.d2h_seconds = now_sec() - td;
   stats.gpu_build_seconds = now_sec() - t0;
   if (builder == Builder::v8) {
@@ -1253,7 +1258,7 @@ static int scratch_base(void** out) {
 // same buffers run_build, setup_rows and the radix sort allocate, each rounded
 // up to the arena's 256-byte alignment.
 static size_t resident_build_bytes(const void* d_data, int dtype, int store, uint32_t N, uint32_t dim, uint32_t R,
-                                   uint32_t C, bool rows_ready = false, bool wide_bound = true) {
+                                   uint32_t C, bool rows_ready, bool wide_bound) {
   size_t total = 0;
   auto add = [&](size_t b) { total += (b + 255u) & ~(size_t)255u; };
   const size_t row_bytes = (size_t)dim * elem_bytes(store);
@@ -1279,7 +1284,7 @@ static size_t resident_build_bytes(const void* d_data, int dtype, int store, uin
     add(items * 4);                 // snap_sorted
   }
   add(sizeof(VCounters) * kCtrStripes);
-  add(sizeof(VCounters));           // summed counters (the prune bound's choice for iteration 1)
+  add(sizeof(VCounters));           // summed counters (the bounds' choices)
   add(kMedoidCandidates * 4);       // scores
   add(kMedoidCandidates * 4);       // cands
   const bool wide = wide_bound && store != DANCE_U8 && dim > q_max_dim(1) && dim <= q_max_dim(2);
@@ -1340,14 +1345,9 @@ static int resident_build(const void* d_data, int dtype, uint32_t N, uint32_t di
     arena = Arena{static_cast<char*>(base), kScratchBytes, 0};
   }
   ArenaScope scope(noalloc ? &arena : tl_arena);
-  hipStream_t s = nullptr;  // the null stream unless a stream of our own is made
-  if (!noalloc) DHIP(hipStreamCreate(&s));
-  struct StreamGuard {
-    hipStream_t s;
-    ~StreamGuard() {
-      if (s) (void)hipStreamDestroy(s);
-    }
-  } sg{s};
+  CallLease lease;
+  if (!noalloc) DCHECK(lease.open(resident_build_bytes(d_data, dtype, store, N, dim, R, C) + kTimedBytes));
+  hipStream_t s = lease.stream();  // the null stream of an allocation-free build
   Rows rows;
   DCHECK(setup_rows(rows, d_data, true, dtype, store, N, dim, s));
   State st;
@@ -1362,6 +1362,7 @@ static int resident_build(const void* d_data, int dtype, uint32_t N, uint32_t di
   st.deg_cur.release();
   if (r != 0) return r;
   DHIP(hipStreamSynchronize(s));
+  lease.done();
   stats.gpu_build_seconds = now_sec() - t0;
   g_last_stats = stats;
   g_last_medoid = medoid;

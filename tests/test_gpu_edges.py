@@ -118,3 +118,46 @@ def test_packed_base_rows(kind, dim, shift, nq, L):
     for a in (got, D.search(x, graph, degree, starts, qs, k, L)):
         assert np.array_equal(a[0], want[0])
         assert np.array_equal(a[1].view(np.uint32), want[1].view(np.uint32))
+
+
+# calls of different sizes share leased memory, also from several threads at a
+# time and after a call that fails with its lease open
+def test_leased_memory_reuse():
+    import threading
+    import torch
+    dims, R, k = (33, 96, 200, 17), 16, 10
+    cases = []
+    for i, dim in enumerate(dims):
+        n = 1500 + 700 * i
+        x, qs = rows("f32", n, dim, seed=i), rows("f32", 5 + 60 * i, dim, seed=i + 9)
+        og, od, om = O.vnew2_build(x, R, 32, 24, 16)
+        cases.append((x, qs, og, od, O.query_search(x, og, od, om, qs, k, 40), om))
+    errors = []
+
+    def work(t):
+        try:
+            for r in range(6):
+                x, qs, og, od, want, om = cases[(r + t) % len(cases)]
+                n, dim = x.shape
+                ids, dd = D.search(x, og, od, om, qs, k, 40)
+                assert np.array_equal(ids, want[0]) and np.array_equal(dd, want[1])
+                if r % 2 == t % 2:
+                    xt = torch.from_numpy(x).cuda()
+                    g = torch.empty((n, R), dtype=torch.int32, device="cuda")
+                    d = torch.empty((n,), dtype=torch.int32, device="cuda")
+                    torch.cuda.synchronize()
+                    D.vamana_build_resident(xt.data_ptr(), D.dtype_code(x), n, dim, R, 32, 24, 16, g.data_ptr(),
+                                            d.data_ptr())
+                    assert np.array_equal(g.cpu().numpy().view(np.uint32), og)
+                wide = np.zeros((4, 3000), np.float32)  # beyond the supported row width
+                with pytest.raises(Exception):
+                    D.search(wide, np.zeros((4, 2), np.uint32), np.ones(4, np.uint32), 0, wide[:1], 1, 4)
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
