@@ -433,11 +433,14 @@ typedef int v4i_t __attribute__((ext_vector_type(4)));
 typedef int v16i_t __attribute__((ext_vector_type(16)));
 
 // v_writelane_b32: lane L of `words` takes the wave-uniform value v; the
-// other lanes keep theirs.
+// other lanes keep theirs. v may come straight from a vector compare, and an
+// SGPR that a vector instruction wrote can be read by another one two wait
+// states later at the earliest; the compiler does not look into the asm, so the
+// wait is part of it.
 template <uint32_t L>
 __device__ __forceinline__ uint32_t write_lane(uint32_t words, uint32_t v) {
   static_assert(L < 64u, "lane index");
-  asm volatile("v_writelane_b32 %0, %1, %2" : "+v"(words) : "s"(v), "n"(L));
+  asm volatile("s_nop 1\n\tv_writelane_b32 %0, %1, %2" : "+v"(words) : "s"(v), "n"(L));
   return words;
 }
 
