@@ -432,7 +432,6 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
   kp.backbone_ms = ms_between(e0, e1);
   double task_ms = 0, row_ms = 0, rev_ms = 0, csr_ms = 0;
   const size_t search_lds = (size_t)kWaves * kSearchLds * 4;
-  const size_t csr_lds = (size_t)kWaves * kCsrLds * 4;
   uint64_t reverse_edges = 0;
   const bool log = filtered_log();
   if (log) {
@@ -540,8 +539,8 @@ int run_filtered(const Rows& rows, const FParams& p, const uint32_t* h_off, cons
         long_done = E.mark(s2);
         if (!long_done) return -1;
       }
-      hipLaunchKernelGGL((k_csr<decltype(dt)::value, decltype(c)::value>), grid_xcd(N), dim3(kBlock), csr_lds,
-                         s, rows.rs, Gb, Ld, Cs);
+      hipLaunchKernelGGL((k_csr<decltype(dt)::value, decltype(c)::value>), grid_xcd(N), dim3(kBlock),
+                         (size_t)kWaves * csr_lds(decltype(dt)::value) * 4, s, rows.rs, Gb, Ld, Cs);
       DHIP(hipGetLastError());
       if (long_done) DHIP(hipStreamWaitEvent(s, long_done, 0));
       if (hub_done) DHIP(hipStreamWaitEvent(s, hub_done, 0));

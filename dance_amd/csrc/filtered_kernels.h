@@ -39,8 +39,14 @@ constexpr uint32_t kCsrRegMax = 64u * kCsrSlots;
 constexpr uint32_t kRandomAttempts = 1u << 20;
 // LDS words per wave: visited cache + one distance batch (ids, distances).
 constexpr uint32_t kSearchLds = kVis + 128u;
-// LDS words per wave of k_csr: forward row + one distance batch.
-constexpr uint32_t kCsrLds = 64u + 128u;
+// LDS words per wave of prune_gram: 128 entries in rank order (ids, distances,
+// squared norms, 4 mask words).
+constexpr uint32_t kGramCap = 128u;
+constexpr uint32_t kGramLds = 7u * kGramCap;
+static_assert(kGramLds <= kSearchLds, "k_row prunes in its search's LDS");
+// LDS words per wave of k_csr: forward row + one distance batch, then the
+// prune's.
+constexpr uint32_t csr_lds(int dt) { return dt == DANCE_U8 ? kGramLds : 64u + 128u; }
 // Candidate lists longer than kCsrRegMax are pruned by k_csr_long, one
 // workgroup of kLongWaves waves per row.
 constexpr uint32_t kLongWaves = 16;
@@ -519,6 +525,156 @@ __device__ __forceinline__ uint32_t prune_regs(const RowSet& rs, const Labels& L
 }
 
 
+// prune_regs for uint8 rows and at most kGramCap entries: the same selection
+// from ranks and masks. Removal never changes a distance, so the entries are
+// ranked once by (distance, id, index), and a round takes the lowest rank left.
+// Every pair's distance comes from int8 MFMA Gram tiles (bytes shifted by -128;
+// 32-bit integers, so each is the integer of the octet sum, converted the same
+// way); bit j of pm[4 i ..] = rank i would remove rank j. A round then costs a
+// few mask operations: it removes from what is left the entries of that word
+// that the selected row covers. uint8 distances are finite, so every entry that
+// is not removed can be selected. A round of prune_regs waits for three
+// reductions and for the selected row and its candidates' rows in turn; the
+// tiles gather each row once, in parallel. 250k x 192, about 90 candidates a row,
+// three rounds: k_csr 26.2 -> 20.3 ms, k_row 70.3 -> 63.2 ms.
+template <int CPL, int E>
+__device__ __forceinline__ uint32_t prune_gram(const RowSet& rs, const Labels& L, uint32_t row, uint32_t R,
+                                               float alpha, const uint32_t (&id)[E], const float (&d)[E],
+                                               uint32_t rem, uint32_t* lds, uint32_t lane, uint32_t& outv,
+                                               uint32_t& ndist) {
+  uint32_t* rid = lds;                                    // rank -> id
+  float* rd = reinterpret_cast<float*>(lds + kGramCap);   // rank -> distance
+  int* nrm = reinterpret_cast<int*>(lds + 2 * kGramCap);  // rank -> |row'|^2
+  uint32_t* pm = lds + 3 * kGramCap;
+  wave_sync();
+  // 1. the entries side by side, then ranked: a lane holds lane and lane + 64
+  uint32_t n = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const bool live = !((rem >> e) & 1u);
+    const uint64_t m = wballot(live);
+    if (live) {
+      rid[n + mbcnt64(m)] = id[e];
+      rd[n + mbcnt64(m)] = d[e];
+    }
+    n += popc64(m);
+  }
+  wave_sync();
+  uint32_t myid[2], myrank[2] = {0u, 0u};
+  int mykey[2];
+  float mydist[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    myid[h] = rid[lane + 64u * (uint32_t)h];
+    mydist[h] = rd[lane + 64u * (uint32_t)h];
+    mykey[h] = fkey(mydist[h]);
+  }
+  wave_sync();
+  for (uint32_t k = 0; k < min(n, 64u); ++k) {
+    const uint32_t ik = (uint32_t)__builtin_amdgcn_readlane((int)myid[0], (int)k);
+    const int kk = __builtin_amdgcn_readlane(mykey[0], (int)k);
+    myrank[0] += kk < mykey[0] || (kk == mykey[0] && (ik < myid[0] || (ik == myid[0] && k < lane))) ? 1u : 0u;
+    myrank[1] += kk < mykey[1] || (kk == mykey[1] && ik <= myid[1]) ? 1u : 0u;
+  }
+  for (uint32_t k = 64; k < n; ++k) {
+    const uint32_t ik = (uint32_t)__builtin_amdgcn_readlane((int)myid[1], (int)(k - 64u));
+    const int kk = __builtin_amdgcn_readlane(mykey[1], (int)(k - 64u));
+    myrank[0] += kk < mykey[0] || (kk == mykey[0] && ik < myid[0]) ? 1u : 0u;
+    myrank[1] += kk < mykey[1] || (kk == mykey[1] && (ik < myid[1] || (ik == myid[1] && k - 64u < lane))) ? 1u : 0u;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    if (lane + 64u * (uint32_t)h < n) {
+      rid[myrank[h]] = myid[h];
+      rd[myrank[h]] = mydist[h];
+    }
+  wave_sync();
+  // 2. the Gram tiles of ranks [32 ti, ..) x [32 tj, ..), tj >= ti
+  constexpr uint32_t S = 4u * CPL;  // K-steps of 32 bytes over the padded row
+  const uint32_t nt = (n + 31u) >> 5, jl = lane & 31u, ih = 4u * (lane >> 5);
+  // Ranks past the last take its row: their bits are masked, and the loads of
+  // a tile stay free of branches, in flight together.
+  for (uint32_t t = 0; t < nt; ++t) {
+    const uint32_t me = rid[min(t * 32u + jl, n - 1u)];
+    int part = 0;
+#pragma unroll
+    for (uint32_t st = 0; st < S; ++st) part = i8_sq4(u8_frag(rs, me, st, lane), part);
+    // lanes l and l + 32 hold the two halves of row t * 32 + l % 32
+    const int both = part + __shfl_xor(part, 32);
+    if (lane < 32u) nrm[t * 32u + lane] = both;
+  }
+  wave_sync();
+  for (uint32_t ti = 0; ti < nt; ++ti)
+    for (uint32_t tj = ti; tj < nt; ++tj) {
+      const uint32_t ia = rid[min(ti * 32u + jl, n - 1u)], ib = rid[min(tj * 32u + jl, n - 1u)];
+      v16i_t acc = {};
+#pragma unroll
+      for (uint32_t st = 0; st < S; ++st)
+        acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(u8_frag(rs, ia, st, lane), u8_frag(rs, ib, st, lane), acc, 0, 0, 0);
+      const uint32_t j = tj * 32u + jl;  // < kGramCap; rd and nrm past n are read, their bits masked
+      const int nj = nrm[j];
+      const float dj = rd[j];
+      const uint64_t jm = wballot(j < n);
+      uint32_t words = 0u;  // lane l < 32 collects the word of tile row l
+      static_for<0, 16>([&](auto vc) {
+        constexpr uint32_t v = decltype(vc)::value, ir = 8u * (v >> 2) + (v & 3u);
+        const uint32_t i = ti * 32u + ir + ih;
+        const float pd = u8_gram_dist(nrm[i], nj, acc[v]);
+        const uint64_t m = jm & wballot(i < j) & wballot(pd > 0.0f) & wballot(alpha * pd <= dj);
+        words = write_lane<ir>(words, (uint32_t)m);
+        words = write_lane<ir + 4u>(words, (uint32_t)(m >> 32));
+      });
+      if (lane < 32u) pm[4u * (ti * 32u + lane) + tj] = words;
+    }
+  wave_sync();
+  // 3. rounds. Words below the diagonal or past the last tile stay unset: they
+  // only meet ranks that have left.
+  const bool use_mask = L.off[row + 1] - L.off[row] <= kMaskLabels;
+  uint32_t r_id[2], r_msk[2] = {0u, 0u}, r_occ[2][4];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const uint32_t r = lane + 64u * (uint32_t)h;
+    r_id[h] = rid[r];
+    if (use_mask && r < n) r_msk[h] = row_mask(L, row, r_id[h]);
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) r_occ[h][q] = pm[4u * r + q];
+  }
+  auto rank_u = [&](uint32_t v0, uint32_t v1, uint32_t r) -> uint32_t {
+    return (uint32_t)__builtin_amdgcn_readlane((int)(r < 64u ? v0 : v1), (int)(r & 63u));
+  };
+  uint64_t live0 = n >= 64u ? ~0ull : (1ull << n) - 1ull;
+  uint64_t live1 = n >= 128u ? ~0ull : n > 64u ? (1ull << (n - 64u)) - 1ull : 0ull;
+  uint32_t sel = 0;
+  outv = DANCE_INV;
+  while (sel < R && (live0 | live1) != 0ull) {
+    const uint32_t r = live0 ? (uint32_t)ffs64(live0) : 64u + (uint32_t)ffs64(live1);
+    const uint32_t I = rank_u(r_id[0], r_id[1], r);
+    if (lane == sel) outv = I;
+    ++sel;
+    if (r < 64u)
+      live0 &= live0 - 1ull;
+    else
+      live1 &= live1 - 1ull;
+    bool c0, c1;
+    if (use_mask) {
+      const uint32_t ms = rank_u(r_msk[0], r_msk[1], r);
+      c0 = (r_msk[0] & ~ms) == 0u;
+      c1 = (r_msk[1] & ~ms) == 0u;
+    } else {
+      c0 = ((live0 >> lane) & 1ull) && covers(L, row, I, r_id[0]);
+      c1 = ((live1 >> lane) & 1ull) && covers(L, row, I, r_id[1]);
+    }
+    const uint64_t t0 = live0 & wballot(c0), t1 = live1 & wballot(c1);
+    ndist += popc64(t0) + popc64(t1);
+    const uint64_t o0 = (uint64_t)rank_u(r_occ[0][0], r_occ[1][0], r) | ((uint64_t)rank_u(r_occ[0][1], r_occ[1][1], r) << 32);
+    const uint64_t o1 = (uint64_t)rank_u(r_occ[0][2], r_occ[1][2], r) | ((uint64_t)rank_u(r_occ[0][3], r_occ[1][3], r) << 32);
+    live0 &= ~(t0 & o0);
+    live1 &= ~(t1 & o1);
+  }
+  wave_sync();
+  return sel;
+}
+
 // ---------------------------------------------------------------------------
 // Kernels.
 // ---------------------------------------------------------------------------
@@ -682,8 +838,14 @@ struct MList {
 // canonical_merge_candidates with the label quota (:4703-4842),
 // canonical_compute_work_distances (:4844-4871) and canonical_exact_prune
 // (:4876-4994) fused; the merged list never leaves the wave.
+// The Gram tiles' accumulators would take the uint8 kernels of one and two
+// chunks per lane below the waves that the search needs in flight: 8 and 7
+// waves per SIMD hold without a spill (without these floors k_row was 69.8 and
+// k_csr 25.6 ms, with them 64.1 and 21.7).
+constexpr int min_waves(int dt, int cpl, int waves) { return dt == DANCE_U8 && cpl <= 2 ? waves : 1; }
+
 template <int DT, int CPL>
-__global__ __launch_bounds__(kBlock) void k_row(RowSet rs, Graph G, Labels L, RowArgs A) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(min_waves(DT, CPL, 8), 8))) void k_row(RowSet rs, Graph G, Labels L, RowArgs A) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t k = xcd_block(grid_block(), grid_blocks()) * kWaves + w;
@@ -838,7 +1000,11 @@ __global__ __launch_bounds__(kBlock) void k_row(RowSet rs, Graph G, Labels L, Ro
   if (lane >= count) rem |= 1u;
   if (lane + 64 >= count) rem |= 2u;
   uint32_t outv;
-  const uint32_t sel = prune_regs<DT, CPL, 2>(rs, L, row, R, A.alpha, id, d, rem, lst, lsd, lane, outv, ndist_prune);
+  uint32_t sel;
+  if constexpr (DT == DANCE_U8)
+    sel = prune_gram<CPL, 2>(rs, L, row, R, A.alpha, id, d, rem, lds, lane, outv, ndist_prune);
+  else
+    sel = prune_regs<DT, CPL, 2>(rs, L, row, R, A.alpha, id, d, rem, lst, lsd, lane, outv, ndist_prune);
   if (lane < R) A.gout[(size_t)row * R + lane] = lane < sel ? outv : DANCE_INV;
   if (lane == 0) {
     A.dout[row] = sel;
@@ -917,7 +1083,7 @@ struct CsrArgs {
 // the selection is unchanged). Rows without reverse sources keep their row;
 // rows of more than kCsrRegMax candidates are left to k_csr_long.
 template <int DT, int CPL>
-__global__ __launch_bounds__(kBlock) void k_csr(RowSet rs, Graph G, Labels L, CsrArgs A) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(min_waves(DT, CPL, 7), 8))) void k_csr(RowSet rs, Graph G, Labels L, CsrArgs A) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t row = xcd_block(grid_block(), grid_blocks()) * kWaves + w;
@@ -934,7 +1100,7 @@ __global__ __launch_bounds__(kBlock) void k_csr(RowSet rs, Graph G, Labels L, Cs
   const uint32_t deg = min(G.d[row], R);
   const uint32_t n = deg + (s1 - s0);
   if (n > kCsrRegMax) return;
-  uint32_t* fw = smem + w * kCsrLds;
+  uint32_t* fw = smem + w * csr_lds(DT);
   uint32_t* lst = fw + 64;
   float* lsd = reinterpret_cast<float*>(fw + 128);
   fw[lane] = lane < deg ? G.g[gb + lane] : DANCE_INV;
@@ -974,7 +1140,15 @@ __global__ __launch_bounds__(kBlock) void k_csr(RowSet rs, Graph G, Labels L, Cs
       wave_sync();
     }
   }
-  const uint32_t sel = prune_regs<DT, CPL, (int)kCsrSlots>(rs, L, row, R, A.alpha, id, d, rem, lst, lsd, lane, outv, npd);
+  uint32_t sel = 0;
+  bool done = false;
+  if constexpr (DT == DANCE_U8) {
+    if (nd <= kGramCap) {  // the live entries
+      sel = prune_gram<CPL, (int)kCsrSlots>(rs, L, row, R, A.alpha, id, d, rem, fw, lane, outv, npd);
+      done = true;
+    }
+  }
+  if (!done) sel = prune_regs<DT, CPL, (int)kCsrSlots>(rs, L, row, R, A.alpha, id, d, rem, lst, lsd, lane, outv, npd);
   if (lane < R) A.gout[gb + lane] = lane < sel ? outv : DANCE_INV;
   if (lane == 0) {
     A.dout[row] = sel;

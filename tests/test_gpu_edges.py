@@ -161,3 +161,26 @@ def test_leased_memory_reuse():
     for t in threads:
         t.join()
     assert not errors, errors
+
+
+# uint8 prunes from Gram tiles: rows of 1 to 16 chunks per lane, reverse lists on
+# both sides of 128 entries, rows of more than 32 labels (no label masks), data
+# full of equal rows and distances
+@pytest.mark.parametrize("dim,R,C,labels,equal", [(7, 32, 64, 3, False), (130, 64, 750, 3, False),
+                                                  (192, 64, 750, 40, False), (300, 32, 64, 3, True),
+                                                  (513, 32, 64, 3, False), (1100, 16, 40, 3, True)])
+def test_filtered_gram_prune(dim, R, C, labels, equal):
+    from dance_amd import filtered as F
+    n, vocab = 1200, 60 if labels > 32 else 6
+    rng = np.random.default_rng(dim)
+    x = rng.integers(0, 256, (n, dim), dtype=np.uint8)
+    if equal:
+        x = np.ascontiguousarray(x[rng.integers(0, 40, n)])
+    ls = F.canonical_labels([rng.choice(vocab, labels, replace=False).tolist() for _ in range(n)], vocab)
+    starts, gs = F.label_starts(x, ls), F.global_start(x)
+    g, d = np.empty((n, R), np.uint32), np.empty(n, np.uint32)
+    rc = F.build_rc(x, ls, starts, R, 48, 32, C, 24, 1.2, D.INVALID, gs, 2, graph=g, degree=d)
+    orc, og, od, _ = O.filtered_build(x, ls.offsets, ls.labels, starts, ls.num_labels, R, 48, 32, C, 24, 1.2,
+                                      D.INVALID, gs, 2, 0)
+    assert rc == orc == 0
+    assert np.array_equal(d, od) and np.array_equal(g, og)
