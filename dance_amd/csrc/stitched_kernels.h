@@ -30,10 +30,11 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint64_t n, uint32_t v) {
 }
 
 struct RemapArgs {
-  const uint32_t* local;      // m x Rs local graph (local ids, INVALID-padded)
-  const uint32_t* local_deg;  // m
-  const uint32_t* ids;        // m: local id -> global id
-  uint32_t m, Rs;
+  const uint32_t* local;      // n x Rs local graph (local ids, INVALID-padded)
+  const uint32_t* local_deg;  // n
+  const uint32_t* ids;        // n: local id -> global id
+  uint32_t first, m;          // the local points of this launch
+  uint32_t n, Rs;
   uint32_t take;              // at most `take` leading entries of each local row (Rstitched)
   uint32_t* graph;            // N x row_cap global rows
   uint32_t* degree;           // N
@@ -54,8 +55,9 @@ __global__ __launch_bounds__(64 * kRemapWaves) void k_stitch_remap(RemapArgs a) 
   __shared__ uint32_t s_row[kRemapWaves][256];
   __shared__ uint32_t s_new[kRemapWaves][64];
   const uint32_t w = wave_index(), lane = lane_id();
-  const uint32_t i = grid_block() * kRemapWaves + w;
-  if (i >= a.m) return;
+  const uint32_t at = grid_block() * kRemapWaves + w;
+  if (at >= a.m) return;
+  const uint32_t i = a.first + at;
   const uint32_t me = a.ids[i];
   const uint32_t deg = min(min(a.local_deg[i], a.take), a.Rs);
   uint32_t* row = a.graph + (size_t)me * a.row_cap;
@@ -67,7 +69,7 @@ __global__ __launch_bounds__(64 * kRemapWaves) void k_stitch_remap(RemapArgs a) 
     const uint32_t j = b + lane;
     const bool in = j < deg;
     const uint32_t nb = in ? a.local[(size_t)i * a.Rs + j] : DANCE_INV;
-    const bool valid = in && nb < a.m;
+    const bool valid = in && nb < a.n;
     const uint32_t g = valid ? a.ids[nb] : DANCE_INV;
     const bool self = valid && g == me;
     const bool cand = valid && !self;

@@ -156,24 +156,26 @@ static uint32_t wave_grid(uint32_t n) { return (n + kWavesPerBlock - 1) / kWaves
 // of 8 workgroups, 2-D beyond 2^32 work-items (grid_dims).
 static dim3 xcd_grid(uint32_t n) { return grid_dims(wave_grid(n), kBlock, 8); }
 
+// nseg > 0: the builds of sg, nc and ns the most one of them takes.
 static int launch_medoid(const Rows& rows, hipStream_t s, float* d_scores, uint32_t* d_cands, uint32_t nc,
-                         uint32_t ns) {
+                         uint32_t ns, Segments sg = {}, uint32_t nseg = 0) {
   const int cpl = pick_cpl(rows.rs.nch);
   return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int CPL = decltype(c)::value;
     constexpr uint32_t KC = medoid_cands(CPL);
-    hipLaunchKernelGGL((k_medoid<decltype(dt)::value, CPL>), dim3((nc + KC - 1) / KC), dim3(64 * medoid_waves(CPL)),
-                       medoid_lds_bytes(CPL), s, rows.rs, rows.N, nc, ns, d_scores, d_cands);
+    hipLaunchKernelGGL((k_medoid<decltype(dt)::value, CPL>), dim3((nc + KC - 1) / KC, std::max(nseg, 1u)),
+                       dim3(64 * medoid_waves(CPL)), medoid_lds_bytes(CPL), s, rows.rs, rows.N, nc, ns, d_scores,
+                       d_cands, sg);
     DHIP(hipGetLastError());
     return 0;
   });
 }
 
-static int launch_init(const Rows& rows, GraphBufs g, hipStream_t s) {
+static int launch_init(const Rows& rows, GraphBufs g, hipStream_t s, Segments sg = {}) {
   const int cpl = pick_cpl(rows.rs.nch);
   return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     hipLaunchKernelGGL((k_init<decltype(dt)::value, decltype(c)::value>), grid_dims(wave_grid(g.N), kBlock), dim3(kBlock), 0, s,
-                       rows.rs, g);
+                       rows.rs, g, sg);
     DHIP(hipGetLastError());
     return 0;
   });
@@ -278,11 +280,11 @@ static int build_qbound(const Rows& rows, DevBuf& buf, hipStream_t s, QBoundSet*
 // build then launches no k_init at L <= 128).
 static int launch_search(const Rows& rows, GraphBufs g, uint32_t L, uint32_t steps, float alpha, uint32_t start,
                          const uint32_t* order, VCounters* ctr, const QBoundSet& qb, hipStream_t s,
-                         bool insert_bound, bool hashed_cur, bool padded) {
+                         bool insert_bound, bool hashed_cur, bool padded, Segments sg = {}) {
   const int cpl = pick_cpl(rows.rs.nch);
   const uint32_t Cp = round64(g.C);
   const size_t lds = (size_t)kWavesPerBlock * search_lds_words(Cp) * 4;
-  SearchArgs a{rows.rs, g, L, steps, start, alpha, order, ctr, qb, padded};
+  SearchArgs a{rows.rs, g, L, steps, start, alpha, order, ctr, qb, padded, sg};
   if (L > kMaxBuildL) {
     std::fprintf(stderr, "[dance_hip] L=%u exceeds the supported maximum %u\n", L, kMaxBuildL);
     return -1;
@@ -735,11 +737,26 @@ static int validate(uint32_t N, uint32_t dim, uint32_t R, uint32_t L, uint32_t C
   return 0;
 }
 
+// The builds of a run_build over several at once: build k has rows[k] rows,
+// which follow those of build k - 1; medoid[k] is set to its entry point,
+// counted from its first row.
+struct BuildGroup {
+  std::vector<uint32_t> rows, medoid;
+};
+static size_t group_bytes(size_t builds, size_t rows) {
+  auto aligned = [](size_t b) { return (b + 255u) & ~(size_t)255u; };
+  return aligned(builds * sizeof(uint4)) + aligned(rows * 4) + 2 * aligned(builds * kMedoidCandidates * 4);
+}
+
 // Runs the whole build. On success st.cur/deg_cur hold the graph.
-// Callers hold g_mu and pass the active profile.
+// Callers hold g_mu and pass the active profile. With `group`, rows are those
+// of its builds one after the other (two builds or more); each build's part of
+// the graph is what a build of its rows alone gives, with ids counted from the
+// first row of all. Then rows are processed in their order (each build's rows
+// fit an XCD's L2), and the first search reads the graph of k_init.
 static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint32_t STEPS, const Profile& prof,
                      State& st, hipStream_t s, GPUVamanaStats* stats, DanceKernelProfile* kp, uint32_t* medoid_out,
-                     bool timed = true, bool wide_bound = true) {
+                     bool timed = true, bool wide_bound = true, BuildGroup* group = nullptr) {
   const uint32_t N = rows.N;
   if (pick_cpl(rows.rs.nch) < 0) {
     std::fprintf(stderr, "[gpu_vamana_build] dim=%u is beyond the supported row width\n", rows.dim);
@@ -764,36 +781,65 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
 
   // Approximate medoid (vnew2.cu:2359-2479): device scores, host top-1.
   const double t_med = now_sec();
-  const uint32_t nc = std::min(kMedoidCandidates, N), ns = std::min(kMedoidSamples, N);
-  DCHECK(scores.alloc(nc * 4));
-  DCHECK(cands.alloc(nc * 4));
-  DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns));
-  float hs[kMedoidCandidates];
-  uint32_t hc[kMedoidCandidates];
-  DHIP(hipMemcpyAsync(hs, scores.p, nc * 4, hipMemcpyDeviceToHost, s));
-  DHIP(hipMemcpyAsync(hc, cands.p, nc * 4, hipMemcpyDeviceToHost, s));
-  DCHECK(record(e_med, s));
-  DHIP(hipStreamSynchronize(s));
-  uint32_t best = DANCE_INV;
-  float bs = FLT_MAX;
-  for (uint32_t i = 0; i < nc; ++i)
-    if (hs[i] < bs) {
-      bs = hs[i];
-      best = i;
+  uint32_t start = 0;
+  Segments sg;
+  DevBuf seg, seg_of;
+  std::vector<uint4> hseg;
+  if (group) {
+    const uint32_t nb = (uint32_t)group->rows.size();
+    uint32_t lo = 0, most = 0;
+    for (uint32_t m : group->rows) {
+      hseg.push_back(make_uint4(lo, m, lo, 0u));
+      lo += m;
+      most = std::max(most, m);
     }
-  const uint32_t start = best == DANCE_INV ? 0u : hc[best];
+    if (lo != N || nb < 2) return -1;
+    const uint32_t nc = std::min(kMedoidCandidates, most), ns = std::min(kMedoidSamples, most);
+    DCHECK(seg.alloc(nb * sizeof(uint4)));
+    DCHECK(seg_of.alloc((size_t)N * 4));
+    DCHECK(scores.alloc((size_t)nb * nc * 4));
+    DCHECK(cands.alloc((size_t)nb * nc * 4));
+    sg = Segments{seg.as<uint4>(), seg_of.as<uint32_t>()};
+    DHIP(hipMemcpyAsync(seg.p, hseg.data(), nb * sizeof(uint4), hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_seg_rows, dim3((N + 255) / 256), dim3(256), 0, s, sg, nb, N, seg_of.as<uint32_t>());
+    DHIP(hipGetLastError());
+    DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns, sg, nb));
+    hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(64), 0, s, scores.as<const float>(), cands.as<const uint32_t>(), nc,
+                       sg);
+    DHIP(hipGetLastError());
+    DCHECK(record(e_med, s));
+  } else {
+    const uint32_t nc = std::min(kMedoidCandidates, N), ns = std::min(kMedoidSamples, N);
+    DCHECK(scores.alloc(nc * 4));
+    DCHECK(cands.alloc(nc * 4));
+    DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns));
+    float hs[kMedoidCandidates];
+    uint32_t hc[kMedoidCandidates];
+    DHIP(hipMemcpyAsync(hs, scores.p, nc * 4, hipMemcpyDeviceToHost, s));
+    DHIP(hipMemcpyAsync(hc, cands.p, nc * 4, hipMemcpyDeviceToHost, s));
+    DCHECK(record(e_med, s));
+    DHIP(hipStreamSynchronize(s));
+    uint32_t best = DANCE_INV;
+    float bs = FLT_MAX;
+    for (uint32_t i = 0; i < nc; ++i)
+      if (hs[i] < bs) {
+        bs = hs[i];
+        best = i;
+      }
+    start = best == DANCE_INV ? 0u : hc[best];
+  }
   if (stats) stats->medoid_seconds = now_sec() - t_med;
 
   // At L <= 128 the first search launch computes the initial rows itself
   // (its hashed-neighbour variants), and nothing reads cur, work or wd
   // before it; k_init runs for the other variants only.
-  const bool init_in_search = L <= 128;
-  if (!init_in_search) DCHECK(launch_init(rows, g, s));
+  const bool init_in_search = L <= 128 && !group;
+  if (!init_in_search) DCHECK(launch_init(rows, g, s, sg));
   DevBuf qbuf;
   QBoundSet qb{};
   DCHECK(build_qbound(rows, qbuf, s, &qb, wide_bound));
   const uint32_t* order = nullptr;
-  DCHECK(build_schedule(rows, qb, rws, s, &order));
+  if (!group) DCHECK(build_schedule(rows, qb, rws, s, &order));
   uint32_t q_iters = qbound_iters();  // later iterations' bits may be set on the way (kDenseFrac)
   bool dense = false;
   const double row_bytes = (double)rows.rs.stride16 * 16.0 * (double)N;
@@ -828,7 +874,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     DCHECK(record(iev[it].s0, s));
     const QBoundSet qb_it = ((q_iters >> it) & 1u) ? qb : QBoundSet{};
     DCHECK(launch_search(rows, g, L, steps, alpha, start, order, ctr, qb_it, s, ((ib_iters >> it) & 1u) != 0,
-                         it == 0, true));  // k_init wrote cur just before
+                         it == 0 && !group, true, sg));
     DCHECK(record(iev[it].s1, s));
     RevCsr rev{};
     DCHECK(build_reverse_csr(g, rws, s, &rev));
@@ -880,6 +926,12 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   }
   DHIP(hipStreamSynchronize(s));
   DHIP(hipGetLastError());
+  if (group) {
+    DHIP(hipMemcpyAsync(hseg.data(), seg.p, hseg.size() * sizeof(uint4), hipMemcpyDeviceToHost, s));
+    DHIP(hipStreamSynchronize(s));
+    group->medoid.clear();
+    for (const uint4& b : hseg) group->medoid.push_back(b.z - b.x);
+  }
 
   VCounters hc_ctr{};
   {
@@ -1429,6 +1481,12 @@ static uint32_t stitched_workers() {
   return std::min(std::max(v, 1u), 16u);
 }
 
+// Rows of the small labels built together, and the padded row bytes of a label
+// that counts as small (the L2 of an XCD).
+constexpr uint32_t kGroupRows = 128u << 10;
+constexpr uint32_t kGroupBuilds = 4096;  // a launch's grid.y, and their medoid scores
+constexpr size_t kGroupLabelBytes = 4ull << 20;
+
 // Callers hold g_mu (the workers take no lock: they touch only their own
 // arena, stream and staging slices).
 static int stitched_build(const StitchedIn& in) {
@@ -1524,10 +1582,9 @@ static int stitched_build(const StitchedIn& in) {
   hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, s, d_ctr.as<uint32_t>(), (uint64_t)6, 0u);
   DHIP(hipGetLastError());
 
-  // The per-label builds run side by side on W worker threads (stitched_
-  // workers()), each with its own stream and its own device arena sized for
-  // the largest label (rows and all of the build's buffers). Small labels
-  // leave most of the GPU idle, so several in flight keep it busy. Each
+  // The builds run side by side on W worker threads (stitched_workers()),
+  // each with its own stream and its own device arena sized for the largest
+  // task (rows and all of the build's buffers). Each
   // label's local graph lands in a staging buffer (label l at off[l] rows);
   // the remaps into the global rows then run on this stream in label order,
   // since the cross-label dedupe of multi-label rows depends on that order.
@@ -1536,12 +1593,36 @@ static int stitched_build(const StitchedIn& in) {
   const uint32_t nch = 8u * (uint32_t)cpl;
   const size_t stride = (size_t)nch * 16;
   auto aligned = [](size_t b) { return (b + 255u) & ~(size_t)255u; };
-  const size_t arena_bytes = m_max ? aligned(stride * m_max) +
-                                         resident_build_bytes(nullptr, store, store, m_max, in.dim, in.Rs, in.C, true)
-                                   : 0;
-  uint32_t nonempty = 0;
-  for (uint32_t l = 0; l < in.num_labels; ++l) nonempty += off[l + 1] > off[l] ? 1u : 0u;
-  const uint32_t W = std::max(1u, std::min(stitched_workers(), nonempty));
+  // Small labels are built together, kGroupRows rows at a time: labels whose
+  // rows fit an XCD's L2 gain nothing from a schedule of their own, and one
+  // launch over many fills the GPU. uint8 rows of 192 (R 32, L 100, C 96), each
+  // label alone on 8 streams and together: 500k in labels of 10k rows 105 -> 98
+  // ms, of 16k 137 -> 128; 100k in labels of 1k 43 -> 21; 50k in labels of 100
+  // 99 -> 7.3. Above the line it hardly matters: labels of 30k 151 -> 148 ms.
+  struct Task {
+    uint32_t l0, l1;  // labels
+    uint32_t builds;  // that have rows
+  };
+  std::vector<Task> tasks;
+  const uint32_t small = (uint32_t)std::min<size_t>(kGroupRows, kGroupLabelBytes / stride);
+  size_t arena_bytes = 0;
+  for (uint32_t l = 0; l < in.num_labels;) {
+    Task t{l, l + 1, off[l + 1] > off[l] ? 1u : 0u};
+    if (off[l + 1] - off[l] <= small)
+      while (t.l1 < in.num_labels && t.builds < kGroupBuilds && off[t.l1 + 1] - off[t.l1] <= small &&
+             off[t.l1 + 1] - off[l] <= kGroupRows) {
+        t.builds += off[t.l1 + 1] > off[t.l1] ? 1u : 0u;
+        ++t.l1;
+      }
+    const uint32_t m = off[t.l1] - off[l];
+    l = t.l1;
+    if (m == 0) continue;
+    tasks.push_back(t);
+    arena_bytes = std::max(arena_bytes, aligned(stride * m) +
+                                            resident_build_bytes(nullptr, store, store, m, in.dim, in.Rs, in.C, true) +
+                                            (t.builds > 1 ? group_bytes(t.builds, m) : 0));
+  }
+  const uint32_t W = std::max(1u, std::min(stitched_workers(), (uint32_t)tasks.size()));
   std::vector<DevBuf> arenas(W);
   for (auto& a : arenas) DCHECK(a.alloc(arena_bytes));
   DevBuf stage_g, stage_d;
@@ -1565,10 +1646,12 @@ static int stitched_build(const StitchedIn& in) {
     double materialize = 0, build_sum = 0, build_max = 0;
   };
   std::vector<WorkerTimes> times(W);
-  // One label on worker w's stream: gather its rows, build, leave the local
-  // graph in the staging buffer.
-  auto build_label = [&](uint32_t w, uint32_t l, hipStream_t ws) -> int {
-    const uint32_t m = off[l + 1] - off[l];
+  // One task on worker w's stream: gather its labels' rows, build, leave the
+  // local graphs in the staging buffer, with ids counted from the task's first
+  // row.
+  auto build_task = [&](uint32_t w, const Task& t, hipStream_t ws) -> int {
+    const uint32_t l = t.l0;
+    const uint32_t m = off[t.l1] - off[l];
     Arena arena{arenas[w].as<char>(), arena_bytes, 0};
     ArenaScope scope(&arena);
     const uint32_t* ids = d_pts.as<uint32_t>() + off[l];
@@ -1594,7 +1677,14 @@ static int stitched_build(const StitchedIn& in) {
     lst.deg_cur.p = stage_d.as<uint32_t>() + off[l];
     lst.deg_cur.bytes = (size_t)m * 4;
     lst.deg_cur.borrowed = true;
-    DCHECK(run_build(rows, in.Rs, in.Ls, in.C, steps, prof, lst, ws, nullptr, nullptr, &local_medoid[l], false));
+    BuildGroup group;
+    for (uint32_t k = t.l0; k < t.l1; ++k)
+      if (off[k + 1] > off[k]) group.rows.push_back(off[k + 1] - off[k]);
+    uint32_t medoid = 0;
+    DCHECK(run_build(rows, in.Rs, in.Ls, in.C, steps, prof, lst, ws, nullptr, nullptr, &medoid, false, true,
+                     t.builds > 1 ? &group : nullptr));
+    for (uint32_t k = t.l0, b = 0; k < t.l1; ++k)
+      if (off[k + 1] > off[k]) local_medoid[k] = t.builds > 1 ? group.medoid[b++] : medoid;
     const double dt = now_sec() - tb;
     const uint64_t used = device_used_bytes();
     for (uint64_t cur = peak_used.load(); used > cur && !peak_used.compare_exchange_weak(cur, used);) {
@@ -1613,8 +1703,8 @@ static int stitched_build(const StitchedIn& in) {
       failed = 1;
       return;
     }
-    for (uint32_t l; !failed && (l = next.fetch_add(1)) < in.num_labels;)
-      if (off[l + 1] > off[l] && build_label(w, l, ws) != 0) failed = 1;
+    for (uint32_t t; !failed && (t = next.fetch_add(1)) < tasks.size();)
+      if (build_task(w, tasks[t], ws) != 0) failed = 1;
     (void)hipStreamDestroy(ws);
   };
   {
@@ -1630,19 +1720,24 @@ static int stitched_build(const StitchedIn& in) {
     st.build_max_seconds = std::max(st.build_max_seconds, t.build_max);
   }
   const double tr = now_sec();
+  // With one label per point no two labels append to a row, and a task's
+  // labels are remapped at once.
+  for (const Task& t : tasks) {
+    const uint32_t base = off[t.l0], n = off[t.l1] - base;
+    for (uint32_t l = t.l0; l < t.l1; l = most <= 1 ? t.l1 : l + 1) {
+      const uint32_t first = off[l] - base, m = most <= 1 ? n : off[l + 1] - off[l];
+      if (m == 0) continue;
+      RemapArgs ra{stage_g.as<uint32_t>() + (size_t)base * in.Rs, stage_d.as<uint32_t>() + base,
+                   d_pts.as<uint32_t>() + base, first, m, n, in.Rs, in.Rout, gg, gd, in.row_cap,
+                   d_ctr.as<unsigned long long>()};
+      hipLaunchKernelGGL(k_stitch_remap, grid_dims(((uint64_t)m + kRemapWaves - 1) / kRemapWaves, 64 * kRemapWaves),
+                         dim3(64 * kRemapWaves), 0, s, ra);
+      DHIP(hipGetLastError());
+    }
+  }
   for (uint32_t l = 0; l < in.num_labels; ++l) {
     const uint32_t m = off[l + 1] - off[l];
-    if (m == 0) {
-      in.medoids[l] = DANCE_INV;
-      continue;
-    }
-    RemapArgs ra{stage_g.as<uint32_t>() + (size_t)off[l] * in.Rs, stage_d.as<uint32_t>() + off[l],
-                 d_pts.as<uint32_t>() + off[l], m, in.Rs, in.Rout, gg, gd, in.row_cap,
-                 d_ctr.as<unsigned long long>()};
-    hipLaunchKernelGGL(k_stitch_remap, grid_dims(((uint64_t)m + kRemapWaves - 1) / kRemapWaves, 64 * kRemapWaves),
-                       dim3(64 * kRemapWaves), 0, s, ra);
-    DHIP(hipGetLastError());
-    in.medoids[l] = in.label_points[off[l] + (local_medoid[l] < m ? local_medoid[l] : 0u)];
+    in.medoids[l] = m == 0 ? DANCE_INV : in.label_points[off[l] + (local_medoid[l] < m ? local_medoid[l] : 0u)];
   }
   DHIP(hipStreamSynchronize(s));
   st.remap_seconds = now_sec() - tr;

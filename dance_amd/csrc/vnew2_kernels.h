@@ -385,6 +385,30 @@ __device__ __forceinline__ uint32_t init_neighbor(uint32_t node, uint32_t i, uin
   return (N <= 1 || nb == DANCE_INV || nb >= N || nb == node) ? DANCE_INV : nb;
 }
 
+// Several small builds in one: the rows of build k are [lo[k], lo[k] + m[k]) of
+// the concatenated rows, and every id stays within them. What depends on a
+// build's own size and ids (the random graph and seeds, the entry point) is
+// computed from the row's build; the rest sees one graph.
+struct Segments {
+  uint4* seg = nullptr;          // per build: first row, rows, entry point, 0; nullptr: one build
+  const uint32_t* of = nullptr;  // per row: its build
+  __device__ __forceinline__ uint4 at(uint32_t node) const { return seg[of[node]]; }
+};
+// The build of each row: one thread per row, a binary search in lo.
+static __global__ void k_seg_rows(Segments sg, uint32_t count, uint32_t N, uint32_t* of) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= N) return;
+  uint32_t a = 0, b = count;  // the last build with lo <= i is in [a, b)
+  while (b - a > 1u) {
+    const uint32_t c = (a + b) / 2u;
+    if (sg.seg[c].x <= i)
+      a = c;
+    else
+      b = c;
+  }
+  of[i] = a;
+}
+
 struct SearchArgs {
   RowSet rs;
   GraphBufs g;
@@ -396,6 +420,7 @@ struct SearchArgs {
   // cur rows hold DANCE_INV past their degree (every graph the build makes):
   // an expansion then needs no degree, one cache line less to gather
   bool padded;
+  Segments sg;  // read without HC only
 };
 
 // Per-wave LDS words of the search kernel: visited cache, work row (ids,
@@ -866,7 +891,11 @@ struct SearchWave {
     for (uint32_t i = lane; i < kVis; i += 64) vis[i] = DANCE_INV;
     wave_sync();
     // Entry point (vnew2.cu:1223-1244).
-    process_batch(lane == 0 && a.start < N && a.start != node ? a.start : DANCE_INV);
+    uint32_t start = a.start;
+    if constexpr (!HC) {
+      if (a.sg.seg) start = uni_u(a.sg.at(node).z);
+    }
+    process_batch(lane == 0 && start < N && start != node ? start : DANCE_INV);
     // Own neighbours with stored distances (vnew2.cu:1246-1278), inserted in
     // row order. When they fit in one batch, the pool holds at most the entry
     // point, no two of them (nor one and the entry point) share a visited
@@ -934,7 +963,16 @@ struct SearchWave {
       wave_sync();
     }
     // INIT_RANDOM_SEEDS hashed seeds (vnew2.cu:1280-1300).
-    process_batch(lane < 8 ? d_det_neighbor(node, lane + 1024u, N) : DANCE_INV);
+    uint32_t lo = 0, m = N;
+    if constexpr (!HC) {
+      if (a.sg.seg) {
+        const uint4 b = a.sg.at(node);
+        lo = uni_u(b.x);
+        m = uni_u(b.y);
+      }
+    }
+    const uint32_t seed = lane < 8 ? d_det_neighbor(node - lo, lane + 1024u, m) : DANCE_INV;
+    process_batch(seed == DANCE_INV ? seed : seed + lo);
     const uint32_t max_steps = min(a.steps, a.L);
     uint32_t n_exp = 0;
     const uint64_t t_seed = dclock() - t_run;
@@ -2237,7 +2275,17 @@ constexpr size_t medoid_lds_bytes(int cpl) { return (size_t)medoid_cands(cpl) * 
 
 template <int DT, int CPL>
 __global__ __launch_bounds__(64 * medoid_waves(CPL)) void k_medoid(RowSet rs, uint32_t N, uint32_t nc, uint32_t ns,
-                                                              float* scores, uint32_t* cands) {
+                                                              float* scores, uint32_t* cands, Segments sg) {
+  if (sg.seg) {  // grid.y: the builds; nc and ns are the most one of them takes, and the scores' stride is nc
+    const uint4 b = sg.seg[blockIdx.y];
+    scores += (size_t)blockIdx.y * nc;
+    cands += (size_t)blockIdx.y * nc;
+    rs.rows += (size_t)uni_u(b.x) * rs.stride16;
+    N = uni_u(b.y);
+    nc = min(nc, N);
+    ns = min(ns, N);
+    if (blockIdx.x * medoid_cands(CPL) >= nc) return;
+  }
   constexpr uint32_t KC = medoid_cands(CPL);
   extern __shared__ uint32_t smem[];
   float* dist = reinterpret_cast<float*>(smem);  // KC x kMedoidMaxSamples
@@ -2292,9 +2340,36 @@ __global__ __launch_bounds__(64 * medoid_waves(CPL)) void k_medoid(RowSet rs, ui
   }
 }
 
+// Entry point of each build from its scores (the first of the least, row 0 of
+// the build if no score is below FLT_MAX): one wave per build.
+static __global__ __launch_bounds__(64) void k_seg_start(const float* __restrict__ scores,
+                                                        const uint32_t* __restrict__ cands, uint32_t stride,
+                                                        Segments sg) {
+  const uint32_t lane = lane_id();
+  const uint4 b = sg.seg[blockIdx.x];
+  const float* mine = scores + (size_t)blockIdx.x * stride;
+  float bs = FLT_MAX;
+  uint32_t best = DANCE_INV;
+  for (uint32_t i = lane; i < min(stride, b.y); i += 64)
+    if (mine[i] < bs) {
+      bs = mine[i];
+      best = i;
+    }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    const float os = __shfl_xor(bs, d);
+    const uint32_t ob = (uint32_t)__shfl_xor((int)best, d);
+    if (os < bs || (os == bs && ob < best)) {
+      bs = os;
+      best = ob;
+    }
+  }
+  if (lane == 0) sg.seg[blockIdx.x].z = b.x + (best == DANCE_INV ? 0u : cands[(size_t)blockIdx.x * stride + best]);
+}
+
 // init_random_graph (vnew2.cu:1066-1117): R hashed neighbours per vertex.
 template <int DT, int CPL>
-__global__ __launch_bounds__(kBlock) void k_init(RowSet rs, GraphBufs g) {
+__global__ __launch_bounds__(kBlock) void k_init(RowSet rs, GraphBufs g, Segments sg) {
   __shared__ uint32_t lstb[kWavesPerBlock][64];
   __shared__ float lsdb[kWavesPerBlock][64];
   const uint32_t w = wave_index();
@@ -2309,9 +2384,16 @@ __global__ __launch_bounds__(kBlock) void k_init(RowSet rs, GraphBufs g) {
   }
   uint4 nv[CPL];
   load_row<CPL>(rs, node, true, sub, nv);
+  uint32_t lo = 0, m_rows = N;
+  if (sg.seg) {
+    const uint4 sb = sg.at(node);
+    lo = uni_u(sb.x);
+    m_rows = uni_u(sb.y);
+  }
   for (uint32_t b = 0; b < R; b += 64) {
     const uint32_t i = b + lane;
-    const uint32_t nb = i < R ? init_neighbor(node, i, N) : DANCE_INV;
+    uint32_t nb = i < R ? init_neighbor(node - lo, i, m_rows) : DANCE_INV;
+    if (nb != DANCE_INV) nb += lo;
     const bool v = i < R && nb != DANCE_INV;
     const uint64_t m = wballot(v);
     const uint32_t n = popc64(m);
@@ -2327,7 +2409,7 @@ __global__ __launch_bounds__(kBlock) void k_init(RowSet rs, GraphBufs g) {
     wave_sync();
   }
   if (lane == 0) {
-    const uint32_t deg = N > 1 ? R : 0u;
+    const uint32_t deg = m_rows > 1 ? R : 0u;
     g.deg_cur[node] = deg;
     g.deg_work[node] = deg;
   }

@@ -117,17 +117,17 @@ int dance_vamana_build_resident_noalloc(const void *d_data, int dtype, uint32_t 
  * must hold every label of a point (labels x min(R_small, R_stitched)) and be
  * at most 256. label_medoids[l] is the global id of label l's medoid
  * (INVALID for a label without points). Label postings and medoids are host
- * arrays. Returns 0, or -1 with a message. The per-label builds run on
- * several streams at once (DANCE_STITCHED_WORKERS, default 8);
- * materialize_seconds and build_sum_seconds add up the per-label times, so
- * they can exceed total_seconds. */
+ * arrays. Returns 0, or -1 with a message. Small labels are built together,
+ * and the builds run on several streams at once (DANCE_STITCHED_WORKERS,
+ * default 8); materialize_seconds and build_sum_seconds add up the times of
+ * the builds, so they can exceed total_seconds. */
 typedef struct {
     double setup_seconds, materialize_seconds, build_sum_seconds, build_max_seconds, remap_seconds, total_seconds;
     uint64_t memberships, remap_invalid_local_ids, remap_self_loops, remap_duplicate_edges;
     uint32_t labels, label_npts_min, label_npts_max, row_cap;
     /* device memory in use (hipMemGetInfo: total - free, GiB, every process
-     * on the GPU counted), the largest of the samples before the label loop,
-     * after each label build and after the remap, as the reference's app
+     * on the GPU counted), the largest of the samples before the builds,
+     * after each of them and after the remap, as the reference's app
      * reports it (apps/utils/gpu_stitched_vamana_index.cpp:231-306) */
     double peak_gpu_mem_gb;
 } DanceStitchedStats;

@@ -163,6 +163,35 @@ def test_leased_memory_reuse():
     assert not errors, errors
 
 
+# small labels built together: empty labels, labels of one row and around a
+# wave, a label too large for a group between them, pools on both sides of 128
+@pytest.mark.parametrize("kind,dim,L", [("u8", 192, 64), ("f32", 96, 64), ("f32", 130, 140), ("f16", 77, 64)])
+def test_stitched_label_groups(kind, dim, L):
+    big = (4 << 20) // {"u8": 256, "f32": 384 if dim == 96 else 1024, "f16": 256}[kind] + 1  # its rows exceed 4 MiB
+    sizes = [0, 1, 2, 63, 64, 65, 1500, 0, big, 300, 3, 1, 0]
+    R, C, steps = 16, 24, 16
+    n = sum(sizes)
+    x = rows(kind, n, dim, centers=30)
+    x[70:74] = x[69]
+    rng = np.random.default_rng(dim)
+    pts = rng.permutation(n).astype(np.uint32)
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.uint32)
+    for a, b in zip(off[:-1], off[1:]):
+        pts[a:b] = np.sort(pts[a:b])
+    g, d, med, st = D.stitched_build(x, off, pts, R, L, C, steps, R)
+    for a, b, m in zip(off[:-1], off[1:], med):
+        ids = pts[a:b]
+        if a == b:
+            assert m == D.INVALID
+            continue
+        og, od, om = O.vnew2_build(np.ascontiguousarray(x[ids]), R, L, C, steps)
+        assert m == ids[om]
+        for i in range(b - a):
+            want = [ids[v] for v in og[i, :od[i]] if v < b - a and v != i]
+            want = list(dict.fromkeys(want))
+            assert d[ids[i]] == len(want) and g[ids[i], :len(want)].tolist() == want
+
+
 # uint8 prunes from Gram tiles: rows of 1 to 16 chunks per lane, reverse lists on
 # both sides of 128 entries, rows of more than 32 labels (no label masks), data
 # full of equal rows and distances
