@@ -835,7 +835,11 @@ struct SearchWave {
     }
   }
 
-  __device__ void run() {
+  // Always inlined: out of line the wave's state would live in scratch and its
+  // uniform values in lanes, and registers spilled around the then divergent
+  // branches are reloaded under the wrong lane mask (the compiler puts a reload
+  // before the mask's restore).
+  __device__ __forceinline__ void run() {
     const uint64_t t_run = dclock();
     const GraphBufs& g = a.g;
     const uint32_t N = g.N, R = g.R, C = g.C;
@@ -1044,8 +1048,10 @@ struct SearchWave {
 // at 3 chunks per lane; three row addresses live in scratch. 5 waves: first
 // search at 1M x 96 113 -> 108 ms, at 4M 457 -> 464 ms). At 129 <= L <= 256 two
 // chunks per lane fit 6 waves without the bound and 5 with it. Without the bound
-// 4 chunks per lane fit 6 waves and 8 chunks 4 (fp16 rows of 4 chunks took 198
-// registers, 2 waves, with no floor). No constraint elsewhere.
+// 4 chunks per lane run 6 waves and 8 chunks 4, with one or two registers in
+// scratch in most variants; odd fp16 rows hold a few registers more for the
+// tail word and run 5 and 3 (5 with the bound at 3 chunks, too), without. No
+// constraint elsewhere.
 #ifndef DANCE_SEARCH_WAVES
 #define DANCE_SEARCH_WAVES 6
 #endif
@@ -1055,15 +1061,17 @@ struct SearchWave {
 #ifndef DANCE_SEARCH_WAVES_IB
 #define DANCE_SEARCH_WAVES_IB 6
 #endif
-template <int CPL, int PS, bool QB, bool IB, bool HC>
+template <int DT, int CPL, int PS, bool QB, bool IB, bool HC>
 constexpr int kSearchMinWaves =
     (CPL <= 3 && PS == 2)
-        ? (IB ? DANCE_SEARCH_WAVES_IB : QB ? DANCE_SEARCH_WAVES_QB : (CPL <= 2 && HC) ? 8 : DANCE_SEARCH_WAVES)
-        : (CPL <= 2 && PS == 4) ? (QB ? 5 : 6) : (PS == 2 && !QB && CPL <= 8) ? (CPL == 4 ? 6 : 4) : 1;
+        ? (IB ? DANCE_SEARCH_WAVES_IB : QB ? (DT == kF16Odd && CPL == 3 ? 5 : DANCE_SEARCH_WAVES_QB)
+                                           : (CPL <= 2 && HC) ? 8 : DANCE_SEARCH_WAVES)
+        : (CPL <= 2 && PS == 4) ? (QB ? 5 : 6)
+        : (PS == 2 && !QB && CPL <= 8) ? (CPL == 4 ? 6 : 4) - (DT == kF16Odd ? 1 : 0) : 1;
 
 // search_prune_kernel_shared (vnew2.cu:1119-1439).
 template <int DT, int CPL, int PS, bool QB, bool IB = false, bool HC = false, int QC = 1>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSearchMinWaves<CPL, PS, QB, IB, HC>, 8))) void k_search(SearchArgs a, uint32_t Cp) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kSearchMinWaves<DT, CPL, PS, QB, IB, HC>, 8))) void k_search(SearchArgs a, uint32_t Cp) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t gw = xcd_block(grid_block(), grid_blocks()) * kWavesPerBlock + w;

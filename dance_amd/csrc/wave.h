@@ -281,15 +281,29 @@ __device__ __forceinline__ float octet_partial_f(const RowSet& rs, uint32_t sub,
       acc += h2_pair_sq(a[c].w, b[c].w);
     }
   } else {
-    // Word (c, w) of this lane is word 4*sub + 32*c + w of the row.
-    const int tl = rs.tail16 - 4 * (int)sub;
+    // Word (c, w) of lane sub is word 4 sub + 32 c + w of the row, so the tail
+    // is the same (c, w) in every octet and belongs to one lane of it: a scalar
+    // branch finds the word, a select the lane. (With the lane in the condition
+    // of every word, each pair distance took a divergent branch per word.) Rows
+    // take the least chunk group that holds them, so the tail is in the last
+    // chunk of up to 4 and in the upper half of 8 and 16.
+    constexpr int first = CPL <= 4 ? CPL - 1 : CPL / 2;
+    const int tw = rs.tail16 & ~28;
+    const bool mine = (int)sub == ((rs.tail16 >> 2) & 7);
 #pragma unroll
     for (int c = 0; c < CPL; ++c) {
       const uint32_t wa[4] = {a[c].x, a[c].y, a[c].z, a[c].w};
       const uint32_t wb[4] = {b[c].x, b[c].y, b[c].z, b[c].w};
 #pragma unroll
-      for (int w = 0; w < 4; ++w)
-        acc = tl == 32 * c + w ? h2_tail_fma(wa[w], wb[w], acc) : acc + h2_pair_sq(wa[w], wb[w]);
+      for (int w = 0; w < 4; ++w) {
+        const float pair = acc + h2_pair_sq(wa[w], wb[w]);
+        if (c >= first && tw == 32 * c + w) {
+          const float tail = h2_tail_fma(wa[w], wb[w], acc);
+          acc = mine ? tail : pair;
+        } else {
+          acc = pair;
+        }
+      }
     }
   }
   return acc;

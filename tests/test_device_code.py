@@ -1,0 +1,60 @@
+"""The built gfx950 code: what the kernels rely on that no output shows."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+import dance_amd as D
+
+READELF = "/opt/rocm/llvm/bin/llvm-readelf"
+
+
+def code_objects():
+    """The gfx950 code objects in the library's offload bundles."""
+    blob = open(D.LIB_PATH, "rb").read()
+    magic, at, out = b"__CLANG_OFFLOAD_BUNDLE__", 0, []
+    while (at := blob.find(magic, at)) >= 0:
+        (count,), p = struct.unpack_from("<Q", blob, at + 24), at + 32
+        for _ in range(count if count < 16 else 0):
+            off, size, n = struct.unpack_from("<QQQ", blob, p)
+            if b"gfx950" in blob[p + 24:p + 24 + n]:
+                out.append(blob[at + off:at + off + size])
+            p += 24 + n
+        at += len(magic)
+    return out
+
+
+@pytest.fixture(scope="module")
+def notes(tmp_path_factory):
+    if not os.path.exists(READELF) or not os.path.exists(D.LIB_PATH):
+        pytest.skip("needs the built library and llvm-readelf")
+    objs = code_objects()
+    assert objs
+    text = ""
+    for i, o in enumerate(objs):
+        path = tmp_path_factory.mktemp("co") / f"{i}.co"
+        path.write_bytes(o)
+        text += subprocess.run([READELF, "--notes", "--symbols", str(path)], check=True, capture_output=True,
+                               text=True).stdout
+    return text
+
+
+def test_search_state_is_not_in_scratch(notes):
+    """A search kernel keeps its wave's state in registers. A variant whose body is
+    not inlined keeps it in scratch (over 400 bytes a lane), and the values
+    that the code takes for uniform are then spilled under lane masks."""
+    sizes = {}
+    for block in notes.split("  - .agpr_count")[1:]:
+        name = re.search(r"\.name:\s+(\S+)", block[block.index(".max_flat_workgroup_size"):]).group(1)
+        sizes[name] = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", block).group(1))
+    search = {k: v for k, v in sizes.items() if "k_search" in k}
+    assert len(search) > 50
+    assert {k: v for k, v in search.items() if v > 32} == {}
+
+
+def test_every_device_function_is_inlined(notes):
+    functions = {m.group(1) for m in re.finditer(r" FUNC\s+\S+\s+\S+\s+\S+\s+(\S+)", notes)}
+    kernels = {m.group(1) for m in re.finditer(r"\.name:\s+(_Z\S+)", notes)}
+    assert kernels and functions - kernels == set()

@@ -213,3 +213,22 @@ def test_filtered_gram_prune(dim, R, C, labels, equal):
                                       D.INVALID, gs, 2, 0)
     assert rc == orc == 0
     assert np.array_equal(d, od) and np.array_equal(g, og)
+
+
+# odd fp16 rows, whose last element is summed on its own: every row group, both
+# sides of 240 dimensions, with the default degrees (batches of any size up to
+# 64), pools of 2 and 4 slots per lane
+@pytest.mark.parametrize("dim,L", [(63, 100), (127, 100), (129, 100), (129, 140), (191, 100), (193, 100), (239, 140),
+                                   (241, 100), (255, 100), (301, 100), (513, 100)])
+def test_odd_f16_builds(dim, L):
+    import torch
+    n, R, C, steps = 400, 64, 80, 24
+    x = rows("f16", n, dim, seed=dim)
+    og, od, om = O.vnew2_build(x, R, L, C, steps)
+    xt = torch.from_numpy(x).cuda()
+    g = torch.empty((n, R), dtype=torch.int32, device="cuda")
+    d = torch.empty((n,), dtype=torch.int32, device="cuda")
+    D.vamana_build_resident(xt.data_ptr(), D.dtype_code(x), n, dim, R, L, C, steps, g.data_ptr(), d.data_ptr())
+    assert D.last_medoid() == om
+    assert np.array_equal(d.cpu().numpy().view(np.uint32), od)
+    assert np.array_equal(g.cpu().numpy().view(np.uint32), og)
