@@ -200,6 +200,14 @@ constexpr uint32_t kQBoundIters = 0x1u;  // first iteration: random graph, HBM-b
 // Infinity Cache: the last iteration at 4M 245 without and 294 ms with it,
 // at 6M (2.3 GB) 426 and 461, at 10M (3.8 GB) 914 and 810; so there it is
 // taken in the last iteration from kClusteredMinBytes on.
+// A row of as many 128-byte lines as its code row (up to 32 fp32 or 64 fp16
+// dimensions, and 113 to 128 fp16 ones) never takes it here: a proved candidate
+// costs as many lines as its row, any other one twice that. The same searches at
+// 200k, lines of a row and its code row in brackets: 24 fp32 (1, 1) 7.9 / 7.5 / 8.6
+// and 10.2 / 9.8 / 11.3 ms, 64 fp16 (1, 1) 10.8 / 11.1 / 14.1 and 13.2 / 13.4 / 16.7,
+// 128 fp16 (2, 2) 25.6 / 27.4 / 34.4 and 29.0 / 30.6 / 38.2; 48 fp32 (2, 1) 19.1 / 21.5
+// / 28.2 and 15.1 / 15.6 / 20.9, 160 fp16 (3, 2) 40.8 / 43.4 / 54.1 and 35.8 / 35.9 /
+// 45.5.
 // Either way the last iteration takes it only when the iteration before it
 // computed more than kQBoundLastMinDist candidate distances per expansion.
 constexpr double kDenseFrac = 0.25;
@@ -842,6 +850,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   if (!group) DCHECK(build_schedule(rows, qb, rws, s, &order));
   uint32_t q_iters = qbound_iters();  // later iterations' bits may be set on the way (kDenseFrac)
   bool dense = false;
+  const bool fewer_lines = qb.rows && pick_cpl(rows.rs.nch) > qb.groups;  // of a code row than of its row
   const double row_bytes = (double)rows.rs.stride16 * 16.0 * (double)N;
   const uint32_t ib_iters = insert_bound_iters();
   uint32_t q_prune_iters = qbound_prune_iters();  // iteration 1's bit may be set after iteration 0
@@ -896,10 +905,10 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
       const double pairs = (double)g.C * (double)(g.C > 0 ? g.C - 1 : 0) / 2.0;
       dense = (double)h.prune_bound_checks > kDenseFrac * pairs * (double)g.N;
       if (dense && qbound_prune_adaptive()) q_prune_iters |= 2u;
-      if (dense && qbound_iters_adaptive() && row_bytes > kDenseMinBytes)
+      if (dense && fewer_lines && qbound_iters_adaptive() && row_bytes > kDenseMinBytes)
         q_iters |= ((1u << (iters - 1)) - 1u) & ~1u;  // the iterations between the first and the last
     }
-    if (qb.rows && qbound_iters_adaptive() && iters > 1 && it + 3 >= iters && it + 1 < iters) {
+    if (fewer_lines && qbound_iters_adaptive() && iters > 1 && it + 3 >= iters && it + 1 < iters) {
       // candidate distances per expansion of the iteration before the last:
       // cumulative counters after iterations iters - 3 and iters - 2
       hipLaunchKernelGGL(k_ctr_sum, dim3(1), dim3(64), 0, s, static_cast<const VCounters*>(ctr),

@@ -43,11 +43,12 @@ typedef struct DanceKernelProfile {
      * candidates tested, and those whose exact distance it made unnecessary
      * (proved >= the pool threshold). DANCE_QBOUND=0 disables the bound;
      * DANCE_QBOUND_ITERS selects the iterations (bit i = iteration i);
-     * unset, the first iteration, and on data without clusters (iteration 0's
-     * prune reached a quarter of the candidate pairs) whose rows exceed 4 MiB
-     * the iterations up to the last; the last one also takes it when the
-     * iteration before it computed more than 24 candidate distances per
-     * expansion and the data is of that kind or its rows exceed 3 GB. */
+     * unset, the first iteration, and where a row takes more 128-byte lines
+     * than its code row: on data without clusters (iteration 0's prune reached
+     * a quarter of the candidate pairs) whose rows exceed 4 MiB the iterations
+     * up to the last; the last one also takes it when the iteration before it
+     * computed more than 24 candidate distances per expansion and the data is
+     * of that kind or its rows exceed 3 GB. */
     uint64_t bound_checks, bound_skips;
     /* The same bound in RobustPrune: pairs tested, and pairs it proved far
      * enough that the candidate survives (DANCE_QBOUND_PRUNE_ITERS selects

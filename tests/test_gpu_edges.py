@@ -232,3 +232,27 @@ def test_odd_f16_builds(dim, L):
     assert D.last_medoid() == om
     assert np.array_equal(d.cpu().numpy().view(np.uint32), od)
     assert np.array_equal(g.cpu().numpy().view(np.uint32), og)
+
+
+# dense rows take the bound after the first iteration only where a row has more
+# 128-byte lines than its code row: 64 fp16 dimensions have 1 and 1, 128 have 2 and
+# 2, 80 have 2 and 1; the graphs are those of the exact searches
+@pytest.mark.parametrize("dim,middle", [(64, False), (80, True), (128, False)])
+def test_dense_rule_compares_lines(dim, middle, monkeypatch):
+    import torch
+    n, R = 34_000, 48
+    x = torch.from_numpy(rows("f16", n, dim)).cuda()
+    out = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv("DANCE_QBOUND", "0")
+        g = torch.empty((n, R), dtype=torch.int32, device="cuda")
+        d = torch.empty((n,), dtype=torch.int32, device="cuda")
+        D.vamana_build_resident(x.data_ptr(), D.DTYPE_F16, n, dim, R, 64, 64, 32, g.data_ptr(), d.data_ptr())
+        out.append((g, d))
+        if not off:
+            checks = D.last_kernel_profile()["bound_checks_iter"]
+            assert checks[0] > 0
+            assert [c > 0 for c in checks[1:3]] == [middle, middle]
+            assert middle or checks[3] == 0
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
