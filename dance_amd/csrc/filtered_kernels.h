@@ -838,14 +838,20 @@ struct MList {
 // canonical_merge_candidates with the label quota (:4703-4842),
 // canonical_compute_work_distances (:4844-4871) and canonical_exact_prune
 // (:4876-4994) fused; the merged list never leaves the wave.
-// The Gram tiles' accumulators would take the uint8 kernels of one and two
-// chunks per lane below the waves that the search needs in flight: 8 and 7
-// waves per SIMD hold without a spill (without these floors k_row was 69.8 and
-// k_csr 25.6 ms, with them 64.1 and 21.7).
-constexpr int min_waves(int dt, int cpl, int waves) { return dt == DANCE_U8 && cpl <= 2 ? waves : 1; }
+// The Gram tiles' accumulators would take the uint8 kernels of up to four chunks
+// per lane below the waves that the search needs in flight. These waves per
+// SIMD hold without a spill, and are at least those of a kernel without tiles:
+// 8 and 7 at one and two chunks (without the floors k_row was 69.8 and k_csr
+// 25.6 ms, with them 64.1 and 21.7), 7 and 5 at three, 5 for k_row at four (a
+// build of 100k rows of 300 bytes 91.4 ms without these floors, 82.1 with them; of
+// 500 bytes 110.8 and 104.5). Wider rows hold the tiles in what they take anyway.
+constexpr int row_waves(int dt, int cpl) {
+  return dt != DANCE_U8 || cpl > 4 ? 1 : cpl <= 2 ? 8 : cpl == 3 ? 7 : 5;
+}
+constexpr int csr_waves(int dt, int cpl) { return dt != DANCE_U8 || cpl > 3 ? 1 : cpl <= 2 ? 7 : 5; }
 
 template <int DT, int CPL>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(min_waves(DT, CPL, 8), 8))) void k_row(RowSet rs, Graph G, Labels L, RowArgs A) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(row_waves(DT, CPL), 8))) void k_row(RowSet rs, Graph G, Labels L, RowArgs A) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t k = xcd_block(grid_block(), grid_blocks()) * kWaves + w;
@@ -1083,7 +1089,7 @@ struct CsrArgs {
 // the selection is unchanged). Rows without reverse sources keep their row;
 // rows of more than kCsrRegMax candidates are left to k_csr_long.
 template <int DT, int CPL>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(min_waves(DT, CPL, 7), 8))) void k_csr(RowSet rs, Graph G, Labels L, CsrArgs A) {
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(csr_waves(DT, CPL), 8))) void k_csr(RowSet rs, Graph G, Labels L, CsrArgs A) {
   extern __shared__ uint32_t smem[];
   const uint32_t w = wave_index();
   const uint32_t row = xcd_block(grid_block(), grid_blocks()) * kWaves + w;

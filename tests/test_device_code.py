@@ -41,14 +41,20 @@ def notes(tmp_path_factory):
     return text
 
 
+def kernels(notes, field):
+    """A metadata field of every kernel, by its mangled name."""
+    out = {}
+    for block in notes.split("  - .agpr_count")[1:]:
+        block = block[:block.find(".wavefront_size")]
+        out[re.search(r"\.name:\s+(_Z\S+)", block).group(1)] = int(re.search(rf"\.{field}:\s+(\d+)", block).group(1))
+    return out
+
+
 def test_search_state_is_not_in_scratch(notes):
     """A search kernel keeps its wave's state in registers. A variant whose body is
     not inlined keeps it in scratch (over 400 bytes a lane), and the values
     that the code takes for uniform are then spilled under lane masks."""
-    sizes = {}
-    for block in notes.split("  - .agpr_count")[1:]:
-        name = re.search(r"\.name:\s+(\S+)", block[block.index(".max_flat_workgroup_size"):]).group(1)
-        sizes[name] = int(re.search(r"\.private_segment_fixed_size:\s+(\d+)", block).group(1))
+    sizes = kernels(notes, "private_segment_fixed_size")
     search = {k: v for k, v in sizes.items() if "k_search" in k}
     assert len(search) > 50
     assert {k: v for k, v in search.items() if v > 32} == {}
@@ -56,5 +62,15 @@ def test_search_state_is_not_in_scratch(notes):
 
 def test_every_device_function_is_inlined(notes):
     functions = {m.group(1) for m in re.finditer(r" FUNC\s+\S+\s+\S+\s+\S+\s+(\S+)", notes)}
-    kernels = {m.group(1) for m in re.finditer(r"\.name:\s+(_Z\S+)", notes)}
-    assert kernels and functions - kernels == set()
+    names = set(kernels(notes, "vgpr_count"))
+    assert names and functions - names == set()
+
+
+@pytest.mark.parametrize("kernel,waves", [("5k_rowILi1ELi1E", 8), ("5k_rowILi1ELi2E", 8), ("5k_rowILi1ELi3E", 7),
+                                          ("5k_rowILi1ELi4E", 5), ("5k_csrILi1ELi2E", 7), ("5k_csrILi1ELi3E", 5),
+                                          ("5k_csrILi1ELi4E", 4)])
+def test_filtered_uint8_kernels_keep_their_waves(notes, kernel, waves):
+    """The Gram tiles of the filtered prune do not take the searches' waves (per SIMD, by registers)."""
+    counts = [v for k, v in kernels(notes, "vgpr_count").items() if kernel in k]
+    assert len(counts) == 1
+    assert 512 // (-(-counts[0] // 8) * 8) >= waves
