@@ -210,10 +210,18 @@ constexpr uint32_t kQBoundIters = 0x1u;  // first iteration: random graph, HBM-b
 // 45.5.
 // Either way the last iteration takes it only when the iteration before it
 // computed more than kQBoundLastMinDist candidate distances per expansion.
+// With long candidate rows the prune reaches fewer of its pairs, and data without
+// clusters can fall short of kDenseFrac; more than kNewFrac of an expanded row's
+// neighbours being new in the iterations between tells it there (R 64: 0.41-0.61
+// without clusters, 0.17-0.23 in the clustered builds that need as many distances
+// in the end). Last search of 353k x 78 fp32 (L 84, C 77) 30.1 ms without the bound,
+// 19.8 with it, of 200k x 96 (L 150, C 100) 23.5 and 16.8, of 1M x 96 (R 48, C 90)
+// 125.7 and 81.8; of 4M x 64 around 64 centers 249 and 296.
 constexpr double kDenseFrac = 0.25;
 constexpr double kDenseMinBytes = 4.0 * (1 << 20);  // one XCD's L2
 constexpr double kClusteredMinBytes = 3e9;
 constexpr double kQBoundLastMinDist = 24.0;
+constexpr double kNewFrac = 0.3;
 static bool qbound_iters_adaptive() {
   const char* e = std::getenv("DANCE_QBOUND_ITERS");
   return !(e && e[0]);
@@ -851,7 +859,11 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   uint32_t q_iters = qbound_iters();  // later iterations' bits may be set on the way (kDenseFrac)
   bool dense = false;
   const bool fewer_lines = qb.rows && pick_cpl(rows.rs.nch) > qb.groups;  // of a code row than of its row
-  const double row_bytes = (double)rows.rs.stride16 * 16.0 * (double)N;
+  // what one build's searches gather from: of a group, its largest build's rows (50
+  // builds of 4000 x 96 fp32 without clusters 50.0 ms; 54.4 with the bound in every
+  // iteration, as their 77 MB together would have it)
+  const uint32_t most_rows = group ? *std::max_element(group->rows.begin(), group->rows.end()) : N;
+  const double row_bytes = (double)rows.rs.stride16 * 16.0 * (double)most_rows;
   const uint32_t ib_iters = insert_bound_iters();
   uint32_t q_prune_iters = qbound_prune_iters();  // iteration 1's bit may be set after iteration 0
   const uint32_t iters = vamana_iters();
@@ -860,6 +872,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   const uint32_t p_rank = prune_rank_iters(rows.dtype);
   DCHECK(record(e_init, s));
 
+  VCounters after_first{};  // cumulative counters after iteration 0
   VCounters before_last{};  // cumulative counters after iteration iters - 3 (zero if none)
   DevBuf snaps;  // timed builds: iters cumulative counter snapshots
   if (timed) DCHECK(snaps.alloc(sizeof(VCounters) * kMaxIters));
@@ -905,6 +918,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
       const double pairs = (double)g.C * (double)(g.C > 0 ? g.C - 1 : 0) / 2.0;
       dense = (double)h.prune_bound_checks > kDenseFrac * pairs * (double)g.N;
       if (dense && qbound_prune_adaptive()) q_prune_iters |= 2u;
+      after_first = h;
       if (dense && fewer_lines && qbound_iters_adaptive() && row_bytes > kDenseMinBytes)
         q_iters |= ((1u << (iters - 1)) - 1u) & ~1u;  // the iterations between the first and the last
     }
@@ -923,7 +937,11 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
         const double cand = (double)(h.search_dist + h.bound_skips) -
                             (double)(before_last.search_dist + before_last.bound_skips);
         const double exps = (double)(h.expansions - before_last.expansions);
-        if (cand > kQBoundLastMinDist * exps && (dense || row_bytes >= kClusteredMinBytes))
+        const double cand1 = (double)(before_last.search_dist + before_last.bound_skips) -
+                             (double)(after_first.search_dist + after_first.bound_skips);
+        const double exps1 = (double)(before_last.expansions - after_first.expansions);
+        const bool many_new = iters > 3 && row_bytes > kDenseMinBytes && cand1 > kNewFrac * R * exps1;
+        if (cand > kQBoundLastMinDist * exps && (dense || many_new || row_bytes >= kClusteredMinBytes))
           q_iters |= 1u << (iters - 1);
       }
     }

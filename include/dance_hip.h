@@ -48,7 +48,8 @@ typedef struct DanceKernelProfile {
      * a quarter of the candidate pairs) whose rows exceed 4 MiB the iterations
      * up to the last; the last one also takes it when the iteration before it
      * computed more than 24 candidate distances per expansion and the data is
-     * of that kind or its rows exceed 3 GB. */
+     * of that kind, the iterations between computed more than 0.3 R, or its
+     * rows exceed 3 GB. */
     uint64_t bound_checks, bound_skips;
     /* The same bound in RobustPrune: pairs tested, and pairs it proved far
      * enough that the candidate survives (DANCE_QBOUND_PRUNE_ITERS selects

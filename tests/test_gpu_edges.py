@@ -256,3 +256,24 @@ def test_dense_rule_compares_lines(dim, middle, monkeypatch):
             assert [c > 0 for c in checks[1:3]] == [middle, middle]
             assert middle or checks[3] == 0
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+# the last iteration's bound on data without clusters whose long candidate rows
+# keep the prune below a quarter of its pairs: most of a row's neighbours are new
+@pytest.mark.parametrize("centers,last", [(0, True), (40, False)])
+def test_last_iteration_bound_with_long_candidate_rows(centers, last, monkeypatch):
+    import torch
+    n, dim, R = 20_000, 96, 48
+    x = torch.from_numpy(rows("f32", n, dim, centers=centers)).cuda()
+    out = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv("DANCE_QBOUND", "0")
+        g = torch.empty((n, R), dtype=torch.int32, device="cuda")
+        d = torch.empty((n,), dtype=torch.int32, device="cuda")
+        D.vamana_build_resident(x.data_ptr(), D.DTYPE_F32, n, dim, R, 100, 90, 40, g.data_ptr(), d.data_ptr())
+        out.append((g, d))
+        if not off:
+            checks = D.last_kernel_profile()["bound_checks_iter"]
+            assert [c > 0 for c in checks[:4]] == [True, False, False, last]
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
