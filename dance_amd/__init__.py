@@ -167,7 +167,7 @@ EXPORTS = [
     "gpu_vamana_get_last_medoid", "gpu_vamana_get_last_stats",
     "gpu_vamana_vnew2_get_last_medoid", "gpu_vamana_vnew2_get_last_stats",
     "dance_vamana_build_resident", "dance_vamana_build_resident_noalloc", "dance_get_last_kernel_profile",
-    "dance_set_profile", "dance_get_profile",
+    "dance_set_profile", "dance_get_profile", "dance_release_memory",
     "dance_stage_distances", "dance_stage_qbound", "dance_stage_insert_bound", "dance_stage_medoid",
     "dance_stage_init", "dance_stage_search",
     "dance_stage_reverse_merge", "dance_stage_prune", "dance_stage_sort_pairs", "dance_stage_scan",
@@ -294,6 +294,8 @@ def lib() -> C.CDLL:
         L.dance_filtered_build_resident.restype = i32
         L.dance_get_last_filtered_profile.argtypes = [C.POINTER(DanceFilteredProfile)]
         L.dance_get_last_filtered_profile.restype = None
+        L.dance_release_memory.argtypes = []
+        L.dance_release_memory.restype = i32
         search_args = [vp, i32, u32, u32, vp, vp, u32, _u32p, u32, vp, u32, u32, u32, vp, vp, vp, _u32p, _f32p]
         for name in ("dance_search", "dance_search_resident"):
             getattr(L, name).argtypes = search_args
@@ -672,6 +674,12 @@ def _search(resident, data_p, dtype, N, dim, graph_p, degree_p, R, starts, queri
                 queries.ctypes.data, nq, k, L, *ptrs, _p(ids, C.c_uint32), _p(dists, C.c_float))
     _check(rc, "dance_search")
     return ids, dists
+
+
+def release_memory() -> None:
+    """Gives back the device and pinned memory that the library keeps between
+    calls (see dance_release_memory in include/dance_hip.h)."""
+    _check(lib().dance_release_memory(), "dance_release_memory")
 
 
 def last_search_stats() -> dict:

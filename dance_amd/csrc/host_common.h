@@ -186,8 +186,9 @@ struct DevBuf {
 // The calls of 16 to 10k queries take 0.15 ms less with it, a build of 100k x 96
 // 2.4 ms (58.3 -> 55.9).
 // Idle slabs are bounded by kKeepBytes over all GPUs, the oldest freed first,
-// and all of a GPU's are freed when an allocation on it fails; a call that
-// needs more than kLeaseBytes allocates for itself. A lease goes back only
+// and all of a GPU's are freed when an allocation on it fails, or by the caller
+// (dance_release_memory); a call that needs more than kLeaseBytes allocates for
+// itself. A lease goes back only
 // after the call's work has completed (CallLease), so the next call, on
 // whatever thread, may write the slab at once.
 // ---------------------------------------------------------------------------
@@ -246,6 +247,13 @@ class CallPool {
     kept_ += s.bytes;
     while (kept_ > kKeepBytes) free_locked(0);
   }
+  // Gives everything idle back (dance_release_memory).
+  void release() {
+    std::lock_guard<std::mutex> lk(mu_);
+    while (!idle_.empty()) free_locked(0);
+    for (const StreamSet& st : streams_) destroy(st);
+    streams_.clear();
+  }
   // Frees the idle slabs of a GPU (an allocation on it failed).
   bool drop(int dev) {
     std::lock_guard<std::mutex> lk(mu_);
@@ -276,13 +284,16 @@ class CallPool {
         return;
       }
     }
+    destroy(st);
+  }
+
+ private:
+  static void destroy(const StreamSet& st) {
     if (st.e0) (void)hipEventDestroy(st.e0);
     if (st.e1) (void)hipEventDestroy(st.e1);
     if (st.host) (void)hipHostFree(st.host);
     (void)hipStreamDestroy(st.s);
   }
-
- private:
   static constexpr size_t kGrain = 2ull << 20;
   void free_locked(size_t i) {
     kept_ -= idle_[i].bytes;
@@ -491,18 +502,30 @@ inline int launch_cells_u8(const Rows& rows, uint32_t N, const uint32_t* piv, ui
 // threads each own a pinned buffer and a stream and move whole chunks, so
 // the DMA of one chunk overlaps the host-side copy of another. Synchronous:
 // returns after every byte has arrived. The pinned buffers are allocated on
-// first use and kept for the life of the process (kCopyThreads x kCopyChunk
+// first use and kept until dance_release_memory (kCopyThreads x kCopyChunk
 // bytes); copies below two chunks take one plain hipMemcpy.
 constexpr size_t kCopyChunk = 32ull << 20;
 constexpr unsigned kCopyThreads = 8;
 
+inline std::mutex g_copy_mu;   // held by a staged copy: concurrent ones would share the staging buffers
+inline std::mutex g_stage_mu;  // g_stage
+inline void* g_stage[kCopyThreads] = {};
+
 inline int pinned_stage(unsigned k, void** out) {
-  static std::mutex mu;
-  static void* bufs[kCopyThreads] = {};
-  std::lock_guard<std::mutex> lock(mu);
-  if (!bufs[k]) DHIP(hipHostMalloc(&bufs[k], kCopyChunk, hipHostMallocPortable));
-  *out = bufs[k];
+  std::lock_guard<std::mutex> lock(g_stage_mu);
+  if (!g_stage[k]) DHIP(hipHostMalloc(&g_stage[k], kCopyChunk, hipHostMallocPortable));
+  *out = g_stage[k];
   return 0;
+}
+
+// Frees the staging buffers (no copy is running while g_copy_mu is held).
+inline void release_stages() {
+  std::lock_guard<std::mutex> copies(g_copy_mu);
+  std::lock_guard<std::mutex> lock(g_stage_mu);
+  for (void*& p : g_stage) {
+    if (p) (void)hipHostFree(p);
+    p = nullptr;
+  }
 }
 
 inline int copy_pageable(void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
@@ -514,8 +537,7 @@ inline int copy_pageable(void* dst, const void* src, size_t bytes, hipMemcpyKind
   DHIP(hipGetDevice(&dev));
   const size_t chunks = (bytes + kCopyChunk - 1) / kCopyChunk;
   const unsigned T = (unsigned)std::min<size_t>(kCopyThreads, chunks);
-  static std::mutex copy_mu;  // concurrent copies would share the staging buffers
-  std::lock_guard<std::mutex> lock(copy_mu);
+  std::lock_guard<std::mutex> lock(g_copy_mu);
   std::atomic<size_t> next{0};
   std::atomic<int> failed{0};
   auto worker = [&](unsigned t) {

@@ -257,6 +257,12 @@ using namespace dance;
 
 extern "C" {
 
+int dance_release_memory(void) {
+  dance::CallPool::get().release();
+  dance::release_stages();
+  return 0;
+}
+
 int dance_search(const void* h_data, int dtype, uint32_t num_points, uint32_t dim, const uint32_t* h_graph,
                  const uint32_t* h_degree, uint32_t R, const uint32_t* starts, uint32_t num_starts,
                  const void* h_queries, uint32_t num_queries, uint32_t k, uint32_t L,

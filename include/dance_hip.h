@@ -108,6 +108,16 @@ int dance_vamana_build_resident_noalloc(const void *d_data, int dtype, uint32_t 
                                         uint32_t R, uint32_t L, uint32_t C, uint32_t STEPS, uint32_t *d_graph,
                                         uint32_t *d_degree);
 
+/* What the library keeps between calls, on top of the scratch array above: at
+ * most 512 MiB of device memory over all GPUs and four streams with 16 MiB of
+ * pinned host memory each (the calls' leased buffers), and 256 MiB of pinned
+ * staging buffers once a copy of 64 MiB or more ran. dance_release_memory gives
+ * back whatever no running call uses; the next calls allocate again. A program
+ * calls it where another allocator needs the memory, and before
+ * hipDeviceReset, which would leave the library with dead streams and
+ * buffers. Returns 0. */
+int dance_release_memory(void);
+
 /* Stitched build (reference: apps/utils/gpu_stitched_vamana_index.cpp,
  * label loop :276-341). For each label l in order 0..num_labels-1 with points
  * label_points[label_offsets[l] .. label_offsets[l+1]) (ascending ids), a

@@ -277,3 +277,26 @@ def test_last_iteration_bound_with_long_candidate_rows(centers, last, monkeypatc
             checks = D.last_kernel_profile()["bound_checks_iter"]
             assert [c > 0 for c in checks[:4]] == [True, False, False, last]
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+# what the calls keep is given back on request, and the next calls run
+def test_release_memory():
+    import torch
+    n, dim, R = 100_000, 96, 16
+    x = rows("f32", n, dim)
+    rng = np.random.default_rng(0)
+    graph, degree = rng.integers(0, n, (n, R), dtype=np.uint32), np.full(n, R, np.uint32)
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    D.release_memory()
+    before = used()
+    want = D.search(x, graph, degree, 0, x[:20], 10, 40)  # host rows: leases all of them
+    assert used() - before > n * dim * 4
+    D.release_memory()
+    assert used() - before < 16 << 20
+    got = D.search(x, graph, degree, 0, x[:20], 10, 40)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
