@@ -215,7 +215,8 @@ class CallPool {
     static CallPool* pool = new CallPool;  // never destroyed: the runtime may be gone before a static's end
     return *pool;
   }
-  int take(size_t need, int dev, Slab* out) {
+  // A slab of at least `need` bytes; false where the GPU has none to give in one piece.
+  bool take(size_t need, int dev, Slab* out) {
     std::lock_guard<std::mutex> lk(mu_);
     size_t best = idle_.size();
     for (size_t i = 0; i < idle_.size(); ++i)
@@ -225,21 +226,20 @@ class CallPool {
       *out = idle_[best];
       kept_ -= out->bytes;
       idle_.erase(idle_.begin() + (ptrdiff_t)best);
-      return 0;
+      return true;
     }
     const size_t bytes = (need + kGrain - 1) / kGrain * kGrain;
     void* p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
       (void)hipGetLastError();
       drop_locked(dev);
-      const hipError_t e = hipMalloc(&p, bytes);
-      if (e != hipSuccess) {
-        std::fprintf(stderr, "[dance_hip] hipMalloc(%zu) failed: %s\n", bytes, hipGetErrorString(e));
-        return -1;
+      if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
       }
     }
     *out = Slab{p, bytes, dev};
-    return 0;
+    return true;
   }
   void give(const Slab& s) {
     std::lock_guard<std::mutex> lk(mu_);
@@ -339,18 +339,20 @@ struct CallLease {
     opened = true;
     prev = tl_arena;
     DCHECK(CallPool::get().take_stream(dev, &set));
-    if (need <= kLeaseBytes) {
-      DCHECK(CallPool::get().take(need, dev, &slab));
+    if (need <= kLeaseBytes && CallPool::get().take(need, dev, &slab)) {
       arena = Arena{static_cast<char*>(slab.p), slab.bytes, 0, true};
       tl_arena = &arena;
     }
     return 0;
   }
   hipStream_t stream() const { return set.s; }
-  int host(char** out) {
-    if (!set.host) DHIP(hipHostMalloc(&set.host, kCallHostBytes, hipHostMallocPortable));
-    *out = static_cast<char*>(set.host);
-    return 0;
+  // kCallHostBytes of pinned memory, or nullptr where there is none.
+  char* host() {
+    if (!set.host && hipHostMalloc(&set.host, kCallHostBytes, hipHostMallocPortable) != hipSuccess) {
+      (void)hipGetLastError();
+      set.host = nullptr;
+    }
+    return static_cast<char*>(set.host);
   }
   void done() { finished = true; }
   ~CallLease() {

@@ -93,22 +93,9 @@ int run_search(const SearchIn& in) {
   const size_t b_in = b_starts + b_off + b_qlab + b_q + arena_bytes(kCtrBytes);
   const size_t b_res = arena_bytes((size_t)in.nq * in.k * 4);
   const uint32_t ntotal = filt ? in.label_offsets[in.N] : 0u;
-  size_t need = b_in + 2 * b_res + host_rows_bytes(in.dtype, in.dtype, in.nq, in.dim) +
-                host_rows_bytes(in.dtype, in.dtype, in.N, in.dim);
-  if (!in.graph_on_device) need += arena_bytes((size_t)in.N * in.R * 4) + arena_bytes((size_t)in.N * 4);
-  if (filt) need += arena_bytes((size_t)(in.N + 1) * 4) + arena_bytes((size_t)std::max(1u, ntotal) * 4);
-  CallLease lease;
-  DCHECK(lease.open(need));
-  const hipStream_t s = lease.stream();
+  CallLease lease;  // opened below, when what it holds is known
   Rows base, qr;
   const size_t stride = row_layout(base, in.dtype, in.N, in.dim);
-  const void* packed = in.data;  // the base rows in device memory, as the caller packed them
-  DevBuf up;
-  if (!in.data_on_device) {
-    DCHECK(up.alloc(row_bytes * in.N));
-    DCHECK(copy_pageable(up.p, in.data, row_bytes * in.N, hipMemcpyHostToDevice));
-    packed = up.p;
-  }
   // Rows that fill the kernels' chunk group are read as they are. Others are
   // copied into padded rows, or read packed when the call gathers fewer rows
   // than that copy would touch: a query gathers about kGathersPerL rows per
@@ -117,10 +104,29 @@ int run_search(const SearchIn& in) {
   // 200 uint8 0.66 / 1.35 and 0.74 / 0.99 ms; 10k of L 100 over 500k x 100 fp32
   // 2.57 / 3.53 and 3.54 / 3.95 ms (packed rows straddle one cache line more, and
   // their last chunk takes more instructions).
-  const bool whole = stride == row_bytes && (reinterpret_cast<uintptr_t>(packed) & 15u) == 0;
+  // (Uploaded rows start at an allocation, which is aligned.)
+  const bool whole =
+      stride == row_bytes && (!in.data_on_device || (reinterpret_cast<uintptr_t>(in.data) & 15u) == 0);
   const int ps = pick_ps(in.L);
   const bool in_place = !whole && pick_cpl(base.rs.nch) <= kPackedCpl && ps <= kPackedPs &&
                         (uint64_t)in.nq * in.L * kGathersPerL < in.N;
+  // The lease holds what this call allocates and no more: 16 queries over 200k
+  // resident rows lease 2 MiB, 10k queries of 96 dimensions 8 MiB.
+  size_t need = b_in + 2 * b_res;
+  if (stride != row_bytes) need += arena_bytes(stride * in.nq);
+  if (!in.data_on_device) need += arena_bytes(row_bytes * in.N);
+  if (!whole && !in_place) need += arena_bytes(stride * in.N);
+  if (!in.graph_on_device) need += arena_bytes((size_t)in.N * in.R * 4) + arena_bytes((size_t)in.N * 4);
+  if (filt) need += arena_bytes((size_t)(in.N + 1) * 4) + arena_bytes((size_t)std::max(1u, ntotal) * 4);
+  DCHECK(lease.open(need));
+  const hipStream_t s = lease.stream();
+  const void* packed = in.data;  // the base rows in device memory, as the caller packed them
+  DevBuf up;
+  if (!in.data_on_device) {
+    DCHECK(up.alloc(row_bytes * in.N));
+    DCHECK(copy_pageable(up.p, in.data, row_bytes * in.N, hipMemcpyHostToDevice));
+    packed = up.p;
+  }
   if (whole)
     base.rs.rows = static_cast<const uint4*>(packed);
   else if (!in_place)
@@ -139,9 +145,9 @@ int run_search(const SearchIn& in) {
   // is still written. With the leased memory and stream: 16 queries of L 50 over
   // 200k x 96 0.40 -> 0.25 ms (kernel 0.22), 10k of L 100 over 1M x 96 2.85 ->
   // 2.69 ms (kernel 2.42), 1k filtered over 100k 0.87 -> 0.66 ms (kernel 0.50).
-  char* pin = nullptr;
-  DCHECK(lease.host(&pin));
-  if (b_in <= kCallHostBytes / 2) {
+  // Without pinned memory the copies are plain ones.
+  char* const pin = lease.host();
+  if (pin && b_in <= kCallHostBytes / 2) {
     size_t sent = 0, at = 0;
     auto put = [&](const void* src, size_t bytes, size_t room) -> int {
       for (size_t o = 0; o < bytes; o += kSendBytes) {  // the first pieces travel while the next are written
@@ -227,7 +233,7 @@ int run_search(const SearchIn& in) {
   unsigned long long c3[kCtrBytes / 8];
   const size_t res_bytes = (size_t)in.nq * in.k * 4;
   const size_t b_out = arena_bytes(kCtrBytes) + 2 * b_res;
-  if (b_out <= kCallHostBytes / 2) {
+  if (pin && b_out <= kCallHostBytes / 2) {
     char* const out = pin + kCallHostBytes / 2;
     DHIP(hipMemcpyAsync(out, d_ctr, b_out, hipMemcpyDeviceToHost, s));
     DHIP(hipStreamSynchronize(s));

@@ -300,3 +300,25 @@ def test_release_memory():
     assert used() - before < 16 << 20
     got = D.search(x, graph, degree, 0, x[:20], 10, 40)
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+
+
+# a search leases what it allocates: queries over large resident rows hold no copy
+# of them, be they read as they are (96 dimensions) or packed (97)
+@pytest.mark.parametrize("dim", [96, 97])
+def test_small_search_leases_little(dim):
+    import torch
+    n, R = 200_000, 16
+    x = torch.rand(n, dim, device="cuda")
+    g = torch.randint(0, n, (n, R), dtype=torch.int32, device="cuda")
+    d = torch.full((n,), R, dtype=torch.int32, device="cuda")
+    q = np.ones((16, dim), np.float32)
+
+    def used():
+        torch.cuda.synchronize()
+        free, total = torch.cuda.mem_get_info()
+        return total - free
+
+    D.release_memory()
+    before = used()
+    D.search_resident(x.data_ptr(), D.DTYPE_F32, n, dim, g.data_ptr(), d.data_ptr(), R, 0, q, 10, 50)
+    assert used() - before < 16 << 20
