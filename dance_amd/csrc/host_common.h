@@ -339,6 +339,14 @@ struct CallLease {
     opened = true;
     prev = tl_arena;
     DCHECK(CallPool::get().take_stream(dev, &set));
+    // A call waits for its stream, which a stream capture forbids: asked of the
+    // idle stream, so that such a call ends before it launches anything.
+    if (hipStreamSynchronize(set.s) != hipSuccess) {
+      (void)hipGetLastError();
+      std::fprintf(stderr, "[dance_hip] a call cannot run during a stream capture\n");
+      finished = true;
+      return -1;
+    }
     if (need <= kLeaseBytes && CallPool::get().take(need, dev, &slab)) {
       arena = Arena{static_cast<char*>(slab.p), slab.bytes, 0, true};
       tl_arena = &arena;
@@ -358,7 +366,8 @@ struct CallLease {
   ~CallLease() {
     if (!opened) return;
     tl_arena = prev;
-    if (!finished) (void)hipDeviceSynchronize();
+    // work that could not be waited for may still use the slab and the stream: neither goes back
+    if (!finished && hipDeviceSynchronize() != hipSuccess) return;
     if (slab.p) CallPool::get().give(slab);
     CallPool::get().give_stream(set);
   }

@@ -322,3 +322,46 @@ def test_small_search_leases_little(dim):
     before = used()
     D.search_resident(x.data_ptr(), D.DTYPE_F32, n, dim, g.data_ptr(), d.data_ptr(), R, 0, q, 10, 50)
     assert used() - before < 16 << 20
+
+
+# a call during a stream capture ends before it launches anything (it would wait
+# for its stream, which a capture forbids), and the next call runs
+CAPTURE = """
+import ctypes
+import numpy as np
+import dance_amd as D
+D.lib()
+hip = ctypes.CDLL("libamdhip64.so")
+n, dim, R = 2000, 96, 32
+x = np.random.default_rng(0).standard_normal((n, dim)).astype(np.float32)
+r = D.vamana_build(x, R, 64, 48, 32)
+def build():
+    return D.vamana_build(x, R, 64, 48, 32)
+def search():
+    return D.search(x, r.graph, r.degree, r.medoid, x[:4], 5, 20)[0]
+want = search()
+stream, graph = ctypes.c_void_p(), ctypes.c_void_p()
+assert hip.hipStreamCreate(ctypes.byref(stream)) == 0
+for call in (build, search):
+    assert hip.hipStreamBeginCapture(stream, 0) == 0  # global: no thread may wait
+    try:
+        call()
+        refused = False
+    except D.BuildError:
+        refused = True
+    hip.hipStreamEndCapture(stream, ctypes.byref(graph))
+    hip.hipGetLastError()
+    assert refused
+assert np.array_equal(search(), want) and np.array_equal(build().graph, r.graph)
+print("done")
+"""
+
+
+def test_calls_during_a_capture():
+    import os
+    import subprocess
+    import sys
+    r = subprocess.run([sys.executable, "-c", CAPTURE], cwd=os.path.dirname(os.path.dirname(D.__file__)), timeout=100,
+                       capture_output=True, text=True)
+    assert r.returncode == 0 and "done" in r.stdout, r.stderr[-2000:]
+    assert r.stderr.count("cannot run during a stream capture") == 2, r.stderr[-2000:]
