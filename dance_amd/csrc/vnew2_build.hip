@@ -156,16 +156,19 @@ static uint32_t wave_grid(uint32_t n) { return (n + kWavesPerBlock - 1) / kWaves
 // of 8 workgroups, 2-D beyond 2^32 work-items (grid_dims).
 static dim3 xcd_grid(uint32_t n) { return grid_dims(wave_grid(n), kBlock, 8); }
 
-// nseg > 0: the builds of sg, nc and ns the most one of them takes.
+// Workgroups of a build's medoid.
+static uint32_t medoid_groups(const Rows& rows, uint32_t n) {
+  const uint32_t kc = medoid_cands(pick_cpl(rows.rs.nch));
+  return (std::min(kMedoidCandidates, n) + kc - 1) / kc;
+}
+// nseg > 0: the builds of sg, with `groups` workgroups in all, nc and ns the most one of them takes.
 static int launch_medoid(const Rows& rows, hipStream_t s, float* d_scores, uint32_t* d_cands, uint32_t nc,
-                         uint32_t ns, Segments sg = {}, uint32_t nseg = 0) {
+                         uint32_t ns, uint32_t groups, Segments sg = {}, uint32_t nseg = 0) {
   const int cpl = pick_cpl(rows.rs.nch);
   return with_dt_cpl(rows.kind(), cpl, [&](auto dt, auto c) {
     constexpr int CPL = decltype(c)::value;
-    constexpr uint32_t KC = medoid_cands(CPL);
-    hipLaunchKernelGGL((k_medoid<decltype(dt)::value, CPL>), dim3((nc + KC - 1) / KC, std::max(nseg, 1u)),
-                       dim3(64 * medoid_waves(CPL)), medoid_lds_bytes(CPL), s, rows.rs, rows.N, nc, ns, d_scores,
-                       d_cands, sg);
+    hipLaunchKernelGGL((k_medoid<decltype(dt)::value, CPL>), dim3(groups), dim3(64 * medoid_waves(CPL)),
+                       medoid_lds_bytes(CPL), s, rows.rs, rows.N, nc, ns, d_scores, d_cands, sg, nseg);
     DHIP(hipGetLastError());
     return 0;
   });
@@ -803,10 +806,11 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
   std::vector<uint4> hseg;
   if (group) {
     const uint32_t nb = (uint32_t)group->rows.size();
-    uint32_t lo = 0, most = 0;
+    uint32_t lo = 0, most = 0, groups = 0;
     for (uint32_t m : group->rows) {
-      hseg.push_back(make_uint4(lo, m, lo, 0u));
+      hseg.push_back(make_uint4(lo, m, lo, groups));
       lo += m;
+      groups += medoid_groups(rows, m);
       most = std::max(most, m);
     }
     if (lo != N || nb < 2) return -1;
@@ -819,7 +823,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     DHIP(hipMemcpyAsync(seg.p, hseg.data(), nb * sizeof(uint4), hipMemcpyHostToDevice, s));
     hipLaunchKernelGGL(k_seg_rows, dim3((N + 255) / 256), dim3(256), 0, s, sg, nb, N, seg_of.as<uint32_t>());
     DHIP(hipGetLastError());
-    DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns, sg, nb));
+    DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns, groups, sg, nb));
     hipLaunchKernelGGL(k_seg_start, dim3(nb), dim3(64), 0, s, scores.as<const float>(), cands.as<const uint32_t>(), nc,
                        sg);
     DHIP(hipGetLastError());
@@ -828,7 +832,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     const uint32_t nc = std::min(kMedoidCandidates, N), ns = std::min(kMedoidSamples, N);
     DCHECK(scores.alloc(nc * 4));
     DCHECK(cands.alloc(nc * 4));
-    DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns));
+    DCHECK(launch_medoid(rows, s, scores.as<float>(), cands.as<uint32_t>(), nc, ns, medoid_groups(rows, N)));
     float hs[kMedoidCandidates];
     uint32_t hc[kMedoidCandidates];
     DHIP(hipMemcpyAsync(hs, scores.p, nc * 4, hipMemcpyDeviceToHost, s));
@@ -2033,7 +2037,7 @@ int dance_stage_medoid(const void* h_data, int dtype, uint32_t N, uint32_t dim, 
   DevBuf sc, ca;
   DCHECK(sc.alloc(nc * 4));
   DCHECK(ca.alloc(nc * 4));
-  DCHECK(launch_medoid(cx.rows, cx.s, sc.as<float>(), ca.as<uint32_t>(), nc, ns));
+  DCHECK(launch_medoid(cx.rows, cx.s, sc.as<float>(), ca.as<uint32_t>(), nc, ns, medoid_groups(cx.rows, N)));
   std::vector<float> hs(nc);
   std::vector<uint32_t> hc(nc);
   DCHECK(down(hs.data(), sc.p, nc * 4, cx.s));

@@ -390,7 +390,8 @@ __device__ __forceinline__ uint32_t init_neighbor(uint32_t node, uint32_t i, uin
 // build's own size and ids (the random graph and seeds, the entry point) is
 // computed from the row's build; the rest sees one graph.
 struct Segments {
-  uint4* seg = nullptr;          // per build: first row, rows, entry point, 0; nullptr: one build
+  // per build: first row, rows, entry point, first workgroup of its medoid; nullptr: one build
+  uint4* seg = nullptr;
   const uint32_t* of = nullptr;  // per row: its build
   __device__ __forceinline__ uint4 at(uint32_t node) const { return seg[of[node]]; }
 };
@@ -2283,22 +2284,36 @@ constexpr size_t medoid_lds_bytes(int cpl) { return (size_t)medoid_cands(cpl) * 
 
 template <int DT, int CPL>
 __global__ __launch_bounds__(64 * medoid_waves(CPL)) void k_medoid(RowSet rs, uint32_t N, uint32_t nc, uint32_t ns,
-                                                              float* scores, uint32_t* cands, Segments sg) {
-  if (sg.seg) {  // grid.y: the builds; nc and ns are the most one of them takes, and the scores' stride is nc
-    const uint4 b = sg.seg[blockIdx.y];
-    scores += (size_t)blockIdx.y * nc;
-    cands += (size_t)blockIdx.y * nc;
+                                                              float* scores, uint32_t* cands, Segments sg,
+                                                              uint32_t nseg) {
+  uint32_t group = blockIdx.x;
+  if (sg.seg) {
+    // The builds' workgroups follow each other (as many as each has candidates
+    // for: with the most of any build for all of them, labels of mixed sizes
+    // launched up to 256 workgroups a label that returned at once). nc and ns are
+    // the most one of them takes, and the scores' stride is nc.
+    uint32_t a = 0, e = nseg;  // the last build that starts at or before this workgroup is in [a, e)
+    while (e - a > 1u) {
+      const uint32_t c = (a + e) / 2u;
+      if (sg.seg[c].w <= group)
+        a = c;
+      else
+        e = c;
+    }
+    const uint4 b = sg.seg[a];
+    group -= b.w;
+    scores += (size_t)a * nc;
+    cands += (size_t)a * nc;
     rs.rows += (size_t)uni_u(b.x) * rs.stride16;
     N = uni_u(b.y);
     nc = min(nc, N);
     ns = min(ns, N);
-    if (blockIdx.x * medoid_cands(CPL) >= nc) return;
   }
   constexpr uint32_t KC = medoid_cands(CPL);
   extern __shared__ uint32_t smem[];
   float* dist = reinterpret_cast<float*>(smem);  // KC x kMedoidMaxSamples
   const uint32_t w = wave_index(), lane = lane_id(), grp = lane >> 3, sub = lane & 7u;
-  const uint32_t c0 = blockIdx.x * KC;
+  const uint32_t c0 = group * KC;
   uint32_t c[KC];
   uint4 cv[KC][CPL];
   uint32_t sq[KC];
