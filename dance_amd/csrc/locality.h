@@ -92,6 +92,13 @@ __global__ __launch_bounds__(kCellsBlock) void k_cells(RowSet rs, uint32_t N, co
   }
 }
 
+// a = s^2 sum(q^2) of a code row from its header {s, r, lo, hi} (lo is a - r^2 up
+// to the bound's slack); 0 for rows without codes, whose r is infinite.
+__device__ __forceinline__ float code_norm(const uint4& h) {
+  const float r = __uint_as_float(h.y), lo = __uint_as_float(h.z);
+  return r < __builtin_inff() ? __builtin_fmaf(r, r, lo) : 0.0f;
+}
+
 // Nearest pivots on the matrix cores, for code rows (U8 = false, 128 bytes) and
 // uint8 rows of STEPS x 32 bytes (U8 = true): one wave per 32 vertices, int8
 // MFMA tiles of 32 pivots (rows) x 32 vertices (columns) over the row's bytes
@@ -148,7 +155,7 @@ __global__ __launch_bounds__(256) void k_cells_mfma(const uint4* __restrict__ ro
   } else if (act) {
     const uint4 h = rows[(size_t)v * stride16];
     xs = __uint_as_float(h.x);
-    xa = __uint_as_float(h.z);
+    xa = code_norm(h);
   }
   Nearest3 nb;
   for (uint32_t t0 = 0; t0 < K; t0 += 32) {
@@ -170,7 +177,7 @@ __global__ __launch_bounds__(256) void k_cells_mfma(const uint4* __restrict__ ro
     } else {
       if (lane < 32u && pok) {
         const uint4 h = rows[(size_t)pid * stride16];
-        pn_f[w][jl] = __uint_as_float(h.z);
+        pn_f[w][jl] = code_norm(h);
         ps_f[w][jl] = __uint_as_float(h.x);
       }
     }

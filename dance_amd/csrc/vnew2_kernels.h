@@ -2440,8 +2440,8 @@ __global__ __launch_bounds__(kBlock) void k_init(RowSet rs, GraphBufs g, Segment
 
 // Approximate nearest pivots for the locality schedule, from integer codes:
 // one thread per vertex, pivot codes staged in LDS 64 at a time. U8 = false
-// reads the quantized rows (header {s, r, a} + 7 chunks of int8 codes;
-// distance ~ a_x + a_p - 2 s_x s_p <q_x, q_p>); U8 = true reads uint8 rows of
+// reads the quantized rows (a header and 7 chunks of int8 codes; distance ~
+// a_x + a_p - 2 s_x s_p <q_x, q_p>, a from code_norm); U8 = true reads uint8 rows of
 // at most 8 chunks (exact squared distance from unsigned dot products). Only
 // the processing order depends on the result, never the graph.
 template <bool U8>
@@ -2475,7 +2475,7 @@ __global__ __launch_bounds__(256) void k_cells_q(const uint4* __restrict__ rows,
     } else if (act) {
       const uint4 h = r[0];
       sx = __uint_as_float(h.x);
-      ax = __uint_as_float(h.z);
+      ax = code_norm(h);
     }
   }
   Nearest3 nb;
@@ -2501,7 +2501,7 @@ __global__ __launch_bounds__(256) void k_cells_q(const uint4* __restrict__ rows,
         psc[threadIdx.x] = 1.0f;
       } else {
         const uint4 h = r[0];
-        pn[threadIdx.x] = __uint_as_float(h.z);
+        pn[threadIdx.x] = code_norm(h);
         psc[threadIdx.x] = __uint_as_float(h.x);
       }
     }
