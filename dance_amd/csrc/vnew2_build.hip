@@ -1242,6 +1242,7 @@ __global__ __launch_bounds__(kBlock) void k_pair_dist(RowSet rs, const uint32_t*
 
 // The search's bound test on explicit pairs: flag[k] = 1 when the quantized
 // bound proves dist(a[k], b[k]) >= T[k] (the querying row is a[k]).
+template <int QC>
 __global__ __launch_bounds__(kBlock) void k_qbound_pairs(QBoundSet qb, const uint32_t* __restrict__ a,
                                                          const uint32_t* __restrict__ b,
                                                          const float* __restrict__ T, uint64_t n,
@@ -1254,13 +1255,13 @@ __global__ __launch_bounds__(kBlock) void k_qbound_pairs(QBoundSet qb, const uin
     const uint64_t k = base + p + grp;
     const bool act = k < n;
     // the querying row differs per octet here, so its header is read per lane
-    const uint4* qa = qb.rows + (size_t)(act ? a[k] : 0u) * kQChunks;
+    const uint4* qa = qb.rows + (size_t)(act ? a[k] : 0u) * q_chunks(QC);
     const uint4 h = qa[0];
     const float s = __uint_as_float(h.x), r = __uint_as_float(h.y), lo = __uint_as_float(h.z);
     const QLower me = q_lower(s, r, lo, q_threshold(qb, r, act ? T[k] : 0.0f));
-    const QCodes<1> code = q_codes<1>(q_load<1>(qb, act ? a[k] : 0u, true, sub), sub);
-    const QCodes<1> bc = q_load<1>(qb, act ? b[k] : 0u, act, sub);
-    const bool rej = q_proves_reject<1>(me, code, bc);
+    const QCodes<QC> code = q_codes<QC>(q_load<QC>(qb, act ? a[k] : 0u, true, sub), sub);
+    const QCodes<QC> bc = q_load<QC>(qb, act ? b[k] : 0u, act, sub);
+    const bool rej = q_proves_reject<QC>(me, code, bc);
     if (act && sub == 0) flag[k] = rej ? 1u : 0u;
   }
 }
@@ -1951,8 +1952,9 @@ int dance_stage_distances(const void* h_data, int dtype, uint32_t N, uint32_t di
   return 0;
 }
 
-int dance_stage_qbound(const void* h_data, int dtype, uint32_t N, uint32_t dim, const uint32_t* a, const uint32_t* b,
-                       const float* T, uint64_t n, uint32_t* flags) {
+// The bound on explicit pairs, for rows whose code rows have `groups` chunk groups.
+static int stage_qbound(const void* h_data, int dtype, uint32_t N, uint32_t dim, const uint32_t* a, const uint32_t* b,
+                        const float* T, uint64_t n, uint32_t* flags, int groups) {
   if (!h_data || !a || !b || !T || !flags || N == 0 || dim == 0) return -1;
   for (uint64_t i = 0; i < n; ++i)
     if (a[i] >= N || b[i] >= N) {
@@ -1964,7 +1966,7 @@ int dance_stage_qbound(const void* h_data, int dtype, uint32_t N, uint32_t dim, 
   DevBuf qbuf, da, db, dt, dout;
   QBoundSet qb{};
   DCHECK(build_qbound(cx.rows, qbuf, cx.s, &qb));
-  if (!qb.rows || qb.groups != 1) {
+  if (!qb.rows || qb.groups != groups) {
     std::fprintf(stderr, "[dance_hip] no distance bound for this row type / width (or DANCE_QBOUND=0)\n");
     return -1;
   }
@@ -1978,13 +1980,27 @@ int dance_stage_qbound(const void* h_data, int dtype, uint32_t N, uint32_t dim, 
   DCHECK(up(dt.p, T, n * 4, cx.s));
   const uint64_t waves = (n + 63) / 64;
   if (waves) {
-    hipLaunchKernelGGL(k_qbound_pairs, dim3((uint32_t)((waves + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kBlock),
-                       0, cx.s, qb, da.as<uint32_t>(), db.as<uint32_t>(), dt.as<float>(), n, dout.as<uint32_t>());
+    auto go = [&](auto g) {
+      hipLaunchKernelGGL(k_qbound_pairs<decltype(g)::value>,
+                         dim3((uint32_t)((waves + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kBlock), 0, cx.s, qb,
+                         da.as<uint32_t>(), db.as<uint32_t>(), dt.as<float>(), n, dout.as<uint32_t>());
+    };
+    groups == 1 ? go(IC<1>{}) : go(IC<2>{});
     DHIP(hipGetLastError());
   }
   DCHECK(down(flags, dout.p, n * 4, cx.s));
   DHIP(hipStreamSynchronize(cx.s));
   return 0;
+}
+
+int dance_stage_qbound(const void* h_data, int dtype, uint32_t N, uint32_t dim, const uint32_t* a, const uint32_t* b,
+                       const float* T, uint64_t n, uint32_t* flags) {
+  return stage_qbound(h_data, dtype, N, dim, a, b, T, n, flags, 1);
+}
+
+int dance_stage_qbound_wide(const void* h_data, int dtype, uint32_t N, uint32_t dim, const uint32_t* a,
+                            const uint32_t* b, const float* T, uint64_t n, uint32_t* flags) {
+  return stage_qbound(h_data, dtype, N, dim, a, b, T, n, flags, 2);
 }
 
 int dance_stage_insert_bound(const void* h_data, int dtype, uint32_t N, uint32_t dim, const uint32_t* a,

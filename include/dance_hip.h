@@ -329,6 +329,9 @@ int dance_stage_distances(const void *h_data, int dtype, uint32_t num_points, ui
  * dist(a[i], b[i]) >= T[i]. fp32/fp16 rows of <= 112 dims; -1 otherwise. */
 int dance_stage_qbound(const void *h_data, int dtype, uint32_t num_points, uint32_t dim, const uint32_t *a,
                        const uint32_t *b, const float *T, uint64_t n, uint32_t *flags);
+/* The same for the two-group code rows of 113 to 240 dims. */
+int dance_stage_qbound_wide(const void *h_data, int dtype, uint32_t num_points, uint32_t dim, const uint32_t *a,
+                            const uint32_t *b, const float *T, uint64_t n, uint32_t *flags);
 
 /* The online insert's occlusion-pair bounds on explicit pairs (no
  * counterpart in the reference; they only skip work), with x = a[i], y = b[i]

@@ -312,3 +312,37 @@ def test_last_iteration_bound_follows_candidate_count(n, R, L, C, steps):
     assert (a["bound_checks_iter"][last] > 0) == fired
     assert f["bound_checks_iter"][last] == 0 and f["bound_checks_iter"][0] > 0
     assert all(a["bound_checks_iter"][i] == 0 for i in range(1, last))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("dim", [113, 128, 129, 191, 192, 240])
+def test_wide_bound_is_sound(dim, dtype):
+    """The two-group code rows of 113 to 240 dimensions, at the threshold and around it."""
+    x = adversarial(3000, dim, seed=dim, dtype=dtype, huge=dtype == np.float32)
+    x[100] = np.inf
+    x[101, dim - 1] = np.nan
+    a, b = pairs(3000, 20000, seed=dim + 1)
+    a = np.concatenate([a, np.full(3000, 100, np.uint32), np.full(3000, 101, np.uint32)])
+    b = np.concatenate([b, np.arange(3000, dtype=np.uint32), np.arange(3000, dtype=np.uint32)])
+    d = D.stage_distances(x, a, b)
+    odd = (a == 100) | (a == 101) | (b == 100) | (b == 101)  # non-finite rows
+    flagged = 0
+    with np.errstate(invalid="ignore", over="ignore"):
+        above = np.nextafter(d, np.float32(np.inf))
+        for T in (d, above, d * np.float32(1 + 1e-6), d * np.float32(0.999), d * np.float32(0.5), np.zeros_like(d),
+                  np.full_like(d, FMAX), np.full_like(d, 1e-38)):
+            f = D.stage_qbound(x, a, b, np.ascontiguousarray(T, np.float32), groups=2).astype(bool)
+            assert not (f & ~(d >= T)).any()
+            assert not f[odd].any()
+            flagged += int(f.sum())
+    assert not D.stage_qbound(x, a, b, above, groups=2)[np.isfinite(d)].any()
+    assert flagged > 0
+    ok = (a != b) & (a >= 100) & (b >= 100) & ~odd
+    assert D.stage_qbound(x, a[ok], b[ok], d[ok] * np.float32(0.9), groups=2).mean() > 0.9
+
+
+def test_wide_bound_takes_its_own_widths():
+    one = np.zeros(1, np.uint32)
+    for dim in (112, 241):
+        with pytest.raises(D.BuildError):
+            D.stage_qbound(np.ones((10, dim), np.float32), one, one, np.zeros(1, np.float32), groups=2)
