@@ -1359,8 +1359,9 @@ __device__ __forceinline__ uint32_t ffs128(uint64_t m0, uint64_t m1) {
 // SIMD; at 8 chunks per lane its batch of exact pairs holds 4 rows of 32
 // registers, which 3 waves leave room for (5 spilled 264 bytes and took 7.3
 // instead of 2.5 ms at 200k x 200). The variant without it fits 6 at rows of
-// up to 4 chunks per lane. Wider rows (and fp16 rows of 4 chunks per lane) get
-// no floor, so no variant spills.
+// up to 4 chunks per lane; wider rows (and fp16 rows of 4 chunks per lane) get
+// no floor. The one-group bound keeps 8 registers in scratch (36 bytes), the other
+// variants none.
 template <int DT, int CPL, int PM>
 constexpr int kRankMinWaves =
     PM != kRankExact ? (PM == kRankBound && CPL >= 8 ? 3 : 5) : (CPL < 4 || (CPL == 4 && !is_f16(DT))) ? 6 : 1;
@@ -1627,6 +1628,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
     // the rounds would make (alpha d <= d(node, j)); every pair is decided
     // before the rounds, and each candidate row is gathered once.
     constexpr uint32_t S = 4u * CPL;  // K-steps of 32 bytes over the padded row
+    // Steps in flight: all of up to 4 chunks per lane, 8 of the 32 and 64 of 8 and
+    // 16 chunks. Unrolled whole, those held every row's loads and spilled 83 and
+    // 339 registers at 5 waves; by 8 they take 57. Builds of 100k rows at R 64, L 100,
+    // C 80: 600 dims 239.2 -> 237.7 ms (101.5 -> 99.5 around 256 centers), 1100 dims
+    // 534.1 -> 519.1 (221.0 -> 208.1).
+    constexpr uint32_t kU = CPL >= 8 ? 8u : S;
     int* nrm = reinterpret_cast<int*>(hq);  // |row'|^2 by rank
     const uint32_t nt = (nvalid + 31u) >> 5;
     const uint32_t jl = lane & 31u, ih = 4u * (lane >> 5);
@@ -1687,7 +1694,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
     } else {
       for (uint32_t t = 0; t < nt; ++t) {
         int part = 0;
-#pragma unroll
+#pragma unroll kU
         for (uint32_t s = 0; s < S; ++s) part = sq4(frag(t * 32u + jl, s), part);
         put_norm(t, part);
       }
@@ -1695,7 +1702,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(kRankMin
       for (uint32_t ti = 0; ti < nt; ++ti)
         for (uint32_t tj = ti; tj < nt; ++tj) {
           v16i_t acc = {};
-#pragma unroll
+#pragma unroll kU
           for (uint32_t s = 0; s < S; ++s)
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(frag(ti * 32u + jl, s), frag(tj * 32u + jl, s), acc, 0, 0, 0);
           decide(ti, tj, acc);

@@ -74,3 +74,11 @@ def test_filtered_uint8_kernels_keep_their_waves(notes, kernel, waves):
     counts = [v for k, v in kernels(notes, "vgpr_count").items() if kernel in k]
     assert len(counts) == 1
     assert 512 // (-(-counts[0] // 8) * 8) >= waves
+
+
+def test_prune_kernels_hardly_spill(notes):
+    """Registers spilled around lane masks are reloaded under the wrong one; what is
+    left holds a few addresses (36 bytes)."""
+    sizes = {k: v for k, v in kernels(notes, "private_segment_fixed_size").items() if "k_prune" in k}
+    assert len(sizes) > 20
+    assert {k: v for k, v in sizes.items() if v > 40} == {}

@@ -365,3 +365,15 @@ def test_calls_during_a_capture():
                        capture_output=True, text=True)
     assert r.returncode == 0 and "done" in r.stdout, r.stderr[-2000:]
     assert r.stderr.count("cannot run during a stream capture") == 2, r.stderr[-2000:]
+
+
+# uint8 prunes from Gram tiles at 8 and 16 chunks per lane, candidate rows of fewer
+# and more than a wave
+@pytest.mark.parametrize("dim", [600, 1100])
+@pytest.mark.parametrize("R,C", [(16, 24), (24, 63), (48, 90)])
+def test_wide_u8_prunes(dim, R, C):
+    x = rows("u8", 700, dim)
+    og, od, om = O.vnew2_build(x, R, 48, C, 24)
+    r = D.vamana_build(x, R, 48, C, 24)
+    assert r.medoid == om
+    assert np.array_equal(r.degree, od) and np.array_equal(r.graph, og)
