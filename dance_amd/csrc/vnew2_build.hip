@@ -194,7 +194,7 @@ constexpr uint32_t kQBoundIters = 0x1u;  // first iteration: random graph, HBM-b
 // the candidate pairs in iteration 0's prune, clustered ones 7-11%) has no
 // locality for the schedule to use, so every gathered row misses L2 once the
 // rows outgrow it: every iteration then takes the bound, above kDenseMinBytes
-// of rows. Searches of iterations 1 / 2 / 3 without and with it: 20k x 96 fp32
+// of rows and per_slot candidates. Searches of iterations 1 / 2 / 3 without and with it: 20k x 96 fp32
 // 1.73 / 1.76 / 2.26 and 1.54 / 1.38 / 1.92 ms, 100k 17.1 / 18.4 / 23.6 and 11.3
 // / 10.5 / 14.7, 1M 202 / 226 / 294 and 128 / 130 / 181, 300k x 100 fp16 37.9 /
 // 42.1 / 54.4 and 28.2 / 28.8 / 38.6.
@@ -220,6 +220,26 @@ constexpr uint32_t kQBoundIters = 0x1u;  // first iteration: random graph, HBM-b
 // in the end). Last search of 353k x 78 fp32 (L 84, C 77) 30.1 ms without the bound,
 // 19.8 with it, of 200k x 96 (L 150, C 100) 23.5 and 16.8, of 1M x 96 (R 48, C 90)
 // 125.7 and 81.8; of 4M x 64 around 64 centers 249 and 296.
+// A bound only spares what a full pool rejects: a search that meets few candidates
+// for its L (few steps, short rows, a wide pool) rejects few, and small rows cost
+// little to begin with. So data without clusters takes it in a later iteration only
+// above a number of candidates per search and pool slot that depends on where the
+// rows lie (below 12 MiB, below the 32 MiB of the eight L2s, beyond): those of
+// iteration 0 for the iterations between, of the one before it for the last. Search
+// times without over with the bound at the sides of the lines, candidates per slot in
+// brackets, from 148 builds of 20k-350k rows (R 24-64, L 84-256, STEPS 20-64).
+// Between: 350k x 79 at R 24 0.92 (4.9) and 1.20 (6.3), 47k 0.85 (4.9) and 1.03
+// (6.2), 20k 0.92 (18) and 1.04 (31; at 3 slots a lane 0.90 at 24.5). Last: 350k x 96
+// at R 64 1.00 (4.4) and 1.23 (7.0), 47k 0.96 (6.8) and 1.19 (7.6), 20k 0.98 (17.4)
+// and 1.11 (22).
+struct PerSlot {
+  double between, last;
+};
+static PerSlot per_slot(double row_bytes) {
+  constexpr double kMiB = 1 << 20;
+  if (row_bytes < 12.0 * kMiB) return {22.0, 18.0};
+  return row_bytes < 32.0 * kMiB ? PerSlot{5.5, 7.5} : PerSlot{5.5, 4.5};
+}
 constexpr double kDenseFrac = 0.25;
 constexpr double kDenseMinBytes = 4.0 * (1 << 20);  // one XCD's L2
 constexpr double kClusteredMinBytes = 3e9;
@@ -923,7 +943,9 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
       dense = (double)h.prune_bound_checks > kDenseFrac * pairs * (double)g.N;
       if (dense && qbound_prune_adaptive()) q_prune_iters |= 2u;
       after_first = h;
-      if (dense && fewer_lines && qbound_iters_adaptive() && row_bytes > kDenseMinBytes)
+      const double cand0 = (double)(h.search_dist + h.bound_skips);
+      if (dense && fewer_lines && qbound_iters_adaptive() && row_bytes > kDenseMinBytes &&
+          cand0 > per_slot(row_bytes).between * (double)L * (double)N)
         q_iters |= ((1u << (iters - 1)) - 1u) & ~1u;  // the iterations between the first and the last
     }
     if (fewer_lines && qbound_iters_adaptive() && iters > 1 && it + 3 >= iters && it + 1 < iters) {
@@ -945,7 +967,9 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
                              (double)(after_first.search_dist + after_first.bound_skips);
         const double exps1 = (double)(before_last.expansions - after_first.expansions);
         const bool many_new = iters > 3 && row_bytes > kDenseMinBytes && cand1 > kNewFrac * R * exps1;
-        if (cand > kQBoundLastMinDist * exps && (dense || many_new || row_bytes >= kClusteredMinBytes))
+        const bool rejects = cand > per_slot(row_bytes).last * (double)L * (double)N;
+        if (cand > kQBoundLastMinDist * exps &&
+            (((dense || many_new) && rejects) || row_bytes >= kClusteredMinBytes))
           q_iters |= 1u << (iters - 1);
       }
     }

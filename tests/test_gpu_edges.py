@@ -248,7 +248,7 @@ def test_dense_rule_compares_lines(dim, middle, monkeypatch):
             monkeypatch.setenv("DANCE_QBOUND", "0")
         g = torch.empty((n, R), dtype=torch.int32, device="cuda")
         d = torch.empty((n,), dtype=torch.int32, device="cuda")
-        D.vamana_build_resident(x.data_ptr(), D.DTYPE_F16, n, dim, R, 64, 64, 32, g.data_ptr(), d.data_ptr())
+        D.vamana_build_resident(x.data_ptr(), D.DTYPE_F16, n, dim, R, 64, 64, 40, g.data_ptr(), d.data_ptr())
         out.append((g, d))
         if not off:
             checks = D.last_kernel_profile()["bound_checks_iter"]
@@ -263,7 +263,7 @@ def test_dense_rule_compares_lines(dim, middle, monkeypatch):
 @pytest.mark.parametrize("centers,last", [(0, True), (40, False)])
 def test_last_iteration_bound_with_long_candidate_rows(centers, last, monkeypatch):
     import torch
-    n, dim, R = 20_000, 96, 48
+    n, dim, R = 40_000, 96, 48
     x = torch.from_numpy(rows("f32", n, dim, centers=centers)).cuda()
     out = []
     for off in (False, True):
@@ -276,6 +276,32 @@ def test_last_iteration_bound_with_long_candidate_rows(centers, last, monkeypatc
         if not off:
             checks = D.last_kernel_profile()["bound_checks_iter"]
             assert [c > 0 for c in checks[:4]] == [True, False, False, last]
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+# later iterations take the bound only where a search meets enough candidates for its
+# pool: few steps, short rows, a wide pool and small rows do without
+@pytest.mark.parametrize("n,dim,R,L,C,steps,between,last", [
+    (47_000, 79, 24, 162, 48, 33, False, False),
+    (47_000, 79, 24, 84, 48, 33, True, False),
+    (47_000, 96, 64, 162, 100, 20, False, False),
+    (20_000, 96, 48, 100, 90, 40, False, False),
+    (47_000, 79, 42, 84, 77, 33, False, True),
+])
+def test_later_bounds_need_candidates(n, dim, R, L, C, steps, between, last, monkeypatch):
+    import torch
+    x = torch.from_numpy(rows("f32", n, dim)).cuda()
+    out = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv("DANCE_QBOUND", "0")
+        g = torch.empty((n, R), dtype=torch.int32, device="cuda")
+        d = torch.empty((n,), dtype=torch.int32, device="cuda")
+        D.vamana_build_resident(x.data_ptr(), D.DTYPE_F32, n, dim, R, L, C, steps, g.data_ptr(), d.data_ptr())
+        out.append((g, d))
+        if not off:
+            checks = D.last_kernel_profile()["bound_checks_iter"]
+            assert [c > 0 for c in checks[:4]] == [True, between, between, last]
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
