@@ -18,7 +18,7 @@
 //
 // Algorithmic bytes reported for the roofline (per kernel, summed over the
 // build; V = bytes of one vector row, counted on device by each wave):
-//   search: (search_dist + insert_dist) * V + expansions * (4R + 4)
+//   search: (search_dist + insert_dist) * V + expansions * 4R
 //           + N * (V + 4R + 4 + 16C)            (own vector, cur row, work row r/w)
 //           + bound_checks * 128                (quantized rows, when the bound is on)
 //   merge : merge_dist * 4 (snapshot distances read) + reverse_edges * 4 + touched_rows * (16C + 8)
@@ -1068,7 +1068,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     // neighbours' rows and writes its work row (8C) instead of reading and
     // writing it (16C).
     const bool init_it = it == 0 && L <= 128;
-    const double adj = init_it ? 0.0 : 4.0 * R + 4.0;
+    const double adj = init_it ? 0.0 : 4.0 * R;
     const double per_vertex = init_it ? V + R * V + 8.0 * C : V + 4.0 * R + 4.0 + 16.0 * C;
     p.search_bytes_iter[it] = (double)(p.search_dist_iter[it] + p.insert_dist_iter[it]) * V +
                               (double)p.expansions_iter[it] * adj + (double)N * per_vertex +
@@ -1085,7 +1085,7 @@ static int run_build(const Rows& rows, uint32_t R, uint32_t L, uint32_t C, uint3
     const double pair_rows = gram_it ? (double)N * C : (double)p.prune_dist_iter[it];
     p.prune_bytes_iter[it] = pair_rows * V + (double)N * (24.0 * C) + qbytes;
   }
-  p.search_bytes = (double)(p.search_dist + p.insert_dist) * V + (double)p.expansions * (4.0 * R + 4.0) +
+  p.search_bytes = (double)(p.search_dist + p.insert_dist) * V + (double)p.expansions * (4.0 * R) +
                    (double)iters * N * (V + 4.0 * R + 4.0 + 16.0 * C) +
                    (double)(p.bound_checks + p.insert_bound_checks) * qrow_bytes;
   if (timed) {  // the per-launch figures know which launch recomputed its adjacency rows

@@ -9,12 +9,13 @@
 //
 // What bounds the searches: iteration 0 the random 128-byte gathers (55-64
 // billion lines a second, whichever memory level serves them); iterations 1-3
-// instruction issue, the scalar port first (79-85% of its rate on uint8
-// rows). So masks come from the predicate at hand instead of being rebuilt
-// from counts, states that only change once (the full pool, the clean row)
-// are flags, and distances are written by every lane of an octet instead of
-// under a lane mask: the searches of iterations 1-3 at 2M x 128 uint8 took
-// 69.5 / 75.3 / 95.3 ms before and 60.7 / 66.3 / 86.0 ms with these.
+// instruction issue (uint8 rows: the vector pipe at 77-81% of its rate, the
+// scalar port at 69-77%; it came first, at 79-85%, before what follows). Masks
+// come from the predicate at hand instead of being rebuilt from counts, states
+// that only change once (the full pool, the clean row) are flags, and distances
+// are written by every lane of an octet instead of under a lane mask: the
+// searches of iterations 1-3 at 2M x 128 uint8 took 69.5 / 75.3 / 95.3 ms before
+// and 60.7 / 66.3 / 86.0 ms with these.
 //
 // Semantics follow /root/reference/src/gpu_vamana_vnew2.cu exactly; each
 // kernel cites the reference kernel it replaces. The visited cache never
